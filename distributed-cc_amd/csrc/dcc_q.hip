@@ -139,8 +139,9 @@ __device__ __forceinline__ double q_zsq(const double *__restrict__ vvoo, const d
            VV(b, c, j, k) * T2(a, d, i, l) + VV(b, d, j, l) * T2(a, c, i, k) + VV(c, d, k, l) * T2(a, b, i, j);
 }
 
-// Workgroup sums of (paren, bracket) into partials[2 * blockIdx.x + {0, 1}].
-__device__ __forceinline__ void q_store_partials(double paren, double bracket, double *__restrict__ partials) {
+// Workgroup sums of (paren, bracket) into partials[2 * wg + {0, 1}].
+__device__ __forceinline__ void q_store_partials(double paren, double bracket, double *__restrict__ partials,
+                                                 int64_t wg) {
     __shared__ double red[2][kQThreads / 64];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -159,8 +160,8 @@ __device__ __forceinline__ void q_store_partials(double paren, double bracket, d
             p += red[0][w];
             q += red[1][w];
         }
-        partials[2 * blockIdx.x] = p;
-        partials[2 * blockIdx.x + 1] = q;
+        partials[2 * wg] = p;
+        partials[2 * wg + 1] = q;
     }
 }
 
@@ -209,7 +210,7 @@ __global__ __launch_bounds__(kQThreads) void q_finalize_kernel(
             bracket += t * q_zsq(vvoo, t2, vp, o, q, i, j, k, l);
         }
     }
-    q_store_partials(paren, bracket, partials);
+    q_store_partials(paren, bracket, partials, blockIdx.x);
 }
 
 // The same update for any nocc, with one o^4 intermediate per workgroup in the global workspace ws
@@ -249,7 +250,320 @@ __global__ __launch_bounds__(kQThreads) void q_finalize_ws_kernel(
             bracket += t * q_zsq(vvoo, t2, vp, (int)o, q, (int)i, (int)j, (int)k, (int)l);
         }
     }
-    q_store_partials(paren, bracket, partials);
+    q_store_partials(paren, bracket, partials, blockIdx.x);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Fused (Q) quadruple: one workgroup forms z4 and t4 of one (a,b,c,d) in LDS and finishes it there.
+//
+// The 24 z4 and 24 t4 terms of rccsdt_q.py:1014-1129 are two kinds of product over the o^4 block:
+//   pair terms, (p,q) one of the six virtual pairs, r < s the other two, x,y,z,n occupied indices that
+//     sit in the slots of p, q, r, s:
+//       z4[x,y,z,n] += sum_e T[p,q,e,x,y,z] V[r,s,e,n]    and the same with r and s (and z, n) swapped
+//       t4[x,y,z,n] -= sum_m Wo[p,q,m,x,y,z] t2[r,s,m,n]  (likewise)
+//     Both share the left operand, so they are one product of o^3 rows by 2 o columns.
+//   square terms, per partition of the four into rows {y,z} and columns {x,s}:
+//       t4 += Wv[x,y,z,e,Y,Z] t2[e,s,X,S],  z4 -= T[x,y,z,m,Y,Z] vooo[s,m,S,X]
+//     for (x,s), (s,x) and with the roles of rows and columns exchanged: four terms of one o^2 x o^2
+//     product accumulated before they are added.  (T[x,y,z,..] with x in any order: T is symmetric.)
+// Products run on v_mfma_f64_16x16x4 with both operands read straight from L2 (rows of T, Wo, Wv and t2
+// are contiguous, 128-byte pieces); every element of the o^4 block is added by one lane per barrier
+// interval, so the sums have a fixed order.  z4 and t4 never reach HBM: written and read back by 48
+// batched GEMMs and a finalize pass they were 811 GB at nocc=8, nvir=40 and bound the evaluation: a whole
+// (Q) call at nocc=8, nvir=38 takes 58 ms this way against 313 ms, at nocc=5, nvir=19 1.4 ms against 5.8 ms.
+// The block is stored with odd strides so that lanes running over any occupied index hit distinct banks.
+struct QQuadArgs {
+    const double *T, *vvvo, *vooo, *t2, *Wv, *Wo, *vvoo, *e_occ, *e_vir;
+    const int *tasks, *slots;   // slots: per task the 12 Wv slots of its ordered block triples, or null
+    int bs, nv, vp;
+    double *partials;
+};
+
+typedef double qd4 __attribute__((ext_vector_type(4)));
+
+template <int O> struct QBlk {
+    static constexpr int O2 = O * O, O3 = O2 * O, O4 = O3 * O;
+    static constexpr int S1 = O | 1, S2 = (O * S1) | 1, S3 = (O * S2) | 1, SZ = O * S3;
+    static constexpr int RF3 = (O3 + 15) / 16;              // row fragments of a pair term
+    static constexpr int CF3 = (2 * O + 15) / 16;           // column fragments of a pair term
+    static constexpr int RB = CF3 == 1 ? (RF3 + 3) / 4 : 4;  // row fragments per wave and pass (registers)
+    static constexpr int RF2 = (O2 + 15) / 16, NF2 = RF2 * RF2, TF2 = (NF2 + 3) / 4;
+    __device__ static int pos(int slot) { return slot == 0 ? S3 : slot == 1 ? S2 : slot == 2 ? S1 : 1; }
+    // LDS position of the linear element x of the o^4 block
+    __device__ static int at(int x) { return x / O3 * S3 + x / O2 % O * S2 + x / O % O * S1 + x % O; }
+};
+
+// dst[x,y,z,n] (+)= sign * sum_k A[k][x,y,z] B1[k][n] and dst[x,y,n,z] (+)= sign * sum_k A[k][x,y,z] B2[k][n]
+// with A of O^3 columns per k and B of O per k; sx..sn: LDS strides of the slots of x, y, z, n.
+template <int O>
+__device__ __forceinline__ void q_pair_term(const double *__restrict__ A, const double *__restrict__ B1,
+                                            const double *__restrict__ B2, int K, double sign, double *dst, int sx,
+                                            int sy, int sz, int sn) {
+    typedef QBlk<O> G;
+    const int lane = threadIdx.x % 64, w = threadIdx.x / 64, lr = lane % 16, lk = lane / 16;
+    const double *bp[G::CF3];
+    bool bok[G::CF3];
+#pragma unroll
+    for (int c = 0; c < G::CF3; ++c) {
+        const int col = lr + 16 * c;
+        bok[c] = col < 2 * O;
+        bp[c] = !bok[c] ? B1 : col < O ? B1 + col : B2 + (col - O);
+    }
+    for (int g = 0; g < G::RF3; g += 4 * G::RB) {
+        const double *ap[G::RB];
+#pragma unroll
+        for (int r = 0; r < G::RB; ++r) ap[r] = A + min((g + w + 4 * r) * 16 + lr, G::O3 - 1);
+        qd4 acc[G::RB][G::CF3];
+#pragma unroll
+        for (int r = 0; r < G::RB; ++r)
+#pragma unroll
+            for (int c = 0; c < G::CF3; ++c) acc[r][c] = qd4{0, 0, 0, 0};
+        // k of this lane in steps of 4; beyond K the last k is read and multiplied by zero
+        double a[2][G::RB], b[2][G::CF3];
+        auto load = [&](int s, int k0) {
+            const int k = k0 + lk, kk = min(k, K - 1);
+#pragma unroll
+            for (int r = 0; r < G::RB; ++r) a[s][r] = ap[r][(int64_t)kk * G::O3];
+#pragma unroll
+            for (int c = 0; c < G::CF3; ++c) {
+                const double x = bp[c][kk * O];
+                b[s][c] = k < K && bok[c] ? x : 0.0;
+            }
+        };
+        auto mul = [&](int s) {
+#pragma unroll
+            for (int r = 0; r < G::RB; ++r)
+#pragma unroll
+                for (int c = 0; c < G::CF3; ++c)
+                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][r], b[s][c], acc[r][c], 0, 0, 0);
+        };
+        load(0, 0);
+        for (int k0 = 0; k0 < K; k0 += 8) {
+            load(1, k0 + 4);
+            mul(0);
+            load(0, k0 + 8);
+            mul(1);
+        }
+        // the two terms of a column group touch the same elements: one barrier interval each
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int c = 0; c < G::CF3; ++c) {
+                const int col = lr + 16 * c, n = t ? col - O : col;
+                if (n < 0 || n >= O) continue;
+#pragma unroll
+                for (int r = 0; r < G::RB; ++r)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int row = (g + w + 4 * r) * 16 + lk + 4 * q;
+                        if (row >= G::O3) continue;
+                        const int x = row / G::O2, y = row / O % O, z = row % O;
+                        double *d = dst + x * sx + y * sy + (t ? z * sn + n * sz : z * sz + n * sn);
+                        *d += sign * acc[r][c][q];
+                    }
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// acc += sum_k A[k ka + row] B[k kb + col] over K for this wave's fragments of an O^2 x O^2 product;
+// TR / TC: the row / column pair (u,v) is stored as [v][u] in its operand.
+template <int O, bool TR, bool TC>
+__device__ __forceinline__ void q_square_acc(const double *__restrict__ A, int64_t ka, const double *__restrict__ B,
+                                             int64_t kb, int K, qd4 *acc) {
+    typedef QBlk<O> G;
+    const int lane = threadIdx.x % 64, w = threadIdx.x / 64, lr = lane % 16, lk = lane / 16;
+    int ar[G::TF2], bc[G::TF2];
+#pragma unroll
+    for (int t = 0; t < G::TF2; ++t) {
+        const int f = min(w + 4 * t, G::NF2 - 1);
+        const int row = min(f % G::RF2 * 16 + lr, G::O2 - 1), col = min(f / G::RF2 * 16 + lr, G::O2 - 1);
+        ar[t] = TR ? row % O * O + row / O : row;
+        bc[t] = TC ? col % O * O + col / O : col;
+    }
+    double a[2][G::TF2], b[2][G::TF2];
+    auto load = [&](int s, int k0) {
+        const int k = k0 + lk, kk = min(k, K - 1);
+        const double *ak = A + kk * ka, *bk = B + kk * kb;
+#pragma unroll
+        for (int t = 0; t < G::TF2; ++t) {
+            a[s][t] = ak[ar[t]];
+            const double x = bk[bc[t]];
+            b[s][t] = k < K ? x : 0.0;
+        }
+    };
+    auto mul = [&](int s) {
+#pragma unroll
+        for (int t = 0; t < G::TF2; ++t)
+            acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][t], b[s][t], acc[t], 0, 0, 0);
+    };
+    load(0, 0);
+    for (int k0 = 0; k0 < K; k0 += 8) {
+        load(1, k0 + 4);
+        mul(0);
+        load(0, k0 + 8);
+        mul(1);
+    }
+}
+
+// dst += sign * acc, rows (y,z) and columns (x,s) with the LDS strides of their slots
+template <int O>
+__device__ __forceinline__ void q_square_add(const qd4 *acc, double sign, double *dst, int sy, int sz, int sx, int ss) {
+    typedef QBlk<O> G;
+    const int lane = threadIdx.x % 64, w = threadIdx.x / 64, lr = lane % 16, lk = lane / 16;
+#pragma unroll
+    for (int t = 0; t < G::TF2; ++t) {
+        const int f = w + 4 * t;
+        const int col = f / G::RF2 * 16 + lr;
+        if (f >= G::NF2 || col >= G::O2) continue;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int row = f % G::RF2 * 16 + lk + 4 * q;
+            if (row < G::O2) dst[row / O * sy + row % O * sz + col / O * sx + col % O * ss] += sign * acc[t][q];
+        }
+    }
+}
+
+template <int O>
+__global__ __launch_bounds__(kQThreads) void q_quad_kernel(const QQuadArgs p, int64_t total) {
+    typedef QBlk<O> G;
+    extern __shared__ double lds[];
+    double *Z = lds, *S = lds + G::SZ;
+    // consecutive quadruples on one XCD: they share T[a,b], T[a,c], T[b,c] slices in its L2
+    const int64_t wg = [&] {
+        const int64_t L = blockIdx.x, q = total / 8, r = total % 8, x = L % 8, y = L / 8;
+        return x < r ? x * (q + 1) + y : r * (q + 1) + (x - r) * q + y;
+    }();
+    const int bs = p.bs, bs3 = bs * bs * bs;
+    const int64_t task = wg / ((int64_t)bs3 * bs);
+    const int e0 = (int)(wg % ((int64_t)bs3 * bs));
+    const int in[4] = {e0 / bs3, e0 / (bs * bs) % bs, e0 / bs % bs, e0 % bs};   // index within each block
+    int v[4];                                                                   // a, b, c, d
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = p.tasks[4 * task + u] + in[u];
+    const double fac = v[0] < p.nv && v[1] < p.nv && v[2] < p.nv && v[3] < p.nv ? q_factor(v[0], v[1], v[2], v[3]) : 0.0;
+    if (fac == 0.0) {   // uniform over the workgroup
+        if (threadIdx.x == 0) {
+            p.partials[2 * wg] = 0.0;
+            p.partials[2 * wg + 1] = 0.0;
+        }
+        return;
+    }
+    const int64_t vp = p.vp;
+    const int K = p.nv;
+    for (int x = threadIdx.x; x < 2 * G::SZ; x += kQThreads) lds[x] = 0.0;
+    __syncthreads();
+    // ---- pair terms: (p,q) over the six pairs, r < s the others ----
+#pragma unroll
+    for (int u = 0; u < 6; ++u) {
+        constexpr int PP[6] = {0, 0, 0, 1, 1, 2}, QQ[6] = {1, 2, 3, 2, 3, 3};
+        constexpr int RR[6] = {2, 1, 1, 0, 0, 0}, SS[6] = {3, 3, 2, 3, 2, 1};
+        const int P = PP[u], Q = QQ[u], R = RR[u], X = SS[u];
+        const int64_t pq = v[P] * vp + v[Q], rs = v[R] * vp + v[X], sr = v[X] * vp + v[R];
+        const double *A = p.T + pq * vp * G::O3, *Ao = p.Wo + pq * O * G::O3;
+        const double *B1 = p.vvvo + rs * vp * O, *B2 = p.vvvo + sr * vp * O;
+        const double *C1 = p.t2 + rs * G::O2, *C2 = p.t2 + sr * G::O2;
+        const int sx = G::pos(P), sy = G::pos(Q), sz = G::pos(R), sn = G::pos(X);
+        q_pair_term<O>(A, B1, B2, K, 1.0, Z, sx, sy, sz, sn);
+        q_pair_term<O>(Ao, C1, C2, O, -1.0, S, sx, sy, sz, sn);
+    }
+    // ---- square terms: columns (a, s), rows the other two ----
+    auto wv = [&](int x, int y, int z) {   // Wv[v[x], v[y], v[z]]
+        if (p.slots == nullptr) return p.Wv + ((v[x] * vp + v[y]) * vp + v[z]) * vp * G::O2;
+        // slot of the ordered block triple: x, and the position of the letter left out among the other three
+        const int left = 6 - x - y - z;
+        const int64_t slot = p.slots[12 * task + 3 * x + (left > x ? left - 1 : left)];
+        return p.Wv + (slot * bs3 + (in[x] * bs + in[y]) * bs + in[z]) * vp * G::O2;
+    };
+    auto tm = [&](int x, int y, int z) { return p.T + ((v[x] * vp + v[y]) * vp + v[z]) * G::O3; };
+    auto t2 = [&](int s) { return p.t2 + v[s] * (int64_t)G::O2; };
+    auto vo = [&](int s) { return p.vooo + v[s] * (int64_t)G::O3; };
+#pragma unroll
+    for (int s = 1; s < 4; ++s) {
+        const int y = s == 1 ? 2 : 1, z = s == 3 ? 2 : 3;
+        qd4 acc[G::TF2];
+#pragma unroll
+        for (int t = 0; t < G::TF2; ++t) acc[t] = qd4{0, 0, 0, 0};
+        const int64_t kt = vp * G::O2;
+        q_square_acc<O, false, false>(wv(0, y, z), G::O2, t2(s), kt, K, acc);
+        q_square_acc<O, false, true>(wv(s, y, z), G::O2, t2(0), kt, K, acc);
+        q_square_acc<O, false, false>(t2(z), kt, wv(y, 0, s), G::O2, K, acc);
+        q_square_acc<O, true, false>(t2(y), kt, wv(z, 0, s), G::O2, K, acc);
+        q_square_add<O>(acc, 1.0, S, G::pos(y), G::pos(z), G::pos(0), G::pos(s));
+#pragma unroll
+        for (int t = 0; t < G::TF2; ++t) acc[t] = qd4{0, 0, 0, 0};
+        q_square_acc<O, false, true>(tm(0, y, z), G::O2, vo(s), G::O2, O, acc);
+        q_square_acc<O, false, false>(tm(s, y, z), G::O2, vo(0), G::O2, O, acc);
+        q_square_acc<O, true, false>(vo(z), G::O2, tm(y, 0, s), G::O2, O, acc);
+        q_square_acc<O, false, false>(vo(y), G::O2, tm(z, 0, s), G::O2, O, acc);
+        q_square_add<O>(acc, -1.0, Z, G::pos(y), G::pos(z), G::pos(0), G::pos(s));
+        __syncthreads();
+    }
+    // ---- P4_444 of (t4 + z4) / D times the factor (see q_finalize_ws_kernel for the expanded form) ----
+    constexpr int NX = (G::O4 + kQThreads - 1) / kQThreads;
+    double val[NX];
+    const double ev = p.e_vir[v[0]] + p.e_vir[v[1]] + p.e_vir[v[2]] + p.e_vir[v[3]];
+#pragma unroll
+    for (int n = 0; n < NX; ++n) {
+        const int x = threadIdx.x + n * kQThreads;
+        if (x < G::O4) S[G::at(x)] += Z[G::at(x)];
+    }
+    __syncthreads();
+    auto ix = [](int i, int j, int k, int l) { return i * G::S3 + j * G::S2 + k * G::S1 + l; };
+#pragma unroll
+    for (int n = 0; n < NX; ++n) {
+        const int x = threadIdx.x + n * kQThreads;
+        if (x >= G::O4) continue;
+        const int i = x / G::O3, j = x / G::O2 % O, k = x / O % O, l = x % O;
+        const double den = p.e_occ[i] + p.e_occ[j] + p.e_occ[k] + p.e_occ[l] - ev;
+        const double num = 2.0 * S[ix(i, j, k, l)] - S[ix(j, i, k, l)] - S[ix(k, j, i, l)] - S[ix(l, j, k, i)];
+        val[n] = fabs(den) > 1e-15 ? num / den : 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NX; ++n) {
+        const int x = threadIdx.x + n * kQThreads;
+        if (x < G::O4) S[G::at(x)] = val[n];
+    }
+    __syncthreads();
+    double paren = 0.0, bracket = 0.0;
+#pragma unroll
+    for (int n = 0; n < NX; ++n) {
+        const int x = threadIdx.x + n * kQThreads;
+        if (x >= G::O4) continue;
+        const int i = x / G::O3, j = x / G::O2 % O, k = x / O % O, l = x % O;
+        val[n] = fac * (4.0 * S[ix(i, j, k, l)] - 2.0 * S[ix(i, k, j, l)] - 2.0 * S[ix(i, l, k, j)] -
+                        2.0 * S[ix(i, j, l, k)] + S[ix(i, l, j, k)] + S[ix(i, k, l, j)]);
+        paren += val[n] * Z[ix(i, j, k, l)];
+    }
+    __syncthreads();
+    // <ab|ij> and t2 of the six pairs, in the space of z4
+    for (int x = threadIdx.x; x < 12 * G::O2; x += kQThreads) {
+        const int m = x / G::O2, u = m % 6, y = x % G::O2;
+        const int a = u < 3 ? 0 : u < 5 ? 1 : 2, b = u < 3 ? u + 1 : u < 5 ? u - 1 : 3;
+        Z[x] = (m < 6 ? p.vvoo : p.t2)[(v[a] * vp + v[b]) * G::O2 + y];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NX; ++n) {
+        const int x = threadIdx.x + n * kQThreads;
+        if (x >= G::O4) continue;
+        const int i = x / G::O3, j = x / G::O2 % O, k = x / O % O, l = x % O;
+        auto VV = [&](int u, int s, int t) { return Z[u * G::O2 + s * O + t]; };
+        auto T2 = [&](int u, int s, int t) { return Z[(6 + u) * G::O2 + s * O + t]; };
+        bracket += val[n] * (VV(0, i, j) * T2(5, k, l) + VV(1, i, k) * T2(4, j, l) + VV(2, i, l) * T2(3, j, k) +
+                             VV(3, j, k) * T2(2, i, l) + VV(4, j, l) * T2(1, i, k) + VV(5, k, l) * T2(0, i, j));
+    }
+    q_store_partials(paren, bracket, p.partials, wg);
+}
+
+template <int O> int q_quads_launch(const QQuadArgs &a, int64_t total, hipStream_t s) {
+    // the two blocks; at the end 12 o^2 matrix elements take their place (more than the blocks at small o)
+    constexpr size_t bytes = sizeof(double) * (2 * QBlk<O>::SZ > 12 * O * O ? 2 * QBlk<O>::SZ : 12 * O * O);
+    hipLaunchKernelGGL(q_quad_kernel<O>, dim3((unsigned)total), dim3(kQThreads), bytes, s, a, total);
+    DCC_LAUNCH_CHECK();
+    return 0;
 }
 
 }  // namespace
@@ -316,6 +630,32 @@ int dcc_q_finalize_f64(const double *t4, const double *z4, const int32_t *tasks,
     }
     DCC_LAUNCH_CHECK();
     return 0;
+}
+
+int dcc_q_quads_f64(const double *T, const double *vvvo, const double *vooo, const double *vvoo, const double *t2,
+                    const double *Wv, const double *Wo, const int32_t *slots, const int32_t *tasks, int64_t ntask,
+                    int64_t blksize, int64_t nocc, int64_t nvir, int64_t vpad, const double *e_occ,
+                    const double *e_vir, double *partials, dcc_stream_t stream) {
+    DCC_CHECK(ntask >= 0 && blksize > 0 && nocc > 0 && nvir > 0 && vpad >= nvir, "bad extents");
+    DCC_CHECK(nocc <= 9, "nocc > 9: the o^4 blocks exceed LDS, use dcc_q_finalize_f64 with a workspace");
+    const int64_t nwg = ntask * blksize * blksize * blksize * blksize;
+    if (nwg == 0) return 0;
+    DCC_CHECK(T && vvvo && vooo && vvoo && t2 && Wv && Wo && tasks && e_occ && e_vir && partials, "null pointer");
+    DCC_CHECK(nwg < ((int64_t)1 << 31), "grid too large");
+    const QQuadArgs a{T,     vvvo,  vooo,  t2,    Wv,           Wo,        vvoo,      e_occ,
+                      e_vir, tasks, slots, (int)blksize, (int)nvir, (int)vpad, partials};
+    hipStream_t s = dcc::as_stream(stream);
+    switch (nocc) {
+        case 1: return q_quads_launch<1>(a, nwg, s);
+        case 2: return q_quads_launch<2>(a, nwg, s);
+        case 3: return q_quads_launch<3>(a, nwg, s);
+        case 4: return q_quads_launch<4>(a, nwg, s);
+        case 5: return q_quads_launch<5>(a, nwg, s);
+        case 6: return q_quads_launch<6>(a, nwg, s);
+        case 7: return q_quads_launch<7>(a, nwg, s);
+        case 8: return q_quads_launch<8>(a, nwg, s);
+        default: return q_quads_launch<9>(a, nwg, s);
+    }
 }
 
 }  // extern "C"

@@ -9,14 +9,15 @@ Layout in HBM (FP64, virtual dimension zero-padded to vp = ceil(v/bs)*bs):
            (nslot, bs, bs, bs, vp, o, o), one per distinct ordered triple of
            the chunk's virtual blocks (the reference builds the block slices
            per task, rccsdt_q.py:390-408,943-947)
+Up to nocc = 9 one kernel (dcc_q_quads_f64) forms the z4_p and t4 of every
+(a,b,c,d) of a chunk of tasks in LDS (rccsdt_q.py:1014-1129) and applies t4 += z4_p,
+the denominator, P4_444, the factor and both dot products (rccsdt_q.py:1131-1153),
+writing per-workgroup partials that are summed in a fixed order into one pair per
+chunk; the host reads the pairs once at the end.  For nocc > 9 (or ``finalize_ws``)
+the o^4 blocks do not fit LDS: each of the 24 z4_p and 24 t4 einsums of a task is one
+batched gather-GEMM over a chunk of tasks into
   z4, t4   (ntask_chunk, bs, bs, bs, bs, o, o, o, o)
-Each of the 24 z4_p einsums and 24 t4 einsums of a task (rccsdt_q.py:1014-1129)
-is one batched gather-GEMM over a chunk of tasks; a fused kernel then applies
-t4 += z4_p, the denominator, P4_444, the factor and both dot products
-(rccsdt_q.py:1131-1153), writing per-workgroup partials that are summed in a
-fixed order into one pair per chunk; the host reads the pairs once at the end.
-For nocc > 9 the fused kernel keeps its o^4 intermediate in a global workspace
-of the size of t4 instead of LDS.
+and the finalize kernel keeps its intermediate in a workspace of the size of t4.
 """
 import numpy as np
 
@@ -101,12 +102,14 @@ class QEngine:
         o, vp, bs = self.o, self.vp, self.bs
         per_task = bs ** 4 * o ** 4 * 8
         self.chunk = max(1, min(int(max_chunk_bytes // per_task), 4096))
+        # the partials of a chunk are two doubles per quadruple
+        self.quad_chunk = max(1, int(max_chunk_bytes // (bs ** 4 * 16)))
         if w_mode is None:
             w_mode = "dense" if vp ** 4 * o * o * 8 <= dense_w_bytes else "task"
         if w_mode not in ("dense", "task"):
             raise ValueError("w_mode must be 'dense' or 'task'")
         self.w_mode = w_mode
-        # the fused finalize keeps two o^4 blocks in LDS up to nocc = 9, a global workspace beyond
+        # z4 and t4 of a quadruple fit LDS up to nocc = 9; beyond, GEMMs and a finalize with a workspace
         self.finalize_ws = (o > 9) if finalize_ws is None else bool(finalize_ws)
         if o > 9 and not self.finalize_ws:
             raise ValueError("nocc > 9 needs the workspace form of the (Q) finalize")
@@ -172,19 +175,22 @@ class QEngine:
         ext = {x: bs for x in 'abcd'}
         ext.update({'e': vp, 'f': vp})
         ext.update({x: o for x in 'ijklmn'})
-        nmax = min(self.chunk, len(tasks))
-        z4 = DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o))
-        t4 = DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o))
-        ws = DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o)) if self.finalize_ws else None
+        # chunks bound z4/t4 and the W_vvvvoo slots; with neither only the partials
+        size = self.quad_chunk if not self.finalize_ws and self.w_mode == "dense" else self.chunk
+        nmax = min(size, len(tasks))
+        fused = not self.finalize_ws
+        z4 = t4 = ws = None
+        if not fused:
+            z4, t4, ws = (DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o)) for _ in range(3))
         part = DeviceArray((nmax * bs ** 4, 2))
-        nchunk = -(-len(tasks) // self.chunk)
+        nchunk = -(-len(tasks) // size)
         tot = DeviceArray((max(nchunk, 1), 2))
         # W_vvvvoo slots of each chunk: one per distinct ordered block triple its t4 terms read
         chunk_keys = []
-        for c0 in range(0, len(tasks), self.chunk):
+        for c0 in range(0, len(tasks), size):
             keys = {}
             if self.w_mode == "task":
-                for (a0, b0, cc, d0) in tasks[c0:c0 + self.chunk]:
+                for (a0, b0, cc, d0) in tasks[c0:c0 + size]:
                     blk = dict(a=a0, b=b0, c=cc, d=d0)
                     for sub, an, _, _ in T4_TERMS:
                         if an == 'Wv':
@@ -193,14 +199,19 @@ class QEngine:
         nslot_max = max((len(k) for k in chunk_keys), default=0)
         Ws = DeviceArray((nslot_max, bs, bs, bs, vp, o, o)) if nslot_max else None
         chunks = []
-        for ci, c0 in enumerate(range(0, len(tasks), self.chunk)):
-            chunk = tasks[c0:c0 + self.chunk]
+        for ci, c0 in enumerate(range(0, len(tasks), size)):
+            chunk = tasks[c0:c0 + size]
             nt = len(chunk)
             ext['H'] = nt
             keys = chunk_keys[ci]
             blocks = [dict(a=a0, b=b0, c=cc, d=d0) for (a0, b0, cc, d0) in chunk]
             launches = self._slot_launches(Ws, nslot_max, list(keys)) if keys else []
-            for out, terms in ((z4, Z4_TERMS), (t4, T4_TERMS)):
+            slots = None
+            if fused and keys:
+                slots = DeviceArray.from_host(np.array(
+                    [[keys[tuple([t[x]] + [t[y] for y in range(4) if y not in (x, l)])]
+                      for x in range(4) for l in range(4) if l != x] for t in chunk], dtype=np.int32))
+            for out, terms in () if fused else ((z4, Z4_TERMS), (t4, T4_TERMS)):
                 C = Operand(out, 'Habcdijkl', (nmax, bs, bs, bs, bs, o, o, o, o))
                 for n, (sub, an, bn, alpha) in enumerate(terms):
                     sa, rest = sub.split(',')
@@ -215,8 +226,8 @@ class QEngine:
                     launches.append(plan_einsum('Q ' + sub, sub, A, self._op(bn, sb), C, alpha,
                                                 0.0 if n == 0 else 1.0, ext, batches))
             tk = DeviceArray.from_host(np.array(chunk, dtype=np.int32).reshape(-1, 4))
-            chunks.append((nt, launches, tk))
-        return z4, t4, ws, part, tot, chunks
+            chunks.append((nt, launches, tk, slots))
+        return z4, t4, ws, Ws, part, tot, chunks
 
     def kernel(self, pppp, t2_oovv, t3_dev, mo_energy, job_idx=0, n_jobs=1, t3_layout="ijk"):
         """(e_[Q], e_(Q)) for the T3 already on the device (``t3_dev``): canonical i<=j<=k blocks
@@ -251,15 +262,21 @@ class QEngine:
             tasks = create_full_task_list(v, bs)
             per = (len(tasks) + n_jobs - 1) // n_jobs
             self.task_plans[key] = self._plan_tasks(tasks[job_idx * per: min(job_idx * per + per, len(tasks))])
-        z4, t4, ws, part, tot, chunks = self.task_plans[key]
+        z4, t4, ws, Ws, part, tot, chunks = self.task_plans[key]
         if not chunks:
             return 0.0, 0.0
-        for ci, (nt, launches, tk) in enumerate(chunks):
+        for ci, (nt, launches, tk, slots) in enumerate(chunks):
             for g in launches:
                 g.run(st)
             nwg = nt * bs ** 4
-            L.call("dcc_q_finalize_f64", t4.vp, z4.vp, tk.vp, nt, bs, o, v, vp, dev['e_occ'].vp, dev['e_vir'].vp,
-                   dev['vvoo'].vp, dev['t2'].vp, ws.vp if ws is not None else None, part.vp, self._s())
+            if ws is None:
+                Wv = Ws if slots is not None else dev['Wv']
+                L.call("dcc_q_quads_f64", dev['T'].vp, dev['vvvo'].vp, dev['vooo'].vp, dev['vvoo'].vp, dev['t2'].vp,
+                       Wv.vp, dev['Wo'].vp, slots.vp if slots is not None else None, tk.vp, nt, bs, o, v, vp,
+                       dev['e_occ'].vp, dev['e_vir'].vp, part.vp, self._s())
+            else:
+                L.call("dcc_q_finalize_f64", t4.vp, z4.vp, tk.vp, nt, bs, o, v, vp, dev['e_occ'].vp,
+                       dev['e_vir'].vp, dev['vvoo'].vp, dev['t2'].vp, ws.vp, part.vp, self._s())
             L.call("dcc_reduce_pairs_f64", part.vp, nwg, tot.offset_ptr(2 * ci), self._s())
         pairs = tot.download(stream=st).reshape(-1, 2)[:len(chunks)]
         paren = bracket = 0.0

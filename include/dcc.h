@@ -322,6 +322,20 @@ int dcc_q_finalize_f64(const double *t4, const double *z4, const int32_t *tasks,
                        int64_t nocc, int64_t nvir, int64_t vpad, const double *e_occ, const double *e_vir,
                        const double *vvoo, const double *t2, double *ws, double *partials, dcc_stream_t stream);
 
+/*
+ * The same partials for a list of (Q) tasks straight from the amplitudes and integrals, nocc <= 9: every
+ * (task, a, b, c, d) forms its z4 and t4 (rccsdt_q.py:1014-1129), the denominator, P4_444, the factor and
+ * both dot products in one workgroup, without z4/t4 in memory.  Layouts (virtual extents padded to vpad):
+ * T (a,b,c,i,j,k), vvvo (a,b,c,i), vooo (a,i,j,k), vvoo and t2 (a,b,i,j), Wo (a,b,m,i,j,k), and Wv either
+ * dense (a,b,c,e,j,k) with slots = NULL, or block slots (slot, bs, bs, bs, vpad, o, o) with slots
+ * int32 (ntask, 12): the slot of the ordered block triple of position x of (a,b,c,d) followed by the others
+ * without position l, at 3 x + (l > x ? l - 1 : l).
+ */
+int dcc_q_quads_f64(const double *T, const double *vvvo, const double *vooo, const double *vvoo, const double *t2,
+                    const double *Wv, const double *Wo, const int32_t *slots, const int32_t *tasks, int64_t ntask,
+                    int64_t blksize, int64_t nocc, int64_t nvir, int64_t vpad, const double *e_occ,
+                    const double *e_vir, double *partials, dcc_stream_t stream);
+
 /* ------------------------------------- lower-order iteration (around T3) */
 
 /*

@@ -659,6 +659,37 @@ class Emulator:
         self._npart = 0
         return 0
 
+    def dcc_q_quads_f64(self, T, vvvo, vooo, vvoo, t2, Wv, Wo, slots, tasks, ntask, bs, nocc, nvir, vpad, e_occ,
+                        e_vir, partials, stream):
+        from distr_cc.q_engine import T4_TERMS, Z4_TERMS
+        nt, bs, o, vp = int(ntask), int(bs), int(nocc), int(vpad)
+        get = lambda p, shp: self.dev.view(_ptr(p), np.float64, int(np.prod(shp))).reshape(shp)
+        arr = {'T': get(T, (vp, vp, vp, o, o, o)), 'vvvo': get(vvvo, (vp, vp, vp, o)), 'vooo': get(vooo, (vp, o, o, o)),
+               't2': get(t2, (vp, vp, o, o)), 'Wo': get(Wo, (vp, vp, o, o, o, o))}
+        if _ptr(slots) is None:
+            arr['Wv'] = get(Wv, (vp, vp, vp, vp, o, o))
+        else:
+            sl = self.dev.view(_ptr(slots), np.int32, 12 * nt).reshape(nt, 12)
+            ws = get(Wv, (int(sl.max()) + 1, bs, bs, bs, vp, o, o))
+        tk = self.dev.view(_ptr(tasks), np.int32, 4 * nt).reshape(nt, 4)
+        bufs = [self.dev.malloc(nt * bs ** 4 * o ** 4 * 8) for _ in range(2)]
+        for buf, terms in zip(bufs, (T4_TERMS, Z4_TERMS)):
+            out = get(buf, (nt, bs, bs, bs, bs, o, o, o, o))
+            for n in range(nt):
+                blk = {x: slice(int(tk[n, d]), int(tk[n, d]) + bs) for d, x in enumerate('abcd')}
+                for sub, an, bn, alpha in terms:
+                    sa, rest = sub.split(',')
+                    sb = rest.split('->')[0]
+                    cut = lambda x, s: x[tuple(blk.get(ch, slice(None)) for ch in s)]
+                    if an == 'Wv' and 'Wv' not in arr:
+                        x, left = 'abcd'.index(sa[0]), 'abcd'.index(next(c for c in 'abcd' if c not in sa))
+                        A = ws[sl[n, 3 * x + (left - 1 if left > x else left)]]
+                    else:
+                        A = cut(arr[an], sa)
+                    out[n] += alpha * np.einsum(sub, A, cut(arr[bn], sb))
+        return self.dcc_q_finalize_f64(bufs[0], bufs[1], tasks, nt, bs, o, nvir, vp, e_occ, e_vir, vvoo, t2, None,
+                                       partials, stream)
+
     def dcc_ring_weights_f64(self, *a):
         return self._ring(np.float64, *a)
 

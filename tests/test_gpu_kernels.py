@@ -288,6 +288,28 @@ def test_q_energy_vs_oracle(dev, o, v, bs, form):
     assert abs(sum(p[1] for p in parts) - got[1]) <= 1e-12 * abs(got[1])
 
 
+@pytest.mark.parametrize("o,v,bs", [(1, 5, 2), (2, 5, 5), (4, 7, 2), (6, 6, 3), (7, 5, 4), (8, 6, 4), (9, 5, 2)])
+@pytest.mark.parametrize("w_mode", ["dense", "task"])
+def test_q_fused_quadruples_vs_oracle(dev, o, v, bs, w_mode):
+    """The fused quadruple kernel at every remaining nocc (its tiles are sized by nocc: full and partial
+    row and column fragments, one and several row passes), with dense W_vvvvoo and with block slots; K
+    (v and o) below, at and above a multiple of the MFMA step.  Bound as test_q_energy_vs_oracle."""
+    from distr_cc.device import DeviceArray
+    from distr_cc.q_engine import QEngine
+    from distr_cc.synthetic import SyntheticSystem
+    from oracle import q_energy as Q
+    from oracle import t3_layout as TL
+    _say("(Q) fused o=%d v=%d blksize=%d %s" % (o, v, bs, w_mode))
+    s = SyntheticSystem(o, v, naux=30, seed=700 + o * v, sigma_t3=1e-3)
+    pppp, t2, t3 = s.pppp(), s.t2(), s.t3_tri()
+    ref = Q.kernel(o, v, pppp, t2, TL.full_t3_from_tri(t3, o), s.mo_energy, blksize=bs)
+    eng = QEngine(o, v, blksize=bs, w_mode=w_mode, max_chunk_bytes=3 * bs ** 4 * o ** 4 * 8)
+    for _ in range(2):
+        got = eng.kernel(pppp, t2, DeviceArray.from_host(t3), s.mo_energy)
+        for g, r in zip(got, ref):
+            assert abs(g - r) <= 1e-12 * abs(r)
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 16, 4), (37, 53, 29), (130, 70, 300)])
 def test_contract_f32_plain_gemm(dev, M, N, K):
     """FP32 MFMA path; pins the v_mfma_f32_16x16x4f32 accumulator layout and masking."""
