@@ -2,6 +2,7 @@
 // MFMA (the tile itself is in dcc_gemm_tile.h) and the split-BF16x3 kernel on BF16 MFMA.
 #include "dcc_common.h"
 #include "dcc_gemm_tile.h"
+#include "dcc_gemm_skinny.h"
 #include "dcc_bf16x3.h"
 
 #include <cstdio>
@@ -24,6 +25,16 @@ void contract_kernel(const ContractArgs<T> p) {
     int tm, tn;
     tile_coords(L - batch * per_batch, p.tiles_m, p.tiles_n, tm, tn);
     contract_tile<T, BM, BN, A_KFAST, B_NFAST, C_MFAST, STAGES>(p, batch, tm, tn, smem);
+}
+
+// One workgroup per skinny tile.
+template <typename T, int FX, int FY, int W>
+__global__ __launch_bounds__(W * 64) void skinny_kernel(const SkinnyArgs<T> p) {
+    __shared__ T smem[SkinnySmem<T, FX, FY, W>::v];
+    const int64_t L = xcd_remap((int64_t)blockIdx.x, p.total_tiles);
+    const int64_t per_batch = (int64_t)p.tiles_x * p.tiles_y;
+    const int64_t batch = L / per_batch, t = L - batch * per_batch;
+    skinny_tile<T, FX, FY, W>(p, batch, (int)(t % p.tiles_x), (int)(t / p.tiles_x), smem);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -561,6 +572,40 @@ bool valid_map(const dcc_idxmap &m) {
     return m.e1 >= 1 && m.e2 >= 1 && m.e1 * m.e2 < (int64_t)1 << 32;
 }
 
+// The launch g as a skinny one of variant v (see skinny_variant).
+template <typename T>
+int contract_skinny(const ContractArgs<T> &g, const dcc_idxmap &ak, const dcc_idxmap &bk, bool swap, int64_t nbatch,
+                    int64_t max_rows, int v, hipStream_t s) {
+    const dcc_idxmap &xk = swap ? bk : ak, &yk = swap ? ak : bk;
+    SkinnyArgs<T> a;
+    a.N = g.N;
+    a.K = g.K;
+    a.alpha = g.alpha;
+    a.beta = g.beta;
+    a.X = swap ? g.B : g.A;
+    a.Y = swap ? g.A : g.B;
+    a.C = g.C;
+    a.xm = swap ? g.bn : g.am;
+    a.ym = swap ? g.am : g.bn;
+    a.cx = swap ? g.cn : g.cm;
+    a.cy = swap ? g.cm : g.cn;
+    a.xk = make_kmap(xk, 16 * kSkinny[v].w);
+    a.yk = make_kmap(yk, 16 * kSkinny[v].w);
+    a.batches = g.batches;
+    a.flags = skinny_flags(a.X, a.xm, xk, a.Y, a.ym, yk, g.K, swap, sizeof(T), kSkinny[v].w);
+    const int64_t rx = swap ? g.N : max_rows, ry = swap ? max_rows : g.N;
+    a.tiles_x = (int)((rx + 16 * kSkinny[v].fx - 1) / (16 * kSkinny[v].fx));
+    a.tiles_y = (int)((ry + 16 * kSkinny[v].fy - 1) / (16 * kSkinny[v].fy));
+    a.total_tiles = nbatch * a.tiles_x * a.tiles_y;
+    DCC_CHECK(a.total_tiles < ((int64_t)1 << 31), "too many tiles");
+    return skinny_dispatch(v, [&](auto fx, auto fy, auto w) {
+        constexpr int FX = decltype(fx)::value, FY = decltype(fy)::value, W = decltype(w)::value;
+        hipLaunchKernelGGL((skinny_kernel<T, FX, FY, W>), dim3((unsigned)a.total_tiles), dim3(W * 64), 0, s, a);
+        DCC_LAUNCH_CHECK();
+        return 0;
+    });
+}
+
 template <typename T>
 int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, const T *A, dcc_idxmap am,
                    dcc_idxmap ak, const T *B, dcc_idxmap bk, dcc_idxmap bn, T *C, dcc_idxmap cm, dcc_idxmap cn,
@@ -603,8 +648,9 @@ int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, c
     const bool c_mfast = inner_stride(cn) != 1;
     hipStream_t s = dcc::as_stream(stream);
     // Workgroup tile: tile_shape 0..3 = 64x64, 128x64, 64x128, 128x128 with the two-stage register
-    // prefetch, 4..7 = the same shapes with one stage; -1 = 64x64 two-stage, or DCC_CONTRACT_TILE
-    // (e.g. "128x64" or "64x64s1") when set.
+    // prefetch, 4..7 = the same shapes with one stage; -1 = DCC_CONTRACT_TILE (e.g. "128x64" or
+    // "64x64s1") when set, otherwise a skinny variant where skinny_variant gives one and 64x64 two-stage
+    // elsewhere.
     static const char *tile_env = getenv("DCC_CONTRACT_TILE");
     int tbm = 64, tbn = 64, stages = 2;
     if (tile_shape >= 0) {
@@ -617,6 +663,12 @@ int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, c
             tbn = 64;
         }
         stages = st == 1 ? 1 : 2;
+    } else {
+        SkinnySize z;
+        if (c_mfast) z.add(N, max_rows, K, nbatch);
+        else z.add(max_rows, N, K, nbatch);
+        const int v = skinny_variant(z);
+        if (v >= 0) return contract_skinny<T>(args, ak, bk, c_mfast, nbatch, max_rows, v, s);
     }
     if (tbm == 128 && tbn == 128) return launch<T, 128, 128>(args, max_rows, a_kfast, b_nfast, c_mfast, stages, s);
     if (tbm == 128 && tbn == 64) return launch<T, 128, 64>(args, max_rows, a_kfast, b_nfast, c_mfast, stages, s);

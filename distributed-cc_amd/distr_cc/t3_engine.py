@@ -109,6 +109,10 @@ def _suffix(dtype):
     return {np.dtype(np.float64): "f64", np.dtype(np.float32): "f32"}[np.dtype(dtype)]
 
 
+# the library's own choice of an FP64/FP32 launch as an autotuner result (its skinny tiles have no tile shape)
+LIBRARY_TILE = 8
+
+
 class GemmLaunch:
     """One dcc_contract_f64 / dcc_contract_f32 call with fixed operands, maps and batch table."""
 
@@ -129,7 +133,7 @@ class GemmLaunch:
         self.max_rows = int(max_rows)
         self.flops = float(flops)
         self.keep = keep  # device tables referenced by maps
-        self.tile = -1    # -1: library default; 0..7: dcc_contract_tiled_* tile_shape (autotuned)
+        self.tile = -1    # -1, LIBRARY_TILE: library default; 0..7: dcc_contract_tiled_* tile_shape (autotuned)
 
     def __call__(self, stream):
         self.run(stream)
@@ -138,7 +142,7 @@ class GemmLaunch:
         s = stream.handle if stream is not None else None
         if self.fn == "dcc_contract_packed_bf16x3":
             L.call(self.fn, *self.args, self.batches.vp, self.nbatch, self.max_rows, self.tile, s)
-        elif self.tile >= 0:
+        elif 0 <= self.tile != LIBRARY_TILE:
             L.call(self.fn.replace("contract_", "contract_tiled_"), *self.args, self.batches.vp, self.nbatch,
                    self.max_rows, self.tile, s)
         else:
@@ -1136,8 +1140,8 @@ class TriplesEngine:
                 g.tile = t
 
     def autotune(self, reps=2, include_lower=True):
-        """Time the workgroup tiles of every contraction launch and keep the fastest: eight for the
-        FP64/FP32 kernels (four shapes x one- or two-stage prefetch), twelve for split-BF16x3
+        """Time the workgroup tiles of every contraction launch and keep the fastest: the library's default
+        and eight for the FP64/FP32 kernels (four shapes x one- or two-stage prefetch), twelve for split-BF16x3
         (the four of 256 threads and 256x128, 128x256, 256x256 of 512 threads on 16 x 16 x 32 MFMAs,
         256x256 on 32 x 32 x 16 MFMAs, and four of those staged by direct global -> LDS requests: 256x256
         with two stages, 256x128 and 128x256 with three, 256x256 on 32 x 32 x 16 with two, and the
@@ -1147,7 +1151,7 @@ class TriplesEngine:
         Run it before a residual (it accumulates into R and the scratch buffers); returns
         {launch name: (tile, ms)}."""
         from distr_cc.device import Event
-        shapes = ("64x64", "128x64", "64x128", "128x128", "64x64s1", "128x64s1", "64x128s1", "128x128s1")
+        shapes = ("64x64", "128x64", "64x128", "128x128", "64x64s1", "128x64s1", "64x128s1", "128x128s1", "library")
         shapes3 = ("64x64", "128x64", "64x128", "128x128", "256x128", "128x256", "256x256", "256x256m32",
                    "256x256lds2", "256x128lds3", "128x256lds3", "256x256m32lds2", "256x256w4", "256x256m32w4")
         launches = self._tunable(include_lower)

@@ -1,4 +1,5 @@
 """GPU parity of the libdcc kernels against NumPy / the oracle (FP64)."""
+import itertools
 import sys
 
 import numpy as np
@@ -784,3 +785,46 @@ def test_t3_abc_layout_kernels_vs_oracle(dev, o, v, vp):
     d = dense.download()
     assert np.array_equal(d[:v, :v, :v], T.transpose(3, 4, 5, 0, 1, 2))
     assert not d[v:].any() and not d[:, v:].any() and not d[:, :, v:].any()
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32])
+@pytest.mark.parametrize("M,N,K", [(5, 5, 1805), (1, 1, 64), (16, 17, 65), (33, 40, 400), (130, 130, 100),
+                                   (400, 350, 97), (15, 5000, 130), (6001, 16, 66), (300, 7, 200), (47, 49, 49)])
+def test_contract_skinny_sizes(dev, dt, M, N, K):
+    """The skinny tiles of the default dispatch (few or narrow outputs): every variant, K and edges off the
+    tile steps, each operand and C contiguous along either index, two batch entries with different row
+    ranges and odd offsets, beta = 1.  Bound: K rounding errors of the sum of magnitudes."""
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    rng = np.random.default_rng(M + 3 * N + 7 * K)
+    fn = "dcc_contract_f64" if dt == np.float64 else "dcc_contract_f32"
+    lin = lambda s: L.IdxMap(None, 0, 1, 1 << 20, 0, 0, s)
+    two = lambda e, s: L.IdxMap(None, 0, 1, e, e * s, 0, s)      # the same offsets through two levels
+    # the last K form has an odd inner extent, so groups of k cross its levels
+    for a_k, b_n, c_n, kmap in itertools.product((True, False), (True, False), (True, False), (lin, None)):
+        A = rng.standard_normal((2, M, K) if a_k else (2, K, M)).astype(dt)
+        B = rng.standard_normal((2, K, N) if b_n else (2, N, K)).astype(dt)
+        C = rng.standard_normal((2, M, N) if c_n else (2, N, M)).astype(dt)
+        sak, sam = (1, K) if a_k else (M, 1)
+        sbk, sbn = (N, 1) if b_n else (1, K)
+        scm, scn = (N, 1) if c_n else (1, M)
+        km = (lambda s: two(5, s)) if kmap is None else kmap
+        pad = 1   # odd base offsets of the second entry when the extents are even too
+        dA, dB = (DeviceArray.from_host(np.concatenate([x[0].ravel(), np.zeros(pad, dt), x[1].ravel()])) for x in (A, B))
+        dC = DeviceArray.from_host(C)
+        bt = np.zeros(2, dtype=L.BATCH_DTYPE)
+        bt["a_off"], bt["b_off"], bt["c_off"] = (0, M * K + pad), (0, K * N + pad), (0, M * N)
+        m1 = M - M // 3
+        bt["m_begin"], bt["m_end"] = (0, M // 4), (M, m1)
+        db = DeviceArray.from_host(bt)
+        L.call(fn, M, N, K, -0.5, 1.0, dA.vp, lin(sam), km(sak), dB.vp, km(sbk), lin(sbn), dC.vp, lin(scm), lin(scn),
+               db.vp, 2, M, None)
+        got = dC.download()
+        for n, (lo, hi) in enumerate(((0, M), (M // 4, m1))):
+            a = (A[n] if a_k else A[n].T).astype(np.float64)
+            b = (B[n] if b_n else B[n].T).astype(np.float64)
+            c, g = ((x if c_n else x.T).astype(np.float64) for x in (C[n], got[n]))
+            ref = c.copy()
+            ref[lo:hi] += -0.5 * (a[lo:hi] @ b)
+            bound = np.finfo(dt).eps * (K * (np.abs(a) @ np.abs(b)) + np.abs(ref) + np.abs(c))
+            assert (np.abs(g - ref) <= bound).all(), (a_k, b_n, c_n)
