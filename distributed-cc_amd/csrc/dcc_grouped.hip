@@ -10,6 +10,7 @@
 // of one launch must write disjoint C regions (no two problems accumulate into the same element).
 #include "dcc_common.h"
 #include "dcc_gemm_tile.h"
+#include "dcc_gemm_skinny.h"
 
 #include <algorithm>
 #include <vector>
@@ -17,6 +18,8 @@
 namespace {
 
 using namespace dcc_gemm;
+
+constexpr int64_t kSkinnyBase = 64;   // launch variants below: tile shape | flags << 3; from here: skinny ones
 
 // flags of a prepared problem: bits 0..2 the loader/epilogue choice of the launch (A K-contiguous,
 // B N-contiguous, C written along m; the same for every problem of a launch), bits 3..4 the pair
@@ -68,6 +71,48 @@ void grouped_kernel(const dcc_gemm_problem *__restrict__ probs, int nprob, int64
     }
 }
 
+// The same walk over skinny tiles (dcc_gemm_skinny.h): flags of a problem are its skinny_flags, tiles_m and
+// tiles_n its tiles along X and Y.
+template <int FX, int FY, int W>
+__global__ __launch_bounds__(W * 64) void grouped_skinny_kernel(const dcc_gemm_problem *__restrict__ probs, int nprob,
+                                                                int64_t total_tiles) {
+    __shared__ double smem[SkinnySmem<double, FX, FY, W>::v];
+    const int64_t grid = gridDim.x;
+    for (int64_t base = 0; base < total_tiles; base += grid) {
+        const int64_t window = min(grid, total_tiles - base);
+        if ((int64_t)blockIdx.x >= window) break;
+        const int64_t t = base + xcd_remap((int64_t)blockIdx.x, window);
+        int lo = 0, hi = nprob - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) / 2;
+            if (probs[mid].tile_begin <= t) lo = mid;
+            else hi = mid - 1;
+        }
+        const dcc_gemm_problem &q = probs[lo];
+        const bool swap = q.flags & kSkinnySwap;
+        SkinnyArgs<double> a;
+        a.N = (int)q.N;
+        a.K = (int)q.K;
+        a.alpha = q.alpha;
+        a.beta = q.beta;
+        a.X = static_cast<const double *>(swap ? q.B : q.A);
+        a.Y = static_cast<const double *>(swap ? q.A : q.B);
+        a.C = static_cast<double *>(q.C);
+        a.xm = swap ? q.bn : q.am;
+        a.ym = swap ? q.am : q.bn;
+        a.cx = swap ? q.cn : q.cm;
+        a.cy = swap ? q.cm : q.cn;
+        a.xk = make_kmap(swap ? q.bk : q.ak, 16 * W);
+        a.yk = make_kmap(swap ? q.ak : q.bk, 16 * W);
+        a.batches = q.batches;
+        a.flags = (int)q.flags;
+        const int64_t local = t - q.tile_begin, per_batch = q.tiles_m * q.tiles_n;
+        const int64_t batch = local / per_batch, r = local - batch * per_batch;
+        __syncthreads();  // the previous tile's sums may still be read
+        skinny_tile<double, FX, FY, W>(a, batch, (int)(r % q.tiles_m), (int)(r / q.tiles_m), smem);
+    }
+}
+
 template <int BM, int BN, int STAGES> struct GroupedLauncher {
     template <bool AK, bool BN_, bool CM>
     static int go(int64_t grid, const dcc_gemm_problem *probs, int nprob, int64_t total, hipStream_t s) {
@@ -104,6 +149,18 @@ template <int BM, int BN, int STAGES> struct GroupedLauncher {
     }
 };
 
+// Extents and index maps that every entry of a group must have.
+int check_problem(const dcc_gemm_problem &p) {
+    DCC_CHECK(p.N >= 0 && p.K >= 0 && p.nbatch >= 0 && p.max_rows >= 0, "negative extent");
+    DCC_CHECK(p.N < ((int64_t)1 << 31) && p.K < ((int64_t)1 << 31), "extent exceeds 2^31");
+    DCC_CHECK(p.ak.table == nullptr && p.bk.table == nullptr, "K index maps must be mixed-radix maps");
+    for (const dcc_idxmap *m : {&p.am, &p.ak, &p.bk, &p.bn, &p.cm, &p.cn})
+        DCC_CHECK(m->table != nullptr ? m->table_bstride >= 0
+                                      : m->e1 >= 1 && m->e2 >= 1 && m->e1 * m->e2 < ((int64_t)1 << 32),
+                  "invalid index map");
+    return 0;
+}
+
 // Loader/epilogue choice of one problem, as dcc_contract_f64 makes it.
 int problem_flags(const dcc_gemm_problem &p) {
     const bool a_kfast = inner_stride(p.ak) == 1 || inner_stride(p.am) != 1;
@@ -127,13 +184,7 @@ int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_sha
     double weight[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int64_t i = 0; i < nprob; ++i) {
         const dcc_gemm_problem &p = probs[i];
-        DCC_CHECK(p.N >= 0 && p.K >= 0 && p.nbatch >= 0 && p.max_rows >= 0, "negative extent");
-        DCC_CHECK(p.N < ((int64_t)1 << 31) && p.K < ((int64_t)1 << 31), "extent exceeds 2^31");
-        DCC_CHECK(p.ak.table == nullptr && p.bk.table == nullptr, "K index maps must be mixed-radix maps");
-        for (const dcc_idxmap *m : {&p.am, &p.ak, &p.bk, &p.bn, &p.cm, &p.cn})
-            DCC_CHECK(m->table != nullptr ? m->table_bstride >= 0
-                                          : m->e1 >= 1 && m->e2 >= 1 && m->e1 * m->e2 < ((int64_t)1 << 32),
-                      "invalid index map");
+        if (const int st = check_problem(p)) return st;
         weight[problem_flags(p)] += (double)p.N * (double)p.K * (double)p.max_rows * (double)p.nbatch;
     }
     const int flags = (int)(std::max_element(weight, weight + 8) - weight);
@@ -155,18 +206,58 @@ int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_sha
     return 0;
 }
 
+int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *total_tiles, int64_t *variant) {
+    DCC_CHECK(nprob >= 0 && total_tiles != nullptr && variant != nullptr, "bad arguments");
+    DCC_CHECK(nprob == 0 || probs != nullptr, "null problems");
+    SkinnySize z;
+    for (int64_t i = 0; i < nprob; ++i) {
+        const dcc_gemm_problem &p = probs[i];
+        if (const int st = check_problem(p)) return st;
+        if (problem_flags(p) & 4) z.add(p.N, p.max_rows, p.K, p.nbatch);
+        else z.add(p.max_rows, p.N, p.K, p.nbatch);
+    }
+    const int v = skinny_variant(z);
+    if (v < 0) return dcc_grouped_prepare(probs, nprob, 0, total_tiles, variant);
+    int64_t acc = 0;
+    for (int64_t i = 0; i < nprob; ++i) {
+        dcc_gemm_problem &p = probs[i];
+        const bool swap = problem_flags(p) & 4;   // C contiguous along m
+        const int64_t rx = swap ? p.N : p.max_rows, ry = swap ? p.max_rows : p.N;
+        p.tiles_m = (rx + 16 * kSkinny[v].fx - 1) / (16 * kSkinny[v].fx);
+        p.tiles_n = (ry + 16 * kSkinny[v].fy - 1) / (16 * kSkinny[v].fy);
+        p.tile_begin = acc;
+        p.flags = swap ? skinny_flags(p.B, p.bn, p.bk, p.A, p.am, p.ak, p.K, true, sizeof(double), kSkinny[v].w)
+                       : skinny_flags(p.A, p.am, p.ak, p.B, p.bn, p.bk, p.K, false, sizeof(double), kSkinny[v].w);
+        acc += p.nbatch * p.tiles_m * p.tiles_n;
+    }
+    DCC_CHECK(acc < ((int64_t)1 << 40), "too many tiles");
+    *total_tiles = acc;
+    *variant = kSkinnyBase + v;
+    return 0;
+}
+
 int dcc_contract_grouped_f64(const dcc_gemm_problem *probs, int64_t nprob, int64_t total_tiles, int64_t variant,
                              int64_t nworkgroups, dcc_stream_t stream) {
     DCC_CHECK(nprob >= 0 && total_tiles >= 0 && nworkgroups >= 0, "negative argument");
     DCC_CHECK(nprob < (1 << 30), "too many problems");
-    DCC_CHECK(variant >= 0 && variant < 64, "variant must come from dcc_grouped_prepare");
+    DCC_CHECK(variant >= 0 && variant < kSkinnyBase + kSkinnyVariants, "variant must come from dcc_grouped_prepare");
     if (nprob == 0 || total_tiles == 0) return 0;
     DCC_CHECK(probs != nullptr, "null problems");
+    hipStream_t s = dcc::as_stream(stream);
+    const int np = (int)nprob;
+    if (variant >= kSkinnyBase)
+        return skinny_dispatch((int)(variant - kSkinnyBase), [&](auto fx, auto fy, auto w) {
+            constexpr int FX = decltype(fx)::value, FY = decltype(fy)::value, W = decltype(w)::value;
+            // one workgroup per tile unless the caller fixes the grid: a tile's start-up is short
+            const int64_t grid = std::min(nworkgroups > 0 ? nworkgroups : int64_t(1) << 20, total_tiles);
+            hipLaunchKernelGGL((grouped_skinny_kernel<FX, FY, W>), dim3((unsigned)grid), dim3(W * 64), 0, s, probs, np,
+                               total_tiles);
+            DCC_LAUNCH_CHECK();
+            return 0;
+        });
     int bm = 0, bn = 0, stages = 0;
     tile_shape_of(variant & 7, bm, bn, stages);
     const int flags = (int)(variant >> 3);
-    hipStream_t s = dcc::as_stream(stream);
-    const int np = (int)nprob;
     if (bm == 64 && bn == 64)
         return stages == 2 ? GroupedLauncher<64, 64, 2>::run(flags, nworkgroups, probs, np, total_tiles, s)
                            : GroupedLauncher<64, 64, 1>::run(flags, nworkgroups, probs, np, total_tiles, s);

@@ -9,7 +9,8 @@ operands from the intermediates, R reset, Y gather, all grouped GEMMs, all final
 graph, so a step is one graph launch.  ``BatchedRCCSDT`` does the same for whole RCCSDT iterations
 (lower order, T3 -> r1/r2/W, triples residual, update and energy of every system); there the
 contractions of the lower-order part are grouped the same way, operation by operation.
-``autotune()`` times the eight tile variants of the grouped kernel for every term and keeps the fastest.
+Every group starts on the tile the library chooses for its sizes; ``autotune()`` times that and the eight tile
+variants of the grouped kernel for every term and keeps the fastest.
 """
 import ctypes
 
@@ -17,10 +18,10 @@ import numpy as np
 
 from distr_cc import _lib as L
 from distr_cc.device import DeviceArray, Event
-from distr_cc.t3_engine import GemmLaunch, TriplesEngine
+from distr_cc.t3_engine import GemmLaunch, LIBRARY_TILE, TriplesEngine
 
 TILE_SHAPES = {0: "64x64", 1: "128x64", 2: "64x128", 3: "128x128",
-               4: "64x64s1", 5: "128x64s1", 6: "64x128s1", 7: "128x128s1"}
+               4: "64x64s1", 5: "128x64s1", 6: "64x128s1", 7: "128x128s1", LIBRARY_TILE: "library"}
 
 
 class _GroupedPhase:
@@ -28,7 +29,7 @@ class _GroupedPhase:
         self.launches = launches
         self.name = launches[0].name
         self.flops = sum(g.flops for g in launches)
-        self.tile = 0
+        self.tile = LIBRARY_TILE
         self.variant = 0
         self.dev = None
         self.total = 0
@@ -47,8 +48,11 @@ class _GroupedPhase:
     def prepare(self, tile, stream):
         arr = self.problems()
         total, variant = ctypes.c_int64(), ctypes.c_int64()
-        L.call("dcc_grouped_prepare", ctypes.cast(arr, ctypes.c_void_p), len(arr), int(tile), ctypes.byref(total),
-               ctypes.byref(variant))
+        ptr = ctypes.cast(arr, ctypes.c_void_p)
+        if tile == LIBRARY_TILE:
+            L.call("dcc_grouped_prepare_auto", ptr, len(arr), ctypes.byref(total), ctypes.byref(variant))
+        else:
+            L.call("dcc_grouped_prepare", ptr, len(arr), int(tile), ctypes.byref(total), ctypes.byref(variant))
         self.tile, self.total, self.variant = int(tile), int(total.value), int(variant.value)
         host = np.frombuffer(bytes(arr), dtype=np.uint8).copy()
         if self.dev is not None:
@@ -77,7 +81,7 @@ class _Grouped:
             items = [e.launches[p] for e in tr_engines]
             if all(isinstance(g, GemmLaunch) for g in items):
                 ph = _GroupedPhase(items)
-                ph.prepare(0, stream)
+                ph.prepare(LIBRARY_TILE, stream)
                 self.phases.append(ph)
             else:
                 self.phases.append(items)
@@ -215,7 +219,7 @@ class BatchedRCCSDT(_Grouped):
             heads = [op[0] for op in ops]
             if all(isinstance(h, GemmLaunch) and h.fn == "dcc_contract_f64" for h in heads):
                 ph = _GroupedPhase(heads)
-                ph.prepare(0, self.stream)
+                ph.prepare(LIBRARY_TILE, self.stream)
                 self.lower_phases.append(ph)
                 self.lower_plan.append((ph, [op[1:] for op in ops]))
             else:

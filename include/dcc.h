@@ -475,9 +475,13 @@ typedef void *dcc_graph_t;
 int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_shape, int64_t *total_tiles,
                         int64_t *variant);
 
+/* The same with the tile the library chooses for the sizes of the whole group: 64x64, or the tiles of
+ * dcc_contract_f64 for few or narrow outputs. */
+int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *total_tiles, int64_t *variant);
+
 /* Persistent grouped FP64 gather-GEMM over a device array of prepared problems whose C regions are
- * disjoint; variant from dcc_grouped_prepare; nworkgroups = 0 launches as many workgroups as are
- * resident at once.  Every workgroup exits when the tile list is exhausted. */
+ * disjoint; variant from dcc_grouped_prepare or dcc_grouped_prepare_auto; nworkgroups = 0 launches as many
+ * workgroups as are resident at once (one per tile for the tiles of few or narrow outputs).  Every workgroup exits when the tile list is exhausted. */
 int dcc_contract_grouped_f64(const dcc_gemm_problem *probs, int64_t nprob, int64_t total_tiles,
                              int64_t variant, int64_t nworkgroups, dcc_stream_t stream);
 

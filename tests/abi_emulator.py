@@ -126,6 +126,9 @@ class Emulator:
         pvariant._obj.value = int(tile)
         return 0
 
+    def dcc_grouped_prepare_auto(self, probs, nprob, ptotal, pvariant):
+        return self.dcc_grouped_prepare(probs, nprob, 0, ptotal, pvariant)
+
     def dcc_contract_grouped_f64(self, probs, nprob, total, variant, nwg, stream):
         if not 0 <= int(variant) < 64:
             raise AssertionError("variant must come from dcc_grouped_prepare")
