@@ -649,8 +649,8 @@ int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, c
     hipStream_t s = dcc::as_stream(stream);
     // Workgroup tile: tile_shape 0..3 = 64x64, 128x64, 64x128, 128x128 with the two-stage register
     // prefetch, 4..7 = the same shapes with one stage; -1 = DCC_CONTRACT_TILE (e.g. "128x64" or
-    // "64x64s1") when set, otherwise a skinny variant where skinny_variant gives one and 64x64 two-stage
-    // elsewhere.
+    // "64x64s1") when set, otherwise a skinny variant where skinny_variant gives one and the shape of
+    // TileChoice elsewhere.
     static const char *tile_env = getenv("DCC_CONTRACT_TILE");
     int tbm = 64, tbn = 64, stages = 2;
     if (tile_shape >= 0) {
@@ -669,6 +669,9 @@ int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, c
         else z.add(max_rows, N, K, nbatch);
         const int v = skinny_variant(z);
         if (v >= 0) return contract_skinny<T>(args, ak, bk, c_mfast, nbatch, max_rows, v, s);
+        TileChoice tc;
+        tc.add(max_rows, N, K, nbatch);
+        tile_shape_of(tc.pick(std::is_same<T, double>::value, a_kfast, b_nfast), tbm, tbn, stages);
     }
     if (tbm == 128 && tbn == 128) return launch<T, 128, 128>(args, max_rows, a_kfast, b_nfast, c_mfast, stages, s);
     if (tbm == 128 && tbn == 64) return launch<T, 128, 64>(args, max_rows, a_kfast, b_nfast, c_mfast, stages, s);
@@ -729,6 +732,31 @@ int run_bf16x3(ContractArgs<float> &args, int64_t nbatch, int64_t max_rows, bool
     return 0;
 }
 
+// Tile shape of a split-BF16x3 launch without one: rounds of resident workgroups times area over rate, as
+// TileChoice.  Rates relative to 128x128 at equal padding, from the launches of one residual at nocc=12,
+// nvir=120 and nocc=9, nvir=71: 256x256 gains most where operands load as 16-byte vectors or K is long
+// (W_vvvv pairs 28.5 -> 22.4 ms, ring 31.1 -> 27.5 ms) and little on short, unaligned K (K = 639: 1.95 ms
+// against 2.19 with the padding of 639 rows); 256x128 suits one side of at most 128 (t3 -> W_vvvo 642 ->
+// 534 us).
+int pick_bf16x3(int64_t rows, int64_t N, int64_t K, int64_t nbatch, bool quads) {
+    static const int shapes[7][4] = {{0, 64, 64, 512},     {1, 128, 64, 512},  {2, 64, 128, 512}, {3, 128, 128, 512},
+                                     {9, 256, 128, 256}, {10, 128, 256, 256}, {8, 256, 256, 256}};
+    const double rate[7] = {0.73, 0.8, 0.8, 1.0, 1.08, 1.03, quads || K >= 1024 ? 1.25 : 1.15};
+    int best = 3;
+    double least = 0.0;
+    for (int c = 0; c < 7; ++c) {
+        const int64_t bm = shapes[c][1], bn = shapes[c][2], slots = shapes[c][3];
+        const int64_t tiles = nbatch * ((rows + bm - 1) / bm) * ((N + bn - 1) / bn);
+        const double rounds = tiles < slots ? 1.0 : (double)tiles / (double)slots;
+        const double cost = rounds * (double)(slots * bm * bn) / rate[c];
+        if (least == 0.0 || cost < least) {
+            least = cost;
+            best = shapes[c][0];
+        }
+    }
+    return best;
+}
+
 int contract_bf16x3_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, const float *A,
                           dcc_idxmap am, dcc_idxmap ak, const float *B, dcc_idxmap bk, dcc_idxmap bn, float *C,
                           dcc_idxmap cm, dcc_idxmap cn, const dcc_batch *batches, int64_t nbatch,
@@ -773,9 +801,8 @@ int contract_bf16x3_entry(int64_t M, int64_t N, int64_t K, double alpha, double 
     // written as vectors by the register-staged tiles)
     if (!c_mfast && vectors_contiguous(C, cm, cn, true, 0, 4, 16)) args.vec |= 4;
     hipStream_t s = dcc::as_stream(stream);
-    // default: 128x128 unless one side of the problem is small
     int shape = (int)tile_shape;
-    if (shape < 0) shape = (max_rows <= 64 ? 0 : 1) + (N <= 64 ? 0 : 2);
+    if (shape < 0) shape = pick_bf16x3(max_rows, N, K, nbatch, mode == 2);
     // shapes 8..13: direct-to-LDS staging, for packed quads with both operands K-contiguous and K a
     // multiple of 32 x stages; otherwise the register-staged kernel of the same tile
     const int stages = (shape == 9 || shape == 10) ? 3 : 2;

@@ -452,4 +452,57 @@ inline bool tile_shape_of(int64_t id, int &bm, int &bn, int &stages) {
     return true;
 }
 
+// Choice of a tile shape for a launch without one: per candidate the rounds of resident workgroups its
+// tiles take, times the tile's area over its rate.  Rates are relative to the 64x64 one-stage tile at
+// equal padding and depend on the layouts (which operand is staged K-contiguous), measured on the launches
+// of one residual: FP64 at nocc=10, nvir=90 and nocc=8, nvir=38, FP32 at nocc=8, nvir=67.  The taller tile
+// pays where A is K-contiguous (ring GEMM 28.4 -> 27.5 ms in FP64 although 900 rows pad to 1024, 3.27 ->
+// 2.96 ms in FP32), the wider one where A is row-contiguous (W_oooo 9.1 -> 8.2 ms), 128x128 where both are
+// K-contiguous and K is long (W_vvvv pairs 22.7 -> 20.6 ms); short K and few rounds stay on 64x64, whose
+// one-stage form keeps four workgroups per CU (T2->T3 at K = 46: 201 -> 154 us against two stages).
+struct TileChoice {
+    int64_t tiles[8] = {};
+    int64_t K = 0;
+    void add(int64_t rows, int64_t n, int64_t k, int64_t nbatch) {
+        for (int id = 0; id < 8; ++id) {
+            int bm, bn, st;
+            tile_shape_of(id, bm, bn, st);
+            tiles[id] += nbatch * ((rows + bm - 1) / bm) * ((n + bn - 1) / bn);
+        }
+        K = k > K ? k : K;
+    }
+    int pick(bool f64, bool a_kfast, bool b_nfast) const {
+        double rate[8] = {};   // 0: not a candidate
+        rate[4] = 1.0;
+        if (a_kfast && !b_nfast) {
+            rate[6] = f64 ? 1.0 : 1.06;
+            if (K >= 1024) {
+                rate[0] = 1.02;
+                rate[3] = f64 ? 1.08 : 1.16;
+            }
+        } else if (f64) {
+            rate[5] = a_kfast ? 1.09 : 1.05;
+            rate[6] = a_kfast ? 1.0 : 1.11;
+        } else {
+            rate[5] = 1.2;
+            rate[7] = 1.19;
+        }
+        static const int per_cu[8] = {3, 3, 3, 2, 4, 3, 3, 2};   // resident workgroups
+        int best = 4;
+        double least = 0.0;
+        for (int id = 0; id < 8; ++id) {
+            if (rate[id] == 0.0) continue;
+            int bm, bn, st;
+            tile_shape_of(id, bm, bn, st);
+            const int64_t slots = 256 * per_cu[id];
+            const double cost = (double)((tiles[id] + slots - 1) / slots) * (double)(slots * bm * bn) / rate[id];
+            if (least == 0.0 || cost < least) {
+                least = cost;
+                best = id;
+            }
+        }
+        return best;
+    }
+};
+
 }  // namespace dcc_gemm

@@ -169,6 +169,17 @@ int problem_flags(const dcc_gemm_problem &p) {
     return (a_kfast ? 1 : 0) | (b_nfast ? 2 : 0) | (c_mfast ? 4 : 0);
 }
 
+// The loaders and epilogue are correct for any strides; their choice only decides coalescing.  One launch
+// has one choice: the one of the problems with the most multiply-adds.
+int group_flags(const dcc_gemm_problem *probs, int64_t nprob) {
+    double weight[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int64_t i = 0; i < nprob; ++i) {
+        const dcc_gemm_problem &p = probs[i];
+        weight[problem_flags(p)] += (double)p.N * (double)p.K * (double)p.max_rows * (double)p.nbatch;
+    }
+    return (int)(std::max_element(weight, weight + 8) - weight);
+}
+
 }  // namespace
 
 extern "C" {
@@ -179,15 +190,9 @@ int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_sha
     DCC_CHECK(nprob == 0 || probs != nullptr, "null problems");
     int bm = 0, bn = 0, stages = 0;
     DCC_CHECK(tile_shape_of(tile_shape_id, bm, bn, stages), "tile shape must be 0..7");
-    // The loaders and epilogue are correct for any strides; their choice only decides coalescing.
-    // One launch has one choice: the one of the problems with the most multiply-adds.
-    double weight[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int64_t i = 0; i < nprob; ++i) {
-        const dcc_gemm_problem &p = probs[i];
-        if (const int st = check_problem(p)) return st;
-        weight[problem_flags(p)] += (double)p.N * (double)p.K * (double)p.max_rows * (double)p.nbatch;
-    }
-    const int flags = (int)(std::max_element(weight, weight + 8) - weight);
+    for (int64_t i = 0; i < nprob; ++i)
+        if (const int st = check_problem(probs[i])) return st;
+    const int flags = group_flags(probs, nprob);
     const bool a_kfast = flags & 1, b_nfast = (flags & 2) != 0;
     int64_t acc = 0;
     for (int64_t i = 0; i < nprob; ++i) {
@@ -217,7 +222,12 @@ int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *to
         else z.add(p.max_rows, p.N, p.K, p.nbatch);
     }
     const int v = skinny_variant(z);
-    if (v < 0) return dcc_grouped_prepare(probs, nprob, 0, total_tiles, variant);
+    if (v < 0) {
+        TileChoice tc;
+        for (int64_t i = 0; i < nprob; ++i) tc.add(probs[i].max_rows, probs[i].N, probs[i].K, probs[i].nbatch);
+        const int flags = group_flags(probs, nprob);
+        return dcc_grouped_prepare(probs, nprob, tc.pick(true, flags & 1, (flags & 2) != 0), total_tiles, variant);
+    }
     int64_t acc = 0;
     for (int64_t i = 0; i < nprob; ++i) {
         dcc_gemm_problem &p = probs[i];
