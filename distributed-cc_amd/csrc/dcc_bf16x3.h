@@ -356,9 +356,9 @@ void contract_bf16x3_dma_kernel(const ContractArgs<float> p) {
     __shared__ __align__(16) uint32_t sa0[AW], sb0[BW], sa1[AW], sb1[BW];
     __shared__ __align__(16) uint32_t sa2[S == 3 ? AW : 4], sb2[S == 3 ? BW : 4];
     __shared__ int64_t ktab[S][2][kBK3];
-    const int64_t L = xcd_remap((int64_t)blockIdx.x, p.total_tiles);
-    const int64_t per_batch = (int64_t)p.tiles_m * p.tiles_n;
-    const int64_t batch = L / per_batch;
+    const uint32_t L = xcd_remap32(blockIdx.x, (uint32_t)p.total_tiles);
+    const uint32_t per_batch = (uint32_t)p.tiles_m * (uint32_t)p.tiles_n;
+    const uint32_t batch = L / per_batch;
     int tm, tn;
     tile_coords(L - batch * per_batch, p.tiles_m, p.tiles_n, tm, tn);
     const dcc_batch bt = p.batches[batch];

@@ -57,6 +57,36 @@ __host__ __device__ inline KMap make_kmap(const dcc_idxmap &m, uint32_t step = 1
     return k;
 }
 
+// The reciprocals of a map in the unused table stride of a prepared K map (its table is null), and the KMap
+// of such a map: the two 64-bit divisions of make_kmap, once on the host instead of once per tile.
+inline void store_magic(dcc_idxmap &m) {
+    uint32_t mul2, mul12, sh;
+    magic((uint32_t)m.e2, mul2, sh);
+    magic((uint32_t)(m.e1 * m.e2), mul12, sh);
+    m.table_bstride = (int64_t)((uint64_t)mul2 | (uint64_t)mul12 << 32);
+}
+
+__device__ __forceinline__ KMap make_kmap_prepared(const dcc_idxmap &m, uint32_t step) {
+    KMap k;
+    k.s0 = m.s0;
+    k.s1 = m.s1;
+    k.s2 = m.s2;
+    k.e1 = (uint32_t)m.e1;
+    k.e2 = (uint32_t)m.e2;
+    k.e12 = k.e1 * k.e2;
+    k.mul2 = (uint32_t)m.table_bstride;
+    k.mul12 = (uint32_t)((uint64_t)m.table_bstride >> 32);
+    k.sh2 = 31 + (k.e2 > 1 ? 32 - __clz(k.e2 - 1) : 0);   // ceil(log2)
+    k.sh12 = 31 + (k.e12 > 1 ? 32 - __clz(k.e12 - 1) : 0);
+    const uint32_t q = step / k.e2;
+    k.d2 = step - q * k.e2;
+    k.d1 = q % k.e1;
+    k.doff = (int64_t)(step / k.e12) * m.s0 + (int64_t)k.d1 * m.s1 + (int64_t)k.d2 * m.s2;
+    k.c2 = m.s1 - (int64_t)k.e2 * m.s2;
+    k.c1 = m.s0 - (int64_t)k.e1 * m.s1;
+    return k;
+}
+
 // Offset of index k under the map, kept up to date while k advances by the map's step.
 struct KIter {
     int64_t off;

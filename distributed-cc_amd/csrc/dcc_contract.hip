@@ -19,9 +19,9 @@ template <typename T, int BM, int BN, bool A_KFAST, bool B_NFAST, bool C_MFAST, 
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(MinWaves<BM, BN, STAGES>::v)))
 void contract_kernel(const ContractArgs<T> p) {
     __shared__ T smem[TileSmem<BM, BN, C_MFAST>::v];
-    const int64_t L = xcd_remap((int64_t)blockIdx.x, p.total_tiles);
-    const int64_t per_batch = (int64_t)p.tiles_m * p.tiles_n;
-    const int64_t batch = L / per_batch;
+    const uint32_t L = xcd_remap32(blockIdx.x, (uint32_t)p.total_tiles);
+    const uint32_t per_batch = (uint32_t)p.tiles_m * (uint32_t)p.tiles_n;
+    const uint32_t batch = L / per_batch;
     int tm, tn;
     tile_coords(L - batch * per_batch, p.tiles_m, p.tiles_n, tm, tn);
     contract_tile<T, BM, BN, A_KFAST, B_NFAST, C_MFAST, STAGES>(p, batch, tm, tn, smem);
@@ -31,10 +31,10 @@ void contract_kernel(const ContractArgs<T> p) {
 template <typename T, int FX, int FY, int W>
 __global__ __launch_bounds__(W * 64) void skinny_kernel(const SkinnyArgs<T> p) {
     __shared__ T smem[SkinnySmem<T, FX, FY, W>::v];
-    const int64_t L = xcd_remap((int64_t)blockIdx.x, p.total_tiles);
-    const int64_t per_batch = (int64_t)p.tiles_x * p.tiles_y;
-    const int64_t batch = L / per_batch, t = L - batch * per_batch;
-    skinny_tile<T, FX, FY, W>(p, batch, (int)(t % p.tiles_x), (int)(t / p.tiles_x), smem);
+    const uint32_t L = xcd_remap32(blockIdx.x, (uint32_t)p.total_tiles);
+    const uint32_t per_batch = (uint32_t)p.tiles_x * (uint32_t)p.tiles_y;
+    const uint32_t batch = L / per_batch, t = L - batch * per_batch, ty = t / (uint32_t)p.tiles_x;
+    skinny_tile<T, FX, FY, W>(p, batch, (int)(t - ty * (uint32_t)p.tiles_x), (int)ty, smem);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -150,17 +150,11 @@ void contract_bf16x3_kernel(const ContractArgs<float> p) {
     unsigned short *const lds = reinterpret_cast<unsigned short *>(smem);
 
     const int tid = threadIdx.x;
-    const int64_t L = xcd_remap((int64_t)blockIdx.x, p.total_tiles);
-    const int64_t per_batch = (int64_t)p.tiles_m * p.tiles_n;
-    const int64_t batch = L / per_batch;
-    const int64_t pid = L - batch * per_batch;
-    const int64_t group_span = (int64_t)kGroupM * p.tiles_n;
-    const int64_t group = pid / group_span;
-    const int first_m = (int)(group * kGroupM);
-    const int gsize = min(p.tiles_m - first_m, kGroupM);
-    const int64_t in_group = pid - group * group_span;
-    const int tm = first_m + (int)(in_group % gsize);
-    const int tn = (int)(in_group / gsize);
+    const uint32_t L = xcd_remap32(blockIdx.x, (uint32_t)p.total_tiles);
+    const uint32_t per_batch = (uint32_t)p.tiles_m * (uint32_t)p.tiles_n;
+    const uint32_t batch = L / per_batch;
+    int tm, tn;
+    tile_coords(L - batch * per_batch, p.tiles_m, p.tiles_n, tm, tn);
 
     const dcc_batch bt = p.batches[batch];
     const int64_t m0 = bt.m_begin + (int64_t)tm * BM;

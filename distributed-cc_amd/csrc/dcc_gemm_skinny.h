@@ -81,6 +81,20 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
     const bool vy = (p.flags & kSkinnyPairY) && ((swap ? bt.a_off : bt.b_off) & 1) == 0;
     const bool sx = p.flags & kSkinnyStepX, sy = p.flags & kSkinnyStepY;
 
+    // this thread's elements of C, their old values loaded while the products run
+    constexpr int NE = (FX * FY * 256 + W * 64 - 1) / (W * 64);
+    T *c[NE];
+    T old[NE];
+#pragma unroll
+    for (int n = 0; n < NE; ++n) {
+        const int e = tid + n * W * 64, f = e / 256, r = e / 64 % 4, el = e % 64;
+        const int64_t x = x0 + f / FY * 16 + MF::row(el / 16, r), y = y0 + f % FY * 16 + el % 16;
+        c[n] = e < FX * FY * 256 && x < xe && y < ye
+                   ? p.C + bt.c_off + map_off(p.cx, (uint32_t)x, batch) + map_off(p.cy, (uint32_t)y, batch)
+                   : nullptr;
+        old[n] = p.beta != 0.0 && c[n] != nullptr ? *c[n] : T(0);
+    }
+
     typedef T T2 __attribute__((ext_vector_type(2)));
     // 4 values of every fragment, zero beyond K: at k .. k+3, or with one wave k, k+4, k+8, k+12
     constexpr int KS = W == 1 ? 4 : 1;
@@ -158,17 +172,16 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
 #pragma unroll
             for (int r = 0; r < 4; ++r) smem[((w * FX * FY + i * FY + j) * 4 + r) * 64 + lane] = acc[i][j][r];
     __syncthreads();
-    for (int e = tid; e < FX * FY * 256; e += W * 64) {
-        const int f = e / 256, r = e / 64 % 4, el = e % 64;
-        const int64_t x = x0 + f / FY * 16 + MF::row(el / 16, r), y = y0 + f % FY * 16 + el % 16;
-        if (x >= xe || y >= ye) continue;
+#pragma unroll
+    for (int n = 0; n < NE; ++n) {
+        if (c[n] == nullptr) continue;
+        const int e = tid + n * W * 64;
         T sum = smem[e];
 #pragma unroll
         for (int q = 1; q < W; ++q) sum += smem[q * FX * FY * 256 + e];
-        T *c = p.C + bt.c_off + map_off(p.cx, (uint32_t)x, batch) + map_off(p.cy, (uint32_t)y, batch);
         double v = p.alpha * (double)sum;
-        if (p.beta != 0.0) v += p.beta * (double)*c;
-        *c = (T)v;
+        if (p.beta != 0.0) v += p.beta * (double)old[n];
+        *c[n] = (T)v;
     }
 }
 

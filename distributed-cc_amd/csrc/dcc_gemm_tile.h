@@ -88,15 +88,22 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t L, int64_t total) {
     return (xcd < r) ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
 }
 
+// The same for a launch (fewer than 2^31 workgroups) in 32-bit arithmetic: a 64-bit division costs a
+// workgroup's start some 0.4 us, which is most of a small launch.
+__device__ __forceinline__ uint32_t xcd_remap32(uint32_t L, uint32_t total) {
+    const uint32_t q = total / 8, r = total % 8, xcd = L % 8, local = L / 8;
+    return (xcd < r) ? xcd * (q + 1) + local : r * (q + 1) + (xcd - r) * q + local;
+}
+
 // Tile (tm, tn) of tile pid within one batch: kGroupM row tiles advance together along N.
-__device__ __forceinline__ void tile_coords(int64_t pid, int tiles_m, int tiles_n, int &tm, int &tn) {
-    const int64_t group_span = (int64_t)kGroupM * tiles_n;
-    const int64_t group = pid / group_span;
-    const int first_m = (int)(group * kGroupM);
-    const int gsize = min(tiles_m - first_m, kGroupM);
-    const int64_t in_group = pid - group * group_span;
-    tm = first_m + (int)(in_group % gsize);
+__device__ __forceinline__ void tile_coords(uint32_t pid, int tiles_m, int tiles_n, int &tm, int &tn) {
+    const uint32_t group_span = (uint32_t)(kGroupM * tiles_n);
+    const uint32_t group = pid / group_span;
+    const uint32_t first_m = group * kGroupM;
+    const uint32_t gsize = min((uint32_t)tiles_m - first_m, (uint32_t)kGroupM);
+    const uint32_t in_group = pid - group * group_span;
     tn = (int)(in_group / gsize);
+    tm = (int)(first_m + (in_group - (uint32_t)tn * gsize));
 }
 
 template <int a, int b> struct CMax { static constexpr int v = a > b ? a : b; };

@@ -54,16 +54,16 @@ void grouped_kernel(const dcc_gemm_problem *__restrict__ probs, int nprob, int64
         a.bn = q.bn;
         a.cm = q.cm;
         a.cn = q.cn;
-        a.ak = make_kmap(q.ak);
-        a.bk = make_kmap(q.bk);
+        a.ak = dcc::make_kmap_prepared(q.ak, kBK);
+        a.bk = dcc::make_kmap_prepared(q.bk, kBK);
         a.batches = q.batches;
         a.tiles_m = (int)q.tiles_m;
         a.tiles_n = (int)q.tiles_n;
         a.total_tiles = 0;
         a.vec = (int)((q.flags >> 3) & 3);
-        const int64_t local = t - q.tile_begin;
-        const int64_t per_batch = q.tiles_m * q.tiles_n;
-        const int64_t batch = local / per_batch;
+        const uint32_t local = (uint32_t)(t - q.tile_begin);   // a problem has fewer than 2^31 tiles
+        const uint32_t per_batch = (uint32_t)(q.tiles_m * q.tiles_n);
+        const uint32_t batch = local / per_batch;
         int tm, tn;
         tile_coords(local - batch * per_batch, a.tiles_m, a.tiles_n, tm, tn);
         __syncthreads();  // the previous tile's epilogue may still read LDS
@@ -102,14 +102,14 @@ __global__ __launch_bounds__(W * 64) void grouped_skinny_kernel(const dcc_gemm_p
         a.ym = swap ? q.am : q.bn;
         a.cx = swap ? q.cn : q.cm;
         a.cy = swap ? q.cm : q.cn;
-        a.xk = make_kmap(swap ? q.bk : q.ak, 16 * W);
-        a.yk = make_kmap(swap ? q.ak : q.bk, 16 * W);
+        a.xk = dcc::make_kmap_prepared(swap ? q.bk : q.ak, 16 * W);
+        a.yk = dcc::make_kmap_prepared(swap ? q.ak : q.bk, 16 * W);
         a.batches = q.batches;
         a.flags = (int)q.flags;
-        const int64_t local = t - q.tile_begin, per_batch = q.tiles_m * q.tiles_n;
-        const int64_t batch = local / per_batch, r = local - batch * per_batch;
+        const uint32_t local = (uint32_t)(t - q.tile_begin), per_batch = (uint32_t)(q.tiles_m * q.tiles_n);
+        const uint32_t batch = local / per_batch, r = local - batch * per_batch, ty = r / (uint32_t)q.tiles_m;
         __syncthreads();  // the previous tile's sums may still be read
-        skinny_tile<double, FX, FY, W>(a, batch, (int)(r % q.tiles_m), (int)(r / q.tiles_m), smem);
+        skinny_tile<double, FX, FY, W>(a, batch, (int)(r - ty * (uint32_t)q.tiles_m), (int)ty, smem);
     }
 }
 
@@ -203,6 +203,9 @@ int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_sha
         const int vec = (pairs_contiguous(p.A, p.am, p.ak, a_kfast, 0, 16) ? 1 : 0) |
                         (pairs_contiguous(p.B, p.bn, p.bk, !b_nfast, p.N, 16) ? 2 : 0);
         p.flags = flags | (vec << 3);
+        dcc::store_magic(p.ak);
+        dcc::store_magic(p.bk);
+        DCC_CHECK(p.nbatch * p.tiles_m * p.tiles_n < ((int64_t)1 << 31), "too many tiles");
         acc += p.nbatch * p.tiles_m * p.tiles_n;
     }
     DCC_CHECK(acc < ((int64_t)1 << 40), "too many tiles");
@@ -238,6 +241,9 @@ int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *to
         p.tile_begin = acc;
         p.flags = swap ? skinny_flags(p.B, p.bn, p.bk, p.A, p.am, p.ak, p.K, true, sizeof(double), kSkinny[v].w)
                        : skinny_flags(p.A, p.am, p.ak, p.B, p.bn, p.bk, p.K, false, sizeof(double), kSkinny[v].w);
+        dcc::store_magic(p.ak);
+        dcc::store_magic(p.bk);
+        DCC_CHECK(p.nbatch * p.tiles_m * p.tiles_n < ((int64_t)1 << 31), "too many tiles");
         acc += p.nbatch * p.tiles_m * p.tiles_n;
     }
     DCC_CHECK(acc < ((int64_t)1 << 40), "too many tiles");
