@@ -142,6 +142,9 @@ _SIGS = {
     "dcc_graph_destroy": ([c_vp], ctypes.c_int),
     "dcc_sum_slices_f64": ([c_vp, c_vp, c_i64, c_i64, c_dbl, c_dbl, c_vp], ctypes.c_int),
     "dcc_sum_slices_f32": ([c_vp, c_vp, c_i64, c_i64, c_dbl, c_dbl, c_vp], ctypes.c_int),
+    "dcc_diis_partials": ([], c_i64),
+    "dcc_diis_push_f64": ([c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp], ctypes.c_int),
+    "dcc_diis_combine_f64": ([c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp], ctypes.c_int),
     "dcc_dot_partials": ([], c_i64),
     "dcc_dot_f64": ([c_vp, c_vp, c_i64, c_vp, c_vp, c_vp], ctypes.c_int),
     "dcc_dot_f32": ([c_vp, c_vp, c_i64, c_vp, c_vp, c_vp], ctypes.c_int),

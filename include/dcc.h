@@ -441,6 +441,18 @@ int dcc_dot_f64(const double *x, const double *y, int64_t n, double *partials, d
 int dcc_dot_f32(const float *x, const float *y, int64_t n, double *partials, double *out, dcc_stream_t stream);
 
 /*
+ * One DIIS step (distr_cc/diis.py:105-145) in two passes over the history.  Push: xs <- x, errors[head] <-
+ * x - xprev and out[i] = errors[head] . errors[i] for the nvec error vectors.  Combine: xnew <- sum_i coef[i]
+ * vectors[i], out[0] = |xnew - xprev|^2, xprev <- xnew.  The pointer and coefficient lists are host arrays
+ * of nvec entries; partials holds dcc_diis_partials() doubles.  Sums have a fixed order.
+ */
+int64_t dcc_diis_partials(void);
+int dcc_diis_push_f64(const double *x, const double *xprev, double *xs, const double *const *errors, int64_t nvec,
+                      int64_t head, int64_t n, double *partials, double *out, dcc_stream_t stream);
+int dcc_diis_combine_f64(double *xnew, double *xprev, const double *const *vectors, const double *coef, int64_t nvec,
+                         int64_t n, double *partials, double *out, dcc_stream_t stream);
+
+/*
  * rank 1: x[i,a] /= eia[i,a]; rank 2: x[i,j,a,b] /= eia[i,a] + eia[j,b], with
  * eia = e_i - e_a - level_shift (the r1r2_divide_e_ call of distr_cc/rccsdt.py:924).
  */

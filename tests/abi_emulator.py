@@ -432,6 +432,29 @@ class Emulator:
         o[0] = float(X @ Y)
         return 0
 
+    def dcc_diis_partials(self):
+        return 4
+
+    def _host_list(self, arr, n):
+        return list(ctypes.cast(arr, ctypes.POINTER(ctypes.c_void_p))[:int(n)])
+
+    def dcc_diis_push_f64(self, x, xprev, xs, errors, nvec, head, n, partials, out, stream):
+        get = lambda p: self.dev.view(_ptr(p), np.float64, int(n))
+        es = [get(p) for p in self._host_list(errors, nvec)]
+        get(xs)[:] = get(x)
+        es[head][:] = get(x) - get(xprev)
+        self.dev.view(_ptr(out), np.float64, int(nvec))[:] = [es[head] @ e for e in es]
+        return 0
+
+    def dcc_diis_combine_f64(self, xnew, xprev, vectors, coef, nvec, n, partials, out, stream):
+        get = lambda p: self.dev.view(_ptr(p), np.float64, int(n))
+        c = ctypes.cast(coef, ctypes.POINTER(ctypes.c_double))[:int(nvec)]
+        new = sum(ci * get(p) for ci, p in zip(c, self._host_list(vectors, nvec)))
+        self.dev.view(_ptr(out), np.float64, 1)[0] = ((new - get(xprev)) ** 2).sum()
+        get(xnew)[:] = new
+        get(xprev)[:] = new
+        return 0
+
     def dcc_denom_divide_f64(self, x, nocc, nvir, rank, eia, stream):
         o, v = int(nocc), int(nvir)
         E = self.dev.view(_ptr(eia), np.float64, o * v).reshape(o, v)

@@ -291,3 +291,25 @@ def test_device_diis_vs_oracle(dev):
             assert np.all(np.abs(hd - ho) <= 1e-12 * scale)
             cd, co = dd.coefficients(nd), od.coefficients(nd)
             assert np.abs(cd - co).max() <= 1e-9 * np.abs(co).max()
+
+
+@pytest.mark.parametrize("n,space,odd", [(1, 1, False), (257, 3, True), (70001, 8, False), (4099, 11, False),
+                                         (300, 17, True)])
+def test_device_diis_history_sizes_vs_oracle(dev, n, space, odd):
+    """The two-pass DIIS kernels at their edges: one to several launches of eight vectors, odd lengths, a
+    vector that is not 16-byte aligned.  Vectors converge geometrically; both sides solve the same
+    well-conditioned systems, so they agree to the rounding of sums of n products."""
+    from distr_cc.device import DeviceArray
+    from distr_cc.diis import DeviceDIIS
+    from oracle.diis import DIIS
+    _say("DeviceDIIS n=%d space=%d" % (n, space))
+    rng = np.random.default_rng(n + space)
+    dd, od = DeviceDIIS(n, space=space), DIIS(space=space)
+    steps = space + 2 if n > space + 1 else 2
+    buf = DeviceArray((n + 1,))
+    x = DeviceArray((n,), ptr=buf.ptr + (8 if odd else 0), owner=False)
+    for _ in range(steps):
+        v = rng.standard_normal(n)
+        x.upload(v)
+        got, ref = dd.update(x).download(), od.update(v.copy())
+        assert np.abs(got - ref).max() <= 1e-9 * np.abs(ref).max()
