@@ -234,11 +234,12 @@ struct SkinnySize {
 //     16 x 32 tiles from 512 16 x 16 tiles on (1600 x 240 x 240: 17 us against 32).
 //   * K up to 64 there: one wave per 16 x 16 tile (240 x 240 x 36: 10 us against 23).
 //   * above that the staged tiles win (900 x 900 x 900, 225 tiles: 73 us against 80).
-inline int skinny_variant(const SkinnySize &z) {
+// `only`: a variant in any case (groups of many small problems).
+inline int skinny_variant(const SkinnySize &z, bool only = false) {
     const int64_t lo = z.rx < z.ry ? z.rx : z.ry, hi = z.rx < z.ry ? z.ry : z.rx;
     if (lo <= 16 && hi >= 64 && z.K > 64 && (z.t64 > 64 || z.t16 > 512))
         return (z.ry >= z.rx ? 5 : 7) + (z.K > 128 ? 1 : 0);
-    if (z.t64 > 128) return -1;
+    if (z.t64 > 128 && !only) return -1;
     if (z.K <= 64) return 9;
     if (z.t16 > 512) return z.ry >= z.rx ? 3 : 4;
     if (z.t16 > 128) return z.K >= 384 ? 1 : 0;

@@ -214,7 +214,8 @@ int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_sha
     return 0;
 }
 
-int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *total_tiles, int64_t *variant) {
+int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t small, int64_t *total_tiles,
+                             int64_t *variant) {
     DCC_CHECK(nprob >= 0 && total_tiles != nullptr && variant != nullptr, "bad arguments");
     DCC_CHECK(nprob == 0 || probs != nullptr, "null problems");
     SkinnySize z;
@@ -224,7 +225,7 @@ int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *to
         if (problem_flags(p) & 4) z.add(p.N, p.max_rows, p.K, p.nbatch);
         else z.add(p.max_rows, p.N, p.K, p.nbatch);
     }
-    const int v = skinny_variant(z);
+    const int v = skinny_variant(z, small != 0);
     if (v < 0) {
         TileChoice tc;
         for (int64_t i = 0; i < nprob; ++i) tc.add(probs[i].max_rows, probs[i].N, probs[i].K, probs[i].nbatch);

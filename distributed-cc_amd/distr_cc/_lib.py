@@ -56,6 +56,14 @@ BATCH_DTYPE = np.dtype([("a_off", np.int64), ("b_off", np.int64), ("c_off", np.i
                         ("m_begin", np.int64), ("m_end", np.int64)])
 S3JOB_DTYPE = np.dtype([("dst", np.int64), ("src", np.int64), ("coef", np.float64, (6,))])
 S3GATHER_DTYPE = np.dtype([("dst", np.int64), ("src", np.int64, (6,)), ("coef", np.float64, (6,))])
+# dcc_combine_term, dcc_combine_job, dcc_dot_job
+TERM_DTYPE = np.dtype([("src", np.int64), ("stride", np.int64, (4,)), ("coef", np.float64), ("count", np.int64),
+                       ("cstride", np.int64), ("f32", np.int64)])
+COMBINE_DTYPE = np.dtype([("dst", np.int64), ("shape", np.int64, (4,)), ("dst_stride", np.int64, (4,)),
+                          ("beta", np.float64), ("acc", np.int64), ("eia", np.int64), ("rank", np.int64),
+                          ("term0", np.int64), ("nterm", np.int64), ("begin", np.int64), ("dst_f32", np.int64)])
+DOT_DTYPE = np.dtype([("x", np.int64), ("y", np.int64), ("u", np.int64), ("out", np.int64), ("n", np.int64),
+                      ("no", np.int64), ("nv", np.int64)])
 assert BATCH_DTYPE.itemsize == ctypes.sizeof(Batch)
 assert S3JOB_DTYPE.itemsize == ctypes.sizeof(S3Job)
 
@@ -134,7 +142,7 @@ _SIGS = {
     "dcc_tensor_axpby_f32_f64": ([c_vp, c_vp, ctypes.POINTER(Strided), c_dbl, c_dbl, c_vp], ctypes.c_int),
     "dcc_tensor_axpby_f64_f32": ([c_vp, c_vp, ctypes.POINTER(Strided), c_dbl, c_dbl, c_vp], ctypes.c_int),
     "dcc_grouped_prepare": ([c_vp, c_i64, c_i64, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)], ctypes.c_int),
-    "dcc_grouped_prepare_auto": ([c_vp, c_i64, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)], ctypes.c_int),
+    "dcc_grouped_prepare_auto": ([c_vp, c_i64, c_i64, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64)], ctypes.c_int),
     "dcc_contract_grouped_f64": ([c_vp, c_i64, c_i64, c_i64, c_i64, c_vp], ctypes.c_int),
     "dcc_graph_capture_begin": ([c_vp], ctypes.c_int),
     "dcc_graph_capture_end": ([c_vp, ctypes.POINTER(c_vp)], ctypes.c_int),
@@ -142,6 +150,9 @@ _SIGS = {
     "dcc_graph_destroy": ([c_vp], ctypes.c_int),
     "dcc_sum_slices_f64": ([c_vp, c_vp, c_i64, c_i64, c_dbl, c_dbl, c_vp], ctypes.c_int),
     "dcc_sum_slices_f32": ([c_vp, c_vp, c_i64, c_i64, c_dbl, c_dbl, c_vp], ctypes.c_int),
+    "dcc_combine": ([c_vp, c_vp, c_i64, c_i64, c_vp], ctypes.c_int),
+    "dcc_dots_partials": ([], c_i64),
+    "dcc_dots_f64": ([c_vp, c_i64, c_vp, c_vp], ctypes.c_int),
     "dcc_diis_partials": ([], c_i64),
     "dcc_diis_push_f64": ([c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp], ctypes.c_int),
     "dcc_diis_combine_f64": ([c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp], ctypes.c_int),

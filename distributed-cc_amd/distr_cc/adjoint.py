@@ -32,7 +32,7 @@ from distr_cc import _lib as L
 from distr_cc.device import DeviceArray, init as device_init
 from distr_cc.distribute_t3 import TP_T3, canonical_case, ijk_to_linear, nocc3
 from distr_cc.rccsdt_engine import plan_einsum_steps, split_k_partial_elems
-from distr_cc.t3_engine import Operand, plan_einsum, plan_t2t3, s3_jobs_array, tensor_axpby
+from distr_cc.t3_engine import Operand, plan_einsum, plan_t2t3, s3_jobs_array, tensor_axpby, upload_tables
 
 
 def _stabiliser(i, j, k):
@@ -116,6 +116,7 @@ class T2T3Adjoint:
                             Operand(self.dt2, "lkbc", (o, o, v, v)), -6.0, 1.0, ext, one),
             ]
             self.chunks.append((DeviceArray.from_host(s3_jobs_array(jobs)), len(jobs), launches))
+        upload_tables(self.fwd + [g for c in self.chunks for g in c[2]])
 
     def _h(self):
         return self.stream.handle if self.stream is not None else None
@@ -231,7 +232,8 @@ class TriplesResidualAdjoint:
         n = o + v
         self.nocc, self.nvir, self.nmo, self.stream = o, v, n, stream
         fock = np.asarray(fock, dtype=np.float64)
-        self.eng = eng = RCCSDTEngine(o, v, fock, pppp, np.diag(fock).copy(), stream=stream, vvvv_pairs=False)
+        self.eng = eng = RCCSDTEngine(o, v, fock, pppp, np.diag(fock).copy(), stream=stream, vvvv_pairs=False,
+                                      schedule=False)
         self.tr = tr = eng.tr
         self.n3 = tr.n3
         tr.set_t3(t3_local)
@@ -265,6 +267,7 @@ class TriplesResidualAdjoint:
         self.keep = []
         self._plan_residual_adjoint()
         self._plan_program_adjoint()
+        upload_tables([step for _, steps in self.res_adj for step in steps] + [step for _, step in self.prog_adj])
 
     # ------------------------------------------------------------------ planning
     def _plan_residual_adjoint(self):
@@ -327,6 +330,8 @@ class TriplesResidualAdjoint:
     def _plan_program_adjoint(self):
         """Reverse of the intermediates program (RCCSDTEngine 'imds3'), as planned launches."""
         eng = self.eng
+        for name in ("dress", "imds3"):   # the programs that forward() runs
+            eng.prog[name].plan()
         grads = {id(eng.G): self.dG, id(eng.t2): self.dt2, id(eng.h_ovvo): self.dh}
         grads.update({id(b): self.d_imd[k] for k, b in eng.imd.items()})
         ext = eng.ext

@@ -25,8 +25,9 @@ TILE_SHAPES = {0: "64x64", 1: "128x64", 2: "64x128", 3: "128x128",
 
 
 class _GroupedPhase:
-    def __init__(self, launches):
+    def __init__(self, launches, small=False):
         self.launches = launches
+        self.small = bool(small)   # problems that are each too small to fill the chip
         self.name = launches[0].name
         self.flops = sum(g.flops for g in launches)
         self.tile = LIBRARY_TILE
@@ -50,7 +51,8 @@ class _GroupedPhase:
         total, variant = ctypes.c_int64(), ctypes.c_int64()
         ptr = ctypes.cast(arr, ctypes.c_void_p)
         if tile == LIBRARY_TILE:
-            L.call("dcc_grouped_prepare_auto", ptr, len(arr), ctypes.byref(total), ctypes.byref(variant))
+            L.call("dcc_grouped_prepare_auto", ptr, len(arr), int(self.small), ctypes.byref(total),
+                   ctypes.byref(variant))
         else:
             L.call("dcc_grouped_prepare", ptr, len(arr), int(tile), ctypes.byref(total), ctypes.byref(variant))
         self.tile, self.total, self.variant = int(tile), int(total.value), int(variant.value)
@@ -196,7 +198,7 @@ class BatchedRCCSDT(_Grouped):
         self.systems = [(int(o), int(v)) for o, v, _, _, _ in systems]
         # plain W_vvvv GEMMs: the phases are grouped launch by launch across the systems
         self.engines = [RCCSDTEngine(o, v, F, g, e, level_shift=level_shift, stream=stream, device=device,
-                                     vvvv_pairs=False) for o, v, F, g, e in systems]
+                                     vvvv_pairs=False, schedule=False) for o, v, F, g, e in systems]
         for e in self.engines:
             e.tr.set_denominators(e.mo_energy, e.level_shift, e.nvir_diis)
         self._group([e.tr for e in self.engines], stream)
@@ -208,8 +210,16 @@ class BatchedRCCSDT(_Grouped):
         launch, followed by the rest of every engine's operation (split-K sums, ...).  Operations
         without a contraction run engine by engine.  If the engines' operation lists differ in length
         (or ``group`` is False), every engine's lower-order work runs on its own."""
-        per = [e.lower_ops() for e in self.engines]
+        from distr_cc.schedule import LowerSchedule
         self.lower_phases = []
+        self.sched = self.energy_dots = None
+        if group and all(LowerSchedule.fits(e) for e in self.engines):
+            # the operations of all systems side by side, stage by stage
+            self.sched = LowerSchedule(self.engines, self.stream)
+            self.lower_phases = self.sched.grouped
+            self.energy_dots = self.sched.energies()
+            return
+        per = [e.lower_ops() for e in self.engines]
         if not group or any(len(p) != len(per[0]) for p in per):
             self.lower_plan = [(None, [[s for op in p for s in op] for p in per])]
             return
@@ -231,6 +241,12 @@ class BatchedRCCSDT(_Grouped):
     def issue_lower(self):
         """issue_lower of every engine, with the contractions of each operation grouped."""
         st = self.stream
+        if self.sched is not None:
+            for name in ("dress", "r1r2", "update12", "imds3"):
+                self.sched.run(name, st)
+            for e in self.engines:
+                e.tr.prepare_residual()
+            return
         for ph, lists in self.lower_plan:
             if ph is not None:
                 ph.run(st)
@@ -260,7 +276,10 @@ class BatchedRCCSDT(_Grouped):
         tm("finalize and energy", "start")
         for e in self.engines:
             e.tr.finalize_launch()
-            e.energy_launch()
+            if self.energy_dots is None:
+                e.energy_launch()
+        if self.energy_dots is not None:
+            self.energy_dots.run(st)
         tm("finalize and energy", "end")
 
     def energies(self):

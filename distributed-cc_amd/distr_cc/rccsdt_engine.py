@@ -24,7 +24,7 @@ import numpy as np
 
 from distr_cc import _lib as L
 from distr_cc.device import DeviceArray
-from distr_cc.t3_engine import Operand, TriplesEngine, plan_einsum, tensor_axpby
+from distr_cc.t3_engine import Operand, TriplesEngine, plan_einsum, tensor_axpby, upload_tables
 
 OCC = "ijklmn"
 VIR = "abcdefgh"
@@ -106,23 +106,26 @@ class _Program:
 
     def __init__(self, engine):
         self.eng = engine
-        self.steps = []
-        self.keep = []
-        # the operations in order, (kind, ...), for programs that are differentiated (adjoint.py)
+        # the operations in order, (kind, ...), for programs that are differentiated (adjoint.py) or
+        # scheduled together (schedule.py)
         self.ops = []
-        # the steps of every operation, one list per operation (a contraction's GemmLaunch first)
-        self.op_steps = []
+        self._plans = []      # per operation a callable giving its steps, planned when the program is run
+        self._op_steps = None
+        self.keep = []
 
     def add(self, steps):
         """An operation given as its list of steps."""
-        self.op_steps.append(list(steps))
-        self.steps += steps
+        self._plans.append(lambda: list(steps))
 
     def ein(self, name, sub, A, B, C, alpha, beta):
         self.ops.append(("ein", name, sub, A, B, C, alpha, beta))
-        steps, keep = plan_einsum_steps(name, sub, A, B, C, alpha, beta, self.eng.ext, self.eng.stream)
-        self.add(steps)
-        self.keep += keep
+
+        def plan():
+            steps, keep = plan_einsum_steps(name, sub, A, B, C, alpha, beta, self.eng.ext, self.eng.stream)
+            self.keep += keep
+            return steps
+
+        self._plans.append(plan)
 
     def axpby(self, dst, src, letters, alpha, beta):
         self.ops.append(("axpby", dst, src, letters, alpha, beta))
@@ -141,23 +144,42 @@ class _Program:
             self.ops.append(("steps", op))
             self.add(op)
 
+    def plan(self):
+        """Plan the steps now (on first use otherwise)."""
+        if self._op_steps is None:
+            self._op_steps = [plan() for plan in self._plans]
+            upload_tables([step for op in self._op_steps for step in op])
+        return self._op_steps
+
+    @property
+    def op_steps(self):
+        """The steps of every operation, one list per operation (a contraction's GemmLaunch first)."""
+        return self.plan()
+
+    @property
+    def steps(self):
+        return [step for op in self.op_steps for step in op]
+
     def run(self, stream):
-        for step in self.steps:
-            step(stream)
+        for op in self.op_steps:
+            for step in op:
+                step(stream)
 
 
 class RCCSDTEngine:
     """Device state of the RCCSDT amplitude iteration for one closed-shell system."""
 
     def __init__(self, nocc, nvir, fock, pppp, mo_energy, level_shift=0.0, nvir_diis=None, stream=None,
-                 device=0, t3_dtype=np.float64, triples_contract="native", vvvv_pairs="auto"):
+                 device=0, t3_dtype=np.float64, triples_contract="native", vvvv_pairs="auto", schedule=True):
         """``t3_dtype`` float32 selects the mixed-precision iteration: T3, the triples residual and its
         operands in FP32 with FP32-MFMA contractions, everything else (integrals, T1/T2, lower-order
         residual, denominators, projection arithmetic, norms, energy, DIIS) in FP64;
         ``triples_contract="bf16x3"`` (with float32) runs those contractions as split-BF16x3.
         ``vvvv_pairs`` is the triples engine's option: the W_vvvv built here (the T1-dressed <ab|de>
         plus <lm|de> t2[l,m,a,b]) is pair-symmetric, so "auto" uses the half-flop pair products
-        whenever the device has room for them."""
+        whenever the device has room for them.  ``schedule``: run the lower-order part in few launches
+        (schedule.LowerSchedule) where the system is small enough; off for an engine whose lower-order part
+        its owner issues (ensembles, the adjoint)."""
         o, v = int(nocc), int(nvir)
         n = o + v
         fock = np.asarray(fock, dtype=np.float64)
@@ -211,13 +233,27 @@ class RCCSDTEngine:
         self.fov0 = DeviceArray((o, v), f64)
         self.tau = DeviceArray((o, o, v, v), f64)
         self.partials = DeviceArray((int(L._lib.dcc_dot_partials()),), f64)
-        self.scal = DeviceArray((8,), f64)
+        self.scal = DeviceArray((8,), f64)   # |r1|^2, |r2|^2, energy pieces, |r3|^2 and its active part
+        tr.norms = DeviceArray((2,), f64, ptr=self.scal.ptr + 32, owner=False)
+        tr.norms.base = self.scal            # keeps the memory
         self.t2.fill(0.0, stream)
         tr.t3.fill(0.0, stream)
         self._setup_constants()
         tr._setup_lower()
         self.prog = self._build_program()
-        self._eprog = self._build_energy_program()   # planned here: its launch tables are uploaded once
+        self._eprog = None
+        self.sched = None
+        if schedule:
+            from distr_cc.schedule import LowerSchedule
+            if LowerSchedule.fits(self):
+                self.sched = LowerSchedule([self], stream)
+                self._eprog = self.sched.energies()
+            else:
+                for p in self.prog.values():
+                    p.plan()
+        if self._eprog is None:
+            self._eprog = self._build_energy_program()
+            self._eprog.plan()
 
     # ------------------------------------------------------------------ views
     def gview(self, buf, letters):
@@ -428,11 +464,11 @@ class RCCSDTEngine:
         record HIP events."""
         st = self.stream
         tick = timer if timer is not None else (lambda name, what: None)
-        phases = [("dress", lambda: self.prog["dress"].run(st)),
-                  ("lower r1/r2", lambda: self.prog["r1r2"].run(st)),
-                  ("T3->r1/r2 + update t1/t2", lambda: self.prog["update12"].run(st)),
-                  ("triples intermediates", lambda: self.prog["imds3"].run(st)),
-                  ("T3->W", lambda: self.tr.t3_to_w(reuse_z=True)),
+        phases = [("dress", lambda: self._lower_phase("dress")),
+                  ("lower r1/r2", lambda: self._lower_phase("r1r2")),
+                  ("T3->r1/r2 + update t1/t2", lambda: self._lower_phase("update12")),
+                  ("triples intermediates", lambda: self._lower_phase("imds3")),
+                  ("T3->W", self._add_t3_to_w),
                   ("ring/oooo operands", self.tr.prepare_residual),
                   ("triples residual", lambda: self.tr.residual(timer=launch_timer))]
         for name, fn in phases:
@@ -440,11 +476,20 @@ class RCCSDTEngine:
             fn()
             tick(name, "end")
         tick("finalize", "start")
-        n3, act = self.tr.finalize(self.mo_energy, self.level_shift, self.nvir_diis)
+        self.tr.set_denominators(self.mo_energy, self.level_shift, self.nvir_diis)
+        self.tr.finalize_launch()
         tick("finalize", "end")
-        self.last_t3_norm_sq, self.last_t3_active_norm_sq = n3, act
         sc = self.scal.download(stream=st)
+        n3 = float(sc[4])
+        self.last_t3_norm_sq, self.last_t3_active_norm_sq = n3, float(sc[5])
         return [float(np.sqrt(max(sc[0], 0.0))), float(np.sqrt(max(sc[1], 0.0))), float(np.sqrt(max(n3, 0.0)))]
+
+    def _lower_phase(self, name):
+        (self.sched or self.prog[name]).run(*((name, self.stream) if self.sched else (self.stream,)))
+
+    def _add_t3_to_w(self):
+        if self.sched is None:   # the schedule's intermediates already hold the T3 terms
+            self.tr.t3_to_w(reuse_z=True)
 
     def energy(self):
         """E_corr = sum (2<ij|ab> - <ij|ba>)(t2 + t1 t1) + 2 sum f_ia t1_ia (rccsdt.py:218-221 closed form)."""
@@ -470,10 +515,9 @@ class RCCSDTEngine:
         """Device work of update_amps before the triples residual, with no host synchronisation (so it
         can be captured in a HIP graph): T1 dressing, lower-order residual, T3 -> r1/r2 and the t1/t2
         update, the T2-dressed triples intermediates, T3 -> W, the residual's operands."""
-        st = self.stream
         for name in ("dress", "r1r2", "update12", "imds3"):
-            self.prog[name].run(st)
-        self.tr.t3_to_w(reuse_z=True)
+            self._lower_phase(name)
+        self._add_t3_to_w()
         self.tr.prepare_residual()
 
     def _build_energy_program(self):

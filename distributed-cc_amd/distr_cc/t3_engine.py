@@ -128,7 +128,8 @@ class GemmLaunch:
         bt = np.zeros(rows.shape[0], dtype=L.BATCH_DTYPE)
         for n, field in enumerate(L.BATCH_DTYPE.names):
             bt[field] = rows[:, n]
-        self.batches = DeviceArray.from_host(bt)
+        self.table = bt
+        self._batches = None     # its device copy (upload_tables, or on first use)
         self.nbatch = len(batches)
         self.max_rows = int(max_rows)
         self.flops = float(flops)
@@ -137,6 +138,12 @@ class GemmLaunch:
 
     def __call__(self, stream):
         self.run(stream)
+
+    @property
+    def batches(self):
+        if self._batches is None:
+            self._batches = DeviceArray.from_host(self.table)
+        return self._batches
 
     def run(self, stream):
         s = stream.handle if stream is not None else None
@@ -147,6 +154,20 @@ class GemmLaunch:
                    self.max_rows, self.tile, s)
         else:
             L.call(self.fn, *self.args, self.batches.vp, self.nbatch, self.max_rows, s)
+
+
+def upload_tables(launches):
+    """The batch tables of many GemmLaunches in one device buffer (an allocation and a copy each otherwise)."""
+    todo = [g for g in launches if isinstance(g, GemmLaunch) and g._batches is None and g.table.size]
+    if not todo:
+        return
+    all_rows = DeviceArray.from_host(np.concatenate([g.table for g in todo]))
+    at = 0
+    for g in todo:
+        g._batches = DeviceArray(g.table.shape, L.BATCH_DTYPE, ptr=all_rows.ptr + at * L.BATCH_DTYPE.itemsize,
+                                 owner=False)
+        g._batches.base, g._batches._host = all_rows, g.table     # keeps the memory; the host copy
+        at += g.table.size
 
 
 def _fuse(letters, ops, ext):
@@ -486,6 +507,7 @@ class TriplesEngine:
         qc = int(max(1, min(n3, qc)))
         self.Xp = DeviceArray((5, qc, v, v, v), dt)
         self.eia = DeviceArray((o, v))
+        self._eia_host = None    # what it holds
         self.norb = int(L._lib.dcc_r3_finalize_tiles(v))
         self.partials = DeviceArray((n3 * self.norb, 2))
         self.norms = DeviceArray((2,))
@@ -531,6 +553,7 @@ class TriplesEngine:
         self._tables = []
         self.ring_g_bytes = int(ring_g_bytes)
         self.launches = self._plan_residual()
+        upload_tables(self.launches)
         self._retarget(self.launches)
         self._yz_direct = False   # Y/Z written as packed words (set by _setup_packing)
         self._packs = self._setup_packing() if contract == "bf16x3" else []
@@ -861,6 +884,7 @@ class TriplesEngine:
             self._retarget([g for g in a2 + a3 if isinstance(g, GemmLaunch)])
             chunks.append((DeviceArray.from_host(s3_jobs_array(jobs)), len(jobs), a2, a3))
         lo['chunks'] = chunks
+        upload_tables([g for ch in chunks for g in ch[2] + ch[3]])
         lo['dw_valid'] = False
         self._lower = lo
 
@@ -1073,8 +1097,10 @@ class TriplesEngine:
         """Upload eia = e_i - e_a - shift (rccsdt.py:737) and fix the active virtual count."""
         o, v = self.nocc, self.nvir
         e = np.asarray(mo_energy, dtype=np.float64)
-        eia = e[:o, None] - e[None, o:] - level_shift
-        self.eia.upload(np.ascontiguousarray(eia), self.stream)
+        eia = np.ascontiguousarray(e[:o, None] - e[None, o:] - level_shift)
+        if not np.array_equal(eia, self._eia_host):   # an upload waits for the stream
+            self.eia.upload(eia, self.stream)
+            self._eia_host = eia
         self.nvir_diis = v if nvir_diis is None else int(nvir_diis)
 
     def finalize_launch(self, r3_out=None):

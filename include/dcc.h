@@ -441,6 +441,47 @@ int dcc_dot_f64(const double *x, const double *y, int64_t n, double *partials, d
 int dcc_dot_f32(const float *x, const float *y, int64_t n, double *partials, double *out, dcc_stream_t stream);
 
 /*
+ * Linear combinations of many tensors in one launch.  Job j (device arrays of jobs and terms):
+ *   dst[x] = (beta dst[x] + sum over its terms, in order, of coef sum_{s < count} src[s cstride + x . stride]) / D
+ * over x in shape (four indices, fewer than 2^31 elements; extent 1 where unused), D = 1 (rank 0), eia[i,a] for
+ * shape (1,1,i,a) (rank 1) or eia[i,a] + eia[j,b] for shape (i,j,a,b) (rank 2); acc, if not null, gets the value
+ * added at the linear index.  f32 flags: the array holds float.  begin: the job's first workgroup, each of 1024
+ * elements, jobs in ascending order; nworkgroups their total.  Jobs of a launch write disjoint data that no
+ * other job of it reads (dst of a job may be among its own sources only through beta).
+ */
+typedef struct dcc_combine_term {
+    const void *src;
+    int64_t stride[4];
+    double coef;
+    int64_t count, cstride, f32;
+} dcc_combine_term;
+
+typedef struct dcc_combine_job {
+    void *dst;
+    int64_t shape[4], dst_stride[4];
+    double beta;
+    double *acc;
+    const double *eia;
+    int64_t rank, term0, nterm, begin, dst_f32;
+} dcc_combine_job;
+
+int dcc_combine(const dcc_combine_job *jobs, const dcc_combine_term *terms, int64_t njobs, int64_t nworkgroups,
+                dcc_stream_t stream);
+
+/*
+ * Dot products of many vector pairs: *out = sum_t x[t] y[t], or with u (no, nv) and n = (no nv)^2 < 2^32 indices
+ * (i,j,a,b): sum x (y + u[i,a] u[j,b]).  jobs in device memory, partials njobs * dcc_dots_partials() doubles.
+ */
+typedef struct dcc_dot_job {
+    const double *x, *y, *u;
+    double *out;
+    int64_t n, no, nv;
+} dcc_dot_job;
+
+int64_t dcc_dots_partials(void);
+int dcc_dots_f64(const dcc_dot_job *jobs, int64_t njobs, double *partials, dcc_stream_t stream);
+
+/*
  * One DIIS step (distr_cc/diis.py:105-145) in two passes over the history.  Push: xs <- x, errors[head] <-
  * x - xprev and out[i] = errors[head] . errors[i] for the nvec error vectors.  Combine: xnew <- sum_i coef[i]
  * vectors[i], out[0] = |xnew - xprev|^2, xprev <- xnew.  The pointer and coefficient lists are host arrays
@@ -487,9 +528,11 @@ typedef void *dcc_graph_t;
 int dcc_grouped_prepare(dcc_gemm_problem *probs, int64_t nprob, int64_t tile_shape, int64_t *total_tiles,
                         int64_t *variant);
 
-/* The same with the tile the library chooses for the sizes of the whole group: 64x64, or the tiles of
- * dcc_contract_f64 for few or narrow outputs. */
-int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t *total_tiles, int64_t *variant);
+/* The same with the tile the library chooses for the sizes of the whole group: one of the shapes, or the
+ * tiles of dcc_contract_f64 for few or narrow outputs; with `small` always one of the latter (a group of
+ * many problems that are each too small to fill the chip). */
+int dcc_grouped_prepare_auto(dcc_gemm_problem *probs, int64_t nprob, int64_t small, int64_t *total_tiles,
+                             int64_t *variant);
 
 /* Persistent grouped FP64 gather-GEMM over a device array of prepared problems whose C regions are
  * disjoint; variant from dcc_grouped_prepare or dcc_grouped_prepare_auto; nworkgroups = 0 launches as many

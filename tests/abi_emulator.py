@@ -126,7 +126,7 @@ class Emulator:
         pvariant._obj.value = int(tile)
         return 0
 
-    def dcc_grouped_prepare_auto(self, probs, nprob, ptotal, pvariant):
+    def dcc_grouped_prepare_auto(self, probs, nprob, small, ptotal, pvariant):
         return self.dcc_grouped_prepare(probs, nprob, 0, ptotal, pvariant)
 
     def dcc_contract_grouped_f64(self, probs, nprob, total, variant, nwg, stream):
@@ -430,6 +430,55 @@ class Emulator:
         X = self.dev.view(_ptr(x), dt, n).astype(np.float64)
         Y = self.dev.view(_ptr(y), dt, n).astype(np.float64)
         o[0] = float(X @ Y)
+        return 0
+
+    def dcc_combine(self, jobs, terms, njobs, nwg, stream):
+        from distr_cc import _lib as L
+        jb = self.dev.view(_ptr(jobs), np.uint8, int(njobs) * L.COMBINE_DTYPE.itemsize).view(L.COMBINE_DTYPE)
+        nt = int((jb["term0"] + jb["nterm"]).max())
+        tm = self.dev.view(_ptr(terms), np.uint8, max(nt, 1) * L.TERM_DTYPE.itemsize).view(L.TERM_DTYPE)
+        at = lambda strides, shape: sum(np.arange(n).reshape([-1 if d == k else 1 for k in range(4)]) * int(s)
+                                        for d, (n, s) in enumerate(zip(shape, strides)))
+        done = 0
+        for j in jb:
+            shape = tuple(int(x) for x in j["shape"])
+            total = int(np.prod(shape))
+            assert j["begin"] == done
+            done += -(-total // 1024)
+            dst = self.dev.view(int(j["dst"]), np.float32 if j["dst_f32"] else np.float64)
+            od = at(j["dst_stride"], shape) + np.zeros(shape, dtype=np.int64)
+            v = np.zeros(shape)
+            if j["beta"] != 0.0:
+                v += j["beta"] * dst[od]
+            for t in tm[int(j["term0"]):int(j["term0"] + j["nterm"])]:
+                src = self.dev.view(int(t["src"]), np.float32 if t["f32"] else np.float64)
+                o = at(t["stride"], shape) + np.zeros(shape, dtype=np.int64)
+                for s in range(int(t["count"])):
+                    v += t["coef"] * src[o + s * int(t["cstride"])]
+            if j["rank"]:
+                n2, n3 = shape[2:]
+                no = n2 if j["rank"] == 1 else shape[0]
+                nv = n3
+                e = self.dev.view(int(j["eia"]), np.float64, no * nv).reshape(no, nv)
+                v /= e[None, None] if j["rank"] == 1 else e[:, None, :, None] + e[None, :, None, :]
+            dst[od] = v
+            if j["acc"]:
+                self.dev.view(int(j["acc"]), np.float64, total)[:] += v.ravel()
+        assert done == int(nwg)
+        return 0
+
+    def dcc_dots_partials(self):
+        return 2
+
+    def dcc_dots_f64(self, jobs, njobs, partials, stream):
+        from distr_cc import _lib as L
+        for j in self.dev.view(_ptr(jobs), np.uint8, int(njobs) * L.DOT_DTYPE.itemsize).view(L.DOT_DTYPE):
+            n, o, v = int(j["n"]), int(j["no"]), int(j["nv"])
+            x, y = (self.dev.view(int(j[k]), np.float64, n) if n else np.zeros(0) for k in ("x", "y"))
+            if j["u"]:
+                u = self.dev.view(int(j["u"]), np.float64, o * v).reshape(o, v)
+                y = y + np.einsum("ia,jb->ijab", u, u).ravel()
+            self.dev.view(int(j["out"]), np.float64, 1)[0] = float(x @ y)
         return 0
 
     def dcc_diis_partials(self):

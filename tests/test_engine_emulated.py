@@ -481,3 +481,26 @@ def test_batched_rccsdt_plan(monkeypatch):
         assert abs(got[n] - ref.energy()) <= 1e-14
         for x, y in zip(bt.engines[n].get_amplitudes(), ref.get_amplitudes()):
             assert abs(x - y).max() <= 1e-13 * max(abs(y).max(), 1e-30)
+
+
+@pytest.mark.parametrize("o,v,shift", [(1, 2, 0.0), (2, 5, 0.1), (5, 3, 0.0), (3, 4, 0.0)])
+def test_lower_schedule_matches_programs(monkeypatch, o, v, shift):
+    """The few-launch schedule of the lower-order part == the one-by-one programs, with a non-canonical Fock
+    matrix (t1 != 0) and a level shift, over two iterations; the denominators follow configure()."""
+    abi_emulator.install(monkeypatch)
+    from ccsdt_cases import molecule_like, random_amplitudes, with_fov
+    from distr_cc.rccsdt_engine import RCCSDTEngine
+    F, g, e, _ = molecule_like(o, v, 70 + o)
+    F = with_fov(F, o, 0.05, 5)
+    engs = [RCCSDTEngine(o, v, F, g, e, level_shift=shift, schedule=s) for s in (True, False)]
+    assert engs[0].sched is not None and engs[1].sched is None
+    for eng in engs:
+        eng.set_amplitudes(*random_amplitudes(o, v, 6))
+    for shift2 in (shift, 0.2):
+        res = []
+        for eng in engs:
+            eng.configure(level_shift=shift2)
+            res.append(eng.update_amps() + [eng.energy()])
+        assert np.allclose(res[0], res[1], rtol=1e-12, atol=1e-15)
+        for x, y in zip(engs[0].get_amplitudes(), engs[1].get_amplitudes()):
+            assert abs(x - y).max() <= 1e-13 * max(abs(y).max(), 1e-30)

@@ -828,3 +828,50 @@ def test_contract_skinny_sizes(dev, dt, M, N, K):
             ref[lo:hi] += -0.5 * (a[lo:hi] @ b)
             bound = np.finfo(dt).eps * (K * (np.abs(a) @ np.abs(b)) + np.abs(ref) + np.abs(c))
             assert (np.abs(g - ref) <= bound).all(), (a_k, b_n, c_n)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 2, 3, 3), (1, 1, 11, 93), (4, 4, 8, 8), (5, 5, 7, 7)])
+def test_combine_and_dots(dev, shape):
+    """Several combination jobs in one launch (sizes around a workgroup's 1024 elements): strided and
+    broadcast sources, slices, FP32 sources and targets, beta, a second output, both denominators; and dot
+    products with and without the outer product.  FP64 sums of a handful of terms: 1e-13 of the scale."""
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    from distr_cc.schedule import Combine, Dots, term
+    from distr_cc.t3_engine import Operand
+    rng = np.random.default_rng(sum(shape))
+    o, v = shape[0], shape[3]
+    a, b = rng.standard_normal(shape), rng.standard_normal((3,) + shape)
+    e = rng.uniform(1.0, 2.0, (o, v))
+    rank2 = shape[0] == shape[1] and shape[2] == shape[3]
+    f = rng.standard_normal(shape).astype(np.float32)
+    dA, dB, dE, dF = (DeviceArray.from_host(x) for x in (a, b, e, f))
+    d0 = rng.standard_normal(shape)
+    acc0 = rng.standard_normal(shape)
+    out, acc, out32, vec = DeviceArray.from_host(d0), DeviceArray.from_host(acc0), DeviceArray(shape, np.float32), \
+        DeviceArray((o, v))
+    op = lambda buf, l: Operand(buf, l, shape)
+    sl = term(Operand(dB, "ijab", shape), "ijab", 0.5, 3, int(np.prod(shape)))
+    tr = [term(op(dA, "jiba"), "ijab", -1.0)] if rank2 else []
+    row = Operand.strided(dE, {"i": v, "a": 1})
+    jobs = [(op(out, "ijab"), "ijab", list(shape), [term(op(dA, "ijab"), "ijab", 2.0), sl] + tr,
+             dict(beta=-0.25, acc=acc, **(dict(eia=dE, rank=2) if rank2 else {}))),
+            (op(out32, "ijab"), "ijab", list(shape), [term(op(dF, "ijab"), "ijab"), term(Operand.strided(
+                dE, {"i": v, "j": 0, "a": 0, "b": 1}), "ijab", 3.0)], {}),
+            (Operand(vec, "ia", (o, v)), "ia", [o, v], [term(row, "ia", 2.0)], dict(eia=dE, rank=1))]
+    Combine(jobs).run(None)
+    ref = 2.0 * a + 0.5 * b.sum(0) - 0.25 * d0 - (a.transpose(1, 0, 3, 2) if rank2 else 0.0)
+    if rank2:
+        ref = ref / (e[:, None, :, None] + e[None, :, None, :])
+    assert np.abs(out.download() - ref).max() <= 1e-13 * max(1.0, np.abs(ref).max())
+    assert np.abs(acc.download() - (acc0 + ref)).max() <= 1e-13 * max(1.0, np.abs(ref).max())
+    assert np.allclose(out32.download(), f + 3.0 * e[:, None, None, :], rtol=1e-6)
+    assert np.array_equal(vec.download(), 2.0 * e / e)
+    res = DeviceArray((2,))
+    n = int(np.prod(shape))
+    Dots([(dA, out, None, res.ptr, n, 0, 0)] + ([(dA, out, dE, res.ptr + 8, n, o, v)] if rank2 else [])).run(None)
+    got = res.download()
+    assert abs(got[0] - (a * ref).sum()) <= 1e-13 * np.abs(a * ref).sum()
+    if rank2:
+        y = ref + np.einsum("ia,jb->ijab", e, e)
+        assert abs(got[1] - (a * y).sum()) <= 1e-13 * np.abs(a * y).sum()
