@@ -270,12 +270,17 @@ __global__ __launch_bounds__(kQThreads) void q_finalize_ws_kernel(
 // are contiguous, 128-byte pieces); every element of the o^4 block is added by one lane per barrier
 // interval, so the sums have a fixed order.  z4 and t4 never reach HBM: written and read back by 48
 // batched GEMMs and a finalize pass they were 811 GB at nocc=8, nvir=40 and bound the evaluation: a whole
-// (Q) call at nocc=8, nvir=38 takes 58 ms this way against 313 ms, at nocc=5, nvir=19 1.4 ms against 5.8 ms.
+// (Q) call at nocc=8, nvir=38 takes 53 ms this way against 312 ms, at nocc=5, nvir=19 1.2 ms against 5.9 ms.
+// The kernel is 41.5 ms of that at nocc=8, 0.64 ms at nocc=5.  Two workgroups fit a CU at nocc=8, so latency
+// bounds it: loads several MFMA steps ahead and the deal over the XCDs took it there from 46.1 and 0.80 ms.
+// (One loop over all terms that also keeps the next term's first loads in flight over the barriers was
+// slower, 50.4 and 0.88 ms: its operands and LDS strides are then no constants of the code.)
 // The block is stored with odd strides so that lanes running over any occupied index hit distinct banks.
 struct QQuadArgs {
     const double *T, *vvvo, *vooo, *t2, *Wv, *Wo, *vvoo, *e_occ, *e_vir;
     const int *tasks, *slots;   // slots: per task the 12 Wv slots of its ordered block triples, or null
     int bs, nv, vp;
+    int64_t total;   // quadruples: tasks * bs^4
     double *partials;
 };
 
@@ -288,6 +293,12 @@ template <int O> struct QBlk {
     static constexpr int CF3 = (2 * O + 15) / 16;           // column fragments of a pair term
     static constexpr int RB = CF3 == 1 ? (RF3 + 3) / 4 : 4;  // row fragments per wave and pass (registers)
     static constexpr int RF2 = (O2 + 15) / 16, NF2 = RF2 * RF2, TF2 = (NF2 + 3) / 4;
+    // MFMA steps per stage of loads: a stage is in flight while the previous one is multiplied, and an L2 load
+    // takes as long as some 20 MFMAs of a wave, so the fewer products a step has the more steps go together
+    static constexpr int KU3 = RB > 4 || CF3 > 1 ? 2 : RB > 2 ? 3 : 2, KU2 = TF2 > 4 ? 1 : TF2 == 3 ? 4 : TF2 > 1 ? 5 : 2;
+    // with four row fragments a wave's fragments w, w + 4, .. share their rows
+    static constexpr int NA2 = RF2 == 4 ? 1 : TF2;
+    static constexpr int WAVES = O == 9 ? 1 : O >= 6 ? 2 : 5;   // resident per SIMD (LDS: two at O = 8, one at 9)
     __device__ static int pos(int slot) { return slot == 0 ? S3 : slot == 1 ? S2 : slot == 2 ? S1 : 1; }
     // LDS position of the linear element x of the o^4 block
     __device__ static int at(int x) { return x / O3 * S3 + x / O2 % O * S2 + x / O % O * S1 + x % O; }
@@ -319,30 +330,39 @@ __device__ __forceinline__ void q_pair_term(const double *__restrict__ A, const 
 #pragma unroll
             for (int c = 0; c < G::CF3; ++c) acc[r][c] = qd4{0, 0, 0, 0};
         // k of this lane in steps of 4; beyond K the last k is read and multiplied by zero
-        double a[2][G::RB], b[2][G::CF3];
+        double a[2][G::KU3][G::RB], b[2][G::KU3][G::CF3];
         auto load = [&](int s, int k0) {
-            const int k = k0 + lk, kk = min(k, K - 1);
 #pragma unroll
-            for (int r = 0; r < G::RB; ++r) a[s][r] = ap[r][(int64_t)kk * G::O3];
+            for (int q = 0; q < G::KU3; ++q) {
+                if (k0 + 4 * q >= K) break;   // uniform
+                const int k = k0 + 4 * q + lk, kk = min(k, K - 1);
 #pragma unroll
-            for (int c = 0; c < G::CF3; ++c) {
-                const double x = bp[c][kk * O];
-                b[s][c] = k < K && bok[c] ? x : 0.0;
+                for (int r = 0; r < G::RB; ++r) a[s][q][r] = ap[r][(int64_t)kk * G::O3];
+#pragma unroll
+                for (int c = 0; c < G::CF3; ++c) {
+                    const double x = bp[c][kk * O];
+                    b[s][q][c] = k < K && bok[c] ? x : 0.0;
+                }
             }
         };
-        auto mul = [&](int s) {
+        auto mul = [&](int s, int k0) {
 #pragma unroll
-            for (int r = 0; r < G::RB; ++r)
+            for (int q = 0; q < G::KU3; ++q) {
+                if (k0 + 4 * q >= K) break;
 #pragma unroll
-                for (int c = 0; c < G::CF3; ++c)
-                    acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][r], b[s][c], acc[r][c], 0, 0, 0);
+                for (int r = 0; r < G::RB; ++r)
+#pragma unroll
+                    for (int c = 0; c < G::CF3; ++c)
+                        acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][q][r], b[s][q][c], acc[r][c], 0, 0, 0);
+            }
         };
+        constexpr int KS = 4 * G::KU3;
         load(0, 0);
-        for (int k0 = 0; k0 < K; k0 += 8) {
-            load(1, k0 + 4);
-            mul(0);
-            load(0, k0 + 8);
-            mul(1);
+        for (int k0 = 0; k0 < K; k0 += 2 * KS) {
+            load(1, k0 + KS);
+            mul(0, k0);
+            load(0, k0 + 2 * KS);
+            mul(1, k0 + KS);
         }
         // the two terms of a column group touch the same elements: one barrier interval each
 #pragma unroll
@@ -374,36 +394,46 @@ __device__ __forceinline__ void q_square_acc(const double *__restrict__ A, int64
                                              int64_t kb, int K, qd4 *acc) {
     typedef QBlk<O> G;
     const int lane = threadIdx.x % 64, w = threadIdx.x / 64, lr = lane % 16, lk = lane / 16;
-    int ar[G::TF2], bc[G::TF2];
+    int ar[G::NA2], bc[G::TF2];
 #pragma unroll
     for (int t = 0; t < G::TF2; ++t) {
         const int f = min(w + 4 * t, G::NF2 - 1);
         const int row = min(f % G::RF2 * 16 + lr, G::O2 - 1), col = min(f / G::RF2 * 16 + lr, G::O2 - 1);
-        ar[t] = TR ? row % O * O + row / O : row;
+        if (t < G::NA2) ar[t] = TR ? row % O * O + row / O : row;
         bc[t] = TC ? col % O * O + col / O : col;
     }
-    double a[2][G::TF2], b[2][G::TF2];
+    double a[2][G::KU2][G::NA2], b[2][G::KU2][G::TF2];
     auto load = [&](int s, int k0) {
-        const int k = k0 + lk, kk = min(k, K - 1);
-        const double *ak = A + kk * ka, *bk = B + kk * kb;
 #pragma unroll
-        for (int t = 0; t < G::TF2; ++t) {
-            a[s][t] = ak[ar[t]];
-            const double x = bk[bc[t]];
-            b[s][t] = k < K ? x : 0.0;
+        for (int q = 0; q < G::KU2; ++q) {
+            if (k0 + 4 * q >= K) break;   // uniform
+            const int k = k0 + 4 * q + lk, kk = min(k, K - 1);
+            const double *ak = A + kk * ka, *bk = B + kk * kb;
+#pragma unroll
+            for (int t = 0; t < G::TF2; ++t) {
+                if (t < G::NA2) a[s][q][t] = ak[ar[t]];
+                const double x = bk[bc[t]];
+                b[s][q][t] = k < K ? x : 0.0;
+            }
         }
     };
-    auto mul = [&](int s) {
+    auto mul = [&](int s, int k0) {
 #pragma unroll
-        for (int t = 0; t < G::TF2; ++t)
-            acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][t], b[s][t], acc[t], 0, 0, 0);
+        for (int q = 0; q < G::KU2; ++q) {
+            if (k0 + 4 * q >= K) break;
+#pragma unroll
+            for (int t = 0; t < G::TF2; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][q][G::NA2 == 1 ? 0 : t], b[s][q][t], acc[t],
+                                                                0, 0, 0);
+        }
     };
+    constexpr int KS = 4 * G::KU2;
     load(0, 0);
-    for (int k0 = 0; k0 < K; k0 += 8) {
-        load(1, k0 + 4);
-        mul(0);
-        load(0, k0 + 8);
-        mul(1);
+    for (int k0 = 0; k0 < K; k0 += 2 * KS) {
+        load(1, k0 + KS);
+        mul(0, k0);
+        load(0, k0 + 2 * KS);
+        mul(1, k0 + KS);
     }
 }
 
@@ -426,18 +456,20 @@ __device__ __forceinline__ void q_square_add(const qd4 *acc, double sign, double
 }
 
 template <int O>
-__global__ __launch_bounds__(kQThreads) void q_quad_kernel(const QQuadArgs p, int64_t total) {
+__global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(QBlk<O>::WAVES)))
+void q_quad_kernel(const QQuadArgs p) {
     typedef QBlk<O> G;
     extern __shared__ double lds[];
     double *Z = lds, *S = lds + G::SZ;
-    // consecutive quadruples on one XCD: they share T[a,b], T[a,c], T[b,c] slices in its L2
-    const int64_t wg = [&] {
-        const int64_t L = blockIdx.x, q = total / 8, r = total % 8, x = L % 8, y = L / 8;
-        return x < r ? x * (q + 1) + y : r * (q + 1) + (x - r) * q + y;
-    }();
-    const int bs = p.bs, bs3 = bs * bs * bs;
-    const int64_t task = wg / ((int64_t)bs3 * bs);
-    const int e0 = (int)(wg % ((int64_t)bs3 * bs));
+    // 256 consecutive quadruples run on one XCD (they share T[a,b], T[a,c], T[b,c] slices in its L2), and such
+    // units are dealt round robin: the early tasks have many (a,b,c,d) without weight, and an eighth of the
+    // list each left XCDs idle a third of the time.
+    const int bs = p.bs, bs3 = bs * bs * bs, bs4 = bs3 * bs;
+    const uint32_t unit = blockIdx.x / 8 / 256 * 8 + blockIdx.x % 8;
+    const int64_t wg = (int64_t)unit * 256 + blockIdx.x / 8 % 256;
+    if (wg >= p.total) return;
+    const int64_t task = wg / (uint32_t)bs4;
+    const int e0 = (int)(wg - task * bs4);
     const int in[4] = {e0 / bs3, e0 / (bs * bs) % bs, e0 / bs % bs, e0 % bs};   // index within each block
     int v[4];                                                                   // a, b, c, d
 #pragma unroll
@@ -558,10 +590,10 @@ __global__ __launch_bounds__(kQThreads) void q_quad_kernel(const QQuadArgs p, in
     q_store_partials(paren, bracket, p.partials, wg);
 }
 
-template <int O> int q_quads_launch(const QQuadArgs &a, int64_t total, hipStream_t s) {
+template <int O> int q_quads_launch(const QQuadArgs &a, int64_t grid, hipStream_t s) {
     // the two blocks; at the end 12 o^2 matrix elements take their place (more than the blocks at small o)
     constexpr size_t bytes = sizeof(double) * (2 * QBlk<O>::SZ > 12 * O * O ? 2 * QBlk<O>::SZ : 12 * O * O);
-    hipLaunchKernelGGL(q_quad_kernel<O>, dim3((unsigned)total), dim3(kQThreads), bytes, s, a, total);
+    hipLaunchKernelGGL(q_quad_kernel<O>, dim3((unsigned)grid), dim3(kQThreads), bytes, s, a);
     DCC_LAUNCH_CHECK();
     return 0;
 }
@@ -641,20 +673,21 @@ int dcc_q_quads_f64(const double *T, const double *vvvo, const double *vooo, con
     const int64_t nwg = ntask * blksize * blksize * blksize * blksize;
     if (nwg == 0) return 0;
     DCC_CHECK(T && vvvo && vooo && vvoo && t2 && Wv && Wo && tasks && e_occ && e_vir && partials, "null pointer");
-    DCC_CHECK(nwg < ((int64_t)1 << 31), "grid too large");
-    const QQuadArgs a{T,     vvvo,  vooo,  t2,    Wv,           Wo,        vvoo,      e_occ,
-                      e_vir, tasks, slots, (int)blksize, (int)nvir, (int)vpad, partials};
+    const QQuadArgs a{T,     vvvo,  vooo,  t2,           Wv,        Wo,        vvoo,  e_occ,
+                      e_vir, tasks, slots, (int)blksize, (int)nvir, (int)vpad, nwg, partials};
     hipStream_t s = dcc::as_stream(stream);
+    const int64_t grid = (nwg + 2047) / 2048 * 2048;   // units of 256 on each of the eight XCDs
+    DCC_CHECK(grid * kQThreads < ((int64_t)1 << 32), "grid too large");
     switch (nocc) {
-        case 1: return q_quads_launch<1>(a, nwg, s);
-        case 2: return q_quads_launch<2>(a, nwg, s);
-        case 3: return q_quads_launch<3>(a, nwg, s);
-        case 4: return q_quads_launch<4>(a, nwg, s);
-        case 5: return q_quads_launch<5>(a, nwg, s);
-        case 6: return q_quads_launch<6>(a, nwg, s);
-        case 7: return q_quads_launch<7>(a, nwg, s);
-        case 8: return q_quads_launch<8>(a, nwg, s);
-        default: return q_quads_launch<9>(a, nwg, s);
+        case 1: return q_quads_launch<1>(a, grid, s);
+        case 2: return q_quads_launch<2>(a, grid, s);
+        case 3: return q_quads_launch<3>(a, grid, s);
+        case 4: return q_quads_launch<4>(a, grid, s);
+        case 5: return q_quads_launch<5>(a, grid, s);
+        case 6: return q_quads_launch<6>(a, grid, s);
+        case 7: return q_quads_launch<7>(a, grid, s);
+        case 8: return q_quads_launch<8>(a, grid, s);
+        default: return q_quads_launch<9>(a, grid, s);
     }
 }
 

@@ -102,8 +102,8 @@ class QEngine:
         o, vp, bs = self.o, self.vp, self.bs
         per_task = bs ** 4 * o ** 4 * 8
         self.chunk = max(1, min(int(max_chunk_bytes // per_task), 4096))
-        # the partials of a chunk are two doubles per quadruple
-        self.quad_chunk = max(1, int(max_chunk_bytes // (bs ** 4 * 16)))
+        # a chunk of fused quadruples: one workgroup each, partials of two doubles
+        self.quad_chunk = max(1, min(int(max_chunk_bytes // (bs ** 4 * 16)), (1 << 23) // bs ** 4))
         if w_mode is None:
             w_mode = "dense" if vp ** 4 * o * o * 8 <= dense_w_bytes else "task"
         if w_mode not in ("dense", "task"):
