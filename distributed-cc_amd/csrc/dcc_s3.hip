@@ -279,6 +279,208 @@ __global__ __launch_bounds__(kThreads) void s3_gather_kernel(T *__restrict__ out
     else s3_gather_tile<T, false>(lds, out, src, nvir, beta, jb, Tc);
 }
 
+constexpr int kOrbitThreads = 1024;
+
+// The elements of a tile that a thread of 1024 owns: as Own, with the planes twice as far apart.
+template <bool PAIR> struct OwnOrbit {
+    static constexpr int PER = TE / kOrbitThreads;
+    int x0, y, z0;
+    __device__ __forceinline__ OwnOrbit() {
+        const int t = threadIdx.x;
+        x0 = __builtin_amdgcn_readfirstlane(PAIR ? t >> 7 : t >> 8);   // the same for a whole wave
+        y = PAIR ? (t >> 3) & (E - 1) : (t >> 4) & (E - 1);
+        z0 = PAIR ? 2 * (t & 7) : t & (E - 1);
+    }
+    static constexpr int dx(int k) { return PAIR ? 8 * (k >> 1) : 4 * k; }
+    static constexpr int dz(int k) { return PAIR ? (k & 1) : 0; }
+};
+
+template <typename T, int W> struct Vec { typedef T t __attribute__((ext_vector_type(W))); };
+template <typename T> struct Vec<T, 1> { typedef T t; };
+template <typename V> __device__ __forceinline__ auto elem(const V &x, int h) {
+    if constexpr (std::is_arithmetic<V>::value) return x;
+    else return x[h];
+}
+
+// As load_tile and store_tile, with the plane in scalar registers and a 32-bit offset of the row: the six
+// tiles of an orbit keep few addresses in vector registers.
+template <typename T, bool PAIR>
+__device__ __forceinline__ void load_rows(const T *__restrict__ blk, int nvir, const I3 Tc, const OwnOrbit<PAIR> &w,
+                                          T *v) {
+    constexpr int kPer = OwnOrbit<PAIR>::PER, W = PAIR ? 2 : 1;
+    typedef typename Vec<T, W>::t V;
+    const int gy = min(Tc.y * E + w.y, nvir - 1), gz = min(Tc.z * E + w.z0, nvir - W);
+    const uint32_t row = (uint32_t)(gy * nvir + gz) * (uint32_t)sizeof(T);
+    const int64_t plane = (int64_t)nvir * nvir;
+#pragma unroll
+    for (int u = 0; u < kPer / W; ++u) {
+        const T *at = blk + min(Tc.x * E + w.x0 + w.dx(W * u), nvir - 1) * plane;   // uniform over the wave
+        const V x = *reinterpret_cast<const V *>(reinterpret_cast<const char *>(at) + row);
+#pragma unroll
+        for (int h = 0; h < W; ++h) v[W * u + h] = elem(x, h);
+    }
+}
+
+template <typename O, bool PAIR>
+__device__ __forceinline__ void store_rows(O *blk, int nvir, const I3 Tc, const OwnOrbit<PAIR> &w, const O *v) {
+    constexpr int kPer = OwnOrbit<PAIR>::PER, W = PAIR ? 2 : 1;
+    typedef typename Vec<O, W>::t V;
+    const int gy = Tc.y * E + w.y, gz = Tc.z * E + w.z0;
+    if (!(gy < nvir && gz < nvir)) return;
+    const uint32_t row = (uint32_t)(gy * nvir + gz) * (uint32_t)sizeof(O);
+    const int64_t plane = (int64_t)nvir * nvir;
+#pragma unroll
+    for (int u = 0; u < kPer / W; ++u) {
+        const int gx = Tc.x * E + w.x0 + w.dx(W * u);
+        if (gx >= nvir) break;
+        V x;
+        if constexpr (PAIR) x = V{v[2 * u], v[2 * u + 1]};
+        else x = v[u];
+        *reinterpret_cast<V *>(reinterpret_cast<char *>(blk + gx * plane) + row) = x;
+    }
+}
+
+template <typename T, bool PAIR>
+__device__ __forceinline__ void stage_rows(T *lds, const OwnOrbit<PAIR> &w, const T *v) {
+    const int base = w.x0 * kSX + w.y * kSY + w.z0;
+#pragma unroll
+    for (int k = 0; k < w.PER; ++k) lds[base + w.dx(k) * kSX + w.dz(k)] = v[k];
+}
+
+// Placement: out[x] += sum over a list of source blocks, each with six coefficients, of
+// sum_p c[p] * src.transpose(p)[x]; the sources lie in up to three buffers.
+//
+// One workgroup of 1024 threads does a whole orbit of 16^3 tiles: the six output tiles stay in registers
+// and every source tile of the orbit is read from memory once, whichever of the six permutations use it.
+// One output tile per workgroup, as above, reads a source once per coefficient; for the ring operator
+// (five coefficients in three sources per part) that was 15 tiles instead of 9 through L2, which bound it.
+// The LDS tile is double buffered (one barrier per source tile) and the loads run three tiles ahead.  HBM
+// bounds it: at nocc=10, nvir=90 in FP64 it moves 14.8 GB in 3.6 ms (7.4 ms a tile at a time); in FP32, rows
+// of half a line, 24 GB in 9.1 ms at nocc=12, nvir=120.
+template <typename T> struct PlaceBufs {
+    const T *b[3];
+};
+
+// kP composed: output tile t of the orbit (coordinates R[kP[t]]) reads, through permutation p, the source
+// tile of index kMul(t, p): source axis p[n] carries R[kP[t][n]].
+constexpr int kPc[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+constexpr int kMul(int t, int p) {
+    int c[3] = {0, 0, 0};
+    for (int n = 0; n < 3; ++n) c[kPc[p][n]] = kPc[t][n];
+    for (int i = 0; i < 6; ++i)
+        if (kPc[i][0] == c[0] && kPc[i][1] == c[1]) return i;
+    return 0;
+}
+
+// The first tile of the orbit with the coordinates of tile s (tiles coincide where AB: A = B, BC: B = C).
+constexpr int kRep(bool AB, bool BC, int s) {
+    const int ab[6] = {0, 1, 0, 1, 4, 4}, bc[6] = {0, 0, 2, 3, 2, 3};
+    return AB && BC ? 0 : AB ? ab[s] : BC ? bc[s] : s;
+}
+// The i-th distinct tile.
+constexpr int kTile(bool AB, bool BC, int i) {
+    const int ab[3] = {0, 1, 4}, bc[3] = {0, 2, 3};
+    return AB && BC ? 0 : AB ? ab[i] : BC ? bc[i] : i;
+}
+
+// AB, BC: which coordinates of the orbit A >= B >= C are equal; known here, so that which output tile a
+// source tile goes to through a permutation costs no run-time test.
+template <typename T, bool PAIR, bool AB, bool BC>
+__device__ __forceinline__ void s3_place_orbit(T (*lds)[kLdsTile], T *__restrict__ dst, const PlaceBufs<T> &bufs,
+                                               int nvir, const dcc_s3_place_src *__restrict__ src, int n, int A,
+                                               int B, int C) {
+    typedef OwnOrbit<PAIR> W;
+    constexpr int NT = AB && BC ? 1 : AB || BC ? 3 : 6;   // distinct tiles
+    constexpr int AHEAD = 3, NS = NT == 1 ? AHEAD : 1;   // sources per turn of the loop
+    const W w;
+    auto coords = [&](int s) { return I3{pick3(kPc[s][0], A, B, C), pick3(kPc[s][1], A, B, C), pick3(kPc[s][2], A, B, C)}; };
+    auto base = [&](int i) {
+        const int64_t b = src[i].buf;
+        return (b == 0 ? bufs.b[0] : b == 1 ? bufs.b[1] : bufs.b[2]) + src[i].off;
+    };
+    // tile i of the turn that starts at source sn: its source, and its place in the orbit
+    auto source = [&](int sn, int i) { return sn + (NT == 1 ? i : i / NT); };
+    auto load = [&](int sn, int i, T *v) {
+        if (source(sn, i) < n) load_rows<T, PAIR>(base(source(sn, i)), nvir, coords(kTile(AB, BC, i % NT)), w, v);
+    };
+    double acc[NT][W::PER] = {};
+    T v[AHEAD][W::PER];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) load(0, i, v[i]);
+    T *tile = lds[0], *other = lds[1];
+#pragma unroll 1
+    for (int sn = 0; sn < n; sn += NS) {
+#pragma unroll
+        for (int i = 0; i < NT * NS; ++i) {
+            if (source(sn, i) >= n) break;   // uniform
+            const double *cf = src[source(sn, i)].coef;
+            stage_rows<T, PAIR>(tile, w, v[i % AHEAD]);
+            __syncthreads();
+            load(sn, i + AHEAD, v[i % AHEAD]);
+#pragma unroll
+            for (int p = 0; p < 6; ++p) {
+                if ((__double_as_longlong(cf[p]) << 1) == 0) continue;   // zero; uniform
+                const int s0 = kPc[p][0] == 0 ? kSX : kPc[p][0] == 1 ? kSY : 1;
+                const int s1 = kPc[p][1] == 0 ? kSX : kPc[p][1] == 1 ? kSY : 1;
+                const int s2 = kPc[p][2] == 0 ? kSX : kPc[p][2] == 1 ? kSY : 1;
+                const T *at = tile + w.x0 * s0 + w.y * s1 + w.z0 * s2;
+                double x[W::PER];
+#pragma unroll
+                for (int k = 0; k < W::PER; ++k) x[k] = (double)at[w.dx(k) * s0 + w.dz(k) * s2];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    if (kRep(AB, BC, kMul(kTile(AB, BC, t), p)) != kTile(AB, BC, i % NT)) continue;
+#pragma unroll
+                    for (int k = 0; k < W::PER; ++k) acc[t][k] += cf[p] * x[k];
+                }
+            }
+            T *u = tile;
+            tile = other;
+            other = u;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        T old[W::PER];
+        load_rows<T, PAIR>(dst, nvir, coords(kTile(AB, BC, t)), w, old);
+#pragma unroll
+        for (int k = 0; k < W::PER; ++k) old[k] = (T)((double)old[k] + acc[t][k]);
+        store_rows<T, PAIR>(dst, nvir, coords(kTile(AB, BC, t)), w, old);
+    }
+}
+
+template <typename T, bool PAIR>
+__device__ __forceinline__ void s3_place_orbit(T (*lds)[kLdsTile], T *dst, const PlaceBufs<T> &bufs, int nvir,
+                                               const dcc_s3_place_src *src, int n, int A, int B, int C) {
+    if (A == B && B == C) s3_place_orbit<T, PAIR, true, true>(lds, dst, bufs, nvir, src, n, A, B, C);
+    else if (A == B) s3_place_orbit<T, PAIR, true, false>(lds, dst, bufs, nvir, src, n, A, B, C);
+    else if (B == C) s3_place_orbit<T, PAIR, false, true>(lds, dst, bufs, nvir, src, n, A, B, C);
+    else s3_place_orbit<T, PAIR, false, false>(lds, dst, bufs, nvir, src, n, A, B, C);
+}
+
+template <typename T, bool PAIR>
+__global__ __launch_bounds__(kOrbitThreads) void s3_place_kernel(T *__restrict__ out, const PlaceBufs<T> bufs,
+                                                                 int nvir,
+                                                                 const dcc_s3_place_job *__restrict__ jobs,
+                                                                 const dcc_s3_place_src *__restrict__ srcs, int nt,
+                                                                 int nso) {
+    __shared__ T lds[2][kLdsTile];
+    // runs of 8 orbits (a 2x2x2 block of tile triples, as in tile_of) on one XCD
+    const int64_t b = dcc_gemm::xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t job = b / (8 * (int64_t)nso);
+    const int r = (int)(b - job * 8 * (int64_t)nso);
+    int SA, SB, SC;
+    decode_orbit(r / 8, SA, SB, SC);
+    const int A = 2 * SA + ((r >> 2) & 1), B = 2 * SB + ((r >> 1) & 1), C = 2 * SC + (r & 1);
+    if (!(A >= B && B >= C && A < nt)) return;
+    const dcc_s3_place_job jb = jobs[job];
+    const dcc_s3_place_src *src = srcs + jb.first;
+    int64_t odd = jb.dst;
+    for (int s = 0; s < jb.count; ++s) odd |= src[s].off;
+    if (PAIR && (odd & 1) == 0) s3_place_orbit<T, true>(lds, out + jb.dst, bufs, nvir, src, jb.count, A, B, C);
+    else s3_place_orbit<T, false>(lds, out + jb.dst, bufs, nvir, src, jb.count, A, B, C);
+}
+
 // The fused projection/update keeps the 8x8x8 tile orbits: one workgroup reads the six tiles of an
 // orbit of R from HBM once and writes the six output tiles.  In the per-output-tile form above the
 // six tiles of an orbit each re-read all six source tiles through L2, one after another, and the
@@ -565,6 +767,26 @@ int s3_gather(T *out, const T *src, int64_t nvir, double beta, const dcc_s3_gath
     return 0;
 }
 
+template <typename T>
+int s3_place(T *out, const T *src0, const T *src1, const T *src2, int64_t nvir, const dcc_s3_place_job *jobs,
+             int64_t njobs, const dcc_s3_place_src *srcs, dcc_stream_t stream) {
+    DCC_CHECK(nvir >= 0 && njobs >= 0, "negative extent");
+    if (nvir == 0 || njobs == 0) return 0;
+    DCC_CHECK(out && src0 && src1 && src2 && jobs && srcs, "null pointer");
+    const int64_t nt = (nvir + E - 1) / E, nso = n_orbits((nt + 1) / 2);
+    DCC_CHECK(8 * nso * njobs * kOrbitThreads < ((int64_t)1 << 32), "grid too large");
+    const PlaceBufs<T> bufs{{src0, src1, src2}};
+    const dim3 grid((unsigned)(8 * nso * njobs));
+    if (pair_ok(nvir, out, src0) && pair_ok(nvir, src1, src2))
+        hipLaunchKernelGGL((s3_place_kernel<T, true>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream), out, bufs,
+                           (int)nvir, jobs, srcs, (int)nt, (int)nso);
+    else
+        hipLaunchKernelGGL((s3_place_kernel<T, false>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream), out, bufs,
+                           (int)nvir, jobs, srcs, (int)nt, (int)nso);
+    DCC_LAUNCH_CHECK();
+    return 0;
+}
+
 template <typename T, typename O = T>
 int s3_transform(O *out, const T *src, int64_t nvir, double beta, const dcc_s3_job *jobs, int64_t njobs,
                  dcc_stream_t stream) {
@@ -656,6 +878,18 @@ int dcc_s3_gather_f64(double *out, const double *src, int64_t nvir, double beta,
 int dcc_s3_gather_f32(float *out, const float *src, int64_t nvir, double beta, const dcc_s3_gather_job *jobs,
                       int64_t njobs, dcc_stream_t stream) {
     return s3_gather<float>(out, src, nvir, beta, jobs, njobs, stream);
+}
+
+int dcc_s3_place_f64(double *out, const double *src0, const double *src1, const double *src2, int64_t nvir,
+                     const dcc_s3_place_job *jobs, int64_t njobs, const dcc_s3_place_src *srcs,
+                     dcc_stream_t stream) {
+    return s3_place<double>(out, src0, src1, src2, nvir, jobs, njobs, srcs, stream);
+}
+
+int dcc_s3_place_f32(float *out, const float *src0, const float *src1, const float *src2, int64_t nvir,
+                     const dcc_s3_place_job *jobs, int64_t njobs, const dcc_s3_place_src *srcs,
+                     dcc_stream_t stream) {
+    return s3_place<float>(out, src0, src1, src2, nvir, jobs, njobs, srcs, stream);
 }
 
 int64_t dcc_r3_finalize_tiles(int64_t nvir) {

@@ -4,9 +4,10 @@ the T3 -> r1/r2/W contributions, as launches of libdcc kernels.
 Data in HBM (FP64, C order):
   t3, R          (n3, v, v, v)     canonical blocks, lexicographic i<=j<=k
   Y              (npairs, o, v, v, v)  Y[(p,q)][l] = T[l,p,q] for p<=q (ring B operand)
-  Z              (npairs, o, v, v, v)  Y[l][b,d,c] + Y[l][c,b,d] stored as [d,b,c], right after Y
+  Z              (npairs, o, v, v, v)  Y[l][d,b,c] - 1/2 (Y[l][b,d,c] + Y[l][c,b,d]), right after Y
   WR1, WR3[2]    (o, v, o, v)      ring weights, rows (r,x), cols (l,d)
-  Gs             (pairs per chunk, o, v, v, v)  G[r;pq][a,b,c] before its placement
+  Gs             (pairs per chunk, o, v, v, v)  ring products of row x = (r,a) before their placement
+                                   (with Z three such buffers, two of them views of Xt and Xp)
   Xt             (i per chunk, o, o, v, v, v)   T2->T3 base term X over ordered (i,j,k)
   pfs            (6, n3, n3)       W_oooo/F_oo prefactors
   W1             (v, v, v, v)      W_vvvv with the F_vv terms folded in
@@ -29,10 +30,13 @@ batched gather-GEMMs (dcc_contract_f64):
                         + W_ovvo[l,a,d,r] Y[l][d,b,c]
                         - 1/2 (W_ovov[l,a,r,d] + W_ovvo[l,a,d,r]) (Y[l][b,d,c] + Y[l][c,b,d]) )
     part 3 of target (i,j,k) is G[i;jk], part 4 is G[j;ik] with (a,b) swapped and
-    part 5 is G[k;ij] read as [c,a,b]; G is computed once for all r (GEMMs batched over
-    the pairs p<=q, rows (r, x)) into a scratch buffer and placed by one S3 gather pass
-    (all three parts of a target at once); with Z the W_ovvo term and the two
-    (W_ovov + W_ovvo) terms are one GEMM over K = (term, l, d), B = [Y; Z];
+    part 5 is G[k;ij] read as [c,a,b].  With Z, three products (batched over the pairs p<=q, rows
+    (r, x) for all r, K = (l, d)) hold all of it:
+        G0[x,b,c] = W_ovvo[l,x,d,r] Z[l][d,b,c]
+        F1[x,y,z] = -W_ovov[l,x,r,d] Y[l][y,d,z],  F2[x,y,z] = -W_ovov[l,x,r,d] Y[l][y,z,d]
+        G[a,b,c] = G0[a,b,c] + F1[b,a,c] + 1/2 F1[a,b,c] + F2[c,a,b] + 1/2 F2[a,c,b]
+    and one placement pass adds the permuted blocks (all three parts of a target at once).  Without Z
+    the five terms are accumulated as they stand into one G;
   * W_oooo/F_oo x T3 (rccsdt.py:616-732): 6 GEMMs M = n3 targets, K = n3 sources,
     N = v^3, with the prefactors built on the device; term 0 goes straight into R, terms
     1..5 into Xp per chunk of targets and are added, permuted, by one S3 gather pass.
@@ -362,7 +366,7 @@ class T2T3Operands:
                self.n, stream.handle if stream is not None else None)
 
 
-def plan_t2t3(o, v, R, t2, W_ovvv, W_oovo, scratch_bytes, packed=False):
+def plan_t2t3(o, v, R, t2, W_ovvv, W_oovo, scratch_bytes, packed=False, min_blocks=0):
     """T2 -> T3 terms (rccsdt.py:388-399) added into the canonical blocks R; returns (Xt, launches).
 
     The twelve terms are the six simultaneous (ijk, abc) permutations of one base term
@@ -373,13 +377,16 @@ def plan_t2t3(o, v, R, t2, W_ovvv, W_oovo, scratch_bytes, packed=False):
     once (two GEMMs -- K = d, then K = l adding into X -- wrote it and then read and rewrote it), and
     one multi-source S3 gather pass adds, for every canonical target, its (up to six) permuted source
     blocks in one read-modify-write.  Ordered triples are processed in chunks of the first index whose
-    X fits ``scratch_bytes``; Xt is that chunk buffer (ic, o, o, v, v, v).  ``packed``: the GEMM runs
+    X fits ``scratch_bytes``; Xt is that chunk buffer (ic, o, o, v, v, v), with room for ``min_blocks``
+    blocks after its use here.  ``packed``: the GEMM runs
     as split-BF16x3 products on operands packed by T2T3Operands (when K = v + o > 16; a shorter K stays
     on FP32 like every such GEMM of the split-BF16x3 engine)."""
     v3 = v ** 3
     dt = R.dtype
     ic = int(max(1, min(o, scratch_bytes // max(1, o * o * v3 * dt.itemsize))))
-    Xt = DeviceArray((ic, o, o, v, v, v), dt)
+    store = DeviceArray((max(ic * o * o, min_blocks), v, v, v), dt)
+    Xt = DeviceArray((ic, o, o, v, v, v), dt, ptr=store.ptr, owner=False)
+    Xt.store = store
     K2 = v + o
     packed = packed and K2 > 16
     Ap = DeviceArray((ic, v, o, v, K2), dt)
@@ -426,6 +433,31 @@ def s3_jobs_array(jobs):
     return arr
 
 
+class S3PlaceLaunch:
+    """One dcc_s3_place call: out[dst] += sum of src.transpose(TP_T3[p]) * coef[p] over a job's sources
+    (buffer index, offset, {permutation: coefficient})."""
+
+    def __init__(self, name, out, bufs, nvir, jobs):
+        self.name, self.flops = name, 0.0
+        self.fn = "dcc_s3_place_" + _suffix(out.dtype)
+        self.out, self.bufs, self.nvir, self.njobs = out, tuple(bufs), int(nvir), len(jobs)
+        job = np.zeros(len(jobs), dtype=L.S3PLACE_JOB_DTYPE)
+        src = np.zeros(sum(len(lst) for _, lst in jobs), dtype=L.S3PLACE_SRC_DTYPE)
+        n = 0
+        for j, (dst, lst) in zip(job, jobs):
+            j['dst'], j['first'], j['count'] = dst, n, len(lst)
+            for buf, off, coef in lst:
+                src[n]['buf'], src[n]['off'] = buf, off
+                for p, c in coef.items():
+                    src[n]['coef'][TP_T3.index(p)] += c
+                n += 1
+        self.jobs, self.srcs = DeviceArray.from_host(job), DeviceArray.from_host(src)
+
+    def run(self, stream):
+        L.call(self.fn, self.out.vp, *(b.vp for b in self.bufs), self.nvir, self.jobs.vp, self.njobs, self.srcs.vp,
+               stream.handle if stream is not None else None)
+
+
 class TriplesEngine:
     """Holds the device state of one RCCSDT triples update for (nocc, nvir)."""
 
@@ -437,10 +469,10 @@ class TriplesEngine:
         only) runs every contraction as split-BF16x3 products on BF16 MFMA instead.
 
         ``ring_fused`` (default: when the device has room for a second Y-sized buffer) stores
-        Z[(p,q)][l][d,b,c] = Y[l][b,d,c] + Y[l][c,b,d] next to Y, so the two terms that share the
-        W_ovov + W_ovvo weight become one, fused along K with the W_ovvo term: three ring
-        GEMMs per part instead of five, and 4/5 of the ring flops.  ``ring_g_bytes`` bounds the
-        scratch buffer of the ring operator G (pairs are processed in chunks that fit).
+        Z[(p,q)][l][d,b,c] = Y[l][d,b,c] - 1/2 (Y[l][b,d,c] + Y[l][c,b,d]) next to Y, so all terms of
+        W_ovvo are one product and each product of W_ovov serves two terms: three ring GEMMs instead
+        of five, and 3/5 of the ring flops.  ``ring_g_bytes`` bounds each scratch buffer of the ring
+        products (pairs are processed in chunks that fit).
 
         ``vvvv_pairs`` runs the three W_vvvv terms as symmetric and antisymmetric products over
         triangular index pairs (half the flops; dcc_vvvv_pair_* in the library), which requires a
@@ -505,7 +537,10 @@ class TriplesEngine:
         if qc >= 32 and -(-qc // 64) * 64 * per_target * 4 <= 5 * ring_g_bytes:
             qc = -(-qc // 64) * 64
         qc = int(max(1, min(n3, qc)))
-        self.Xp = DeviceArray((5, qc, v, v, v), dt)
+        # pairs per chunk of the ring; with Z, Xp and Xt (plan_t2t3) each also hold one of its products
+        self.ring_pairs = int(max(1, min(self.npairs, ring_g_bytes // max(1, o * v3 * dt.itemsize))))
+        self._xp_store = DeviceArray((max(5 * qc, self._ring_blocks()), v, v, v), dt)
+        self.Xp = DeviceArray((5, qc, v, v, v), dt, ptr=self._xp_store.ptr, owner=False)
         self.eia = DeviceArray((o, v))
         self._eia_host = None    # what it holds
         self.norb = int(L._lib.dcc_r3_finalize_tiles(v))
@@ -521,7 +556,7 @@ class TriplesEngine:
                 jobs.append(((pq * o + l) * v3, ijk_to_linear(ci, cj, ck, o) * v3, coef))
         self.y_jobs = DeviceArray.from_host(s3_jobs_array(jobs))
         self.n_y_jobs = len(jobs)
-        # --- Z jobs: Z[(p,q)][l] = Y[(p,q)][l].transpose(1,0,2) + Y[(p,q)][l].transpose(2,1,0), from T ---
+        # --- Z jobs: Z[(p,q)][l] = Y - 1/2 (Y.transpose(1,0,2) + Y.transpose(2,1,0)), from T ---
         if self.ring_fused:
             jobs = []
             for pq, (p, q) in enumerate(self.pairs):
@@ -529,8 +564,8 @@ class TriplesEngine:
                     case, (ci, cj, ck) = canonical_case(l, p, q)
                     a = TP_T3[case]
                     coef = np.zeros(6)
-                    for b in ((1, 0, 2), (2, 1, 0)):
-                        coef[TP_T3.index((a[b[0]], a[b[1]], a[b[2]]))] += 1.0
+                    for b, x in (((0, 1, 2), 1.0), ((1, 0, 2), -0.5), ((2, 1, 0), -0.5)):
+                        coef[TP_T3.index((a[b[0]], a[b[1]], a[b[2]]))] += x
                     jobs.append(((pq * o + l) * v3, ijk_to_linear(ci, cj, ck, o) * v3, coef))
             self.z_jobs = DeviceArray.from_host(s3_jobs_array(jobs))
         # --- pair-symmetric W_vvvv: weights [nS + nA][kpad], split T3 and products for a chunk of blocks
@@ -726,47 +761,97 @@ class TriplesEngine:
     def _plan_t2t3(self):
         """T2 -> T3 terms (plan_t2t3), with the base-term scratch bounded by ``ring_g_bytes``."""
         self.Xt, launches = plan_t2t3(self.nocc, self.nvir, self.R, self.t2, self.W_ovvv, self.W_oovo,
-                                      self.ring_g_bytes, packed=self.contract == "bf16x3")
+                                      self.ring_g_bytes, packed=self.contract == "bf16x3",
+                                      min_blocks=self._ring_blocks())
         return launches
 
-    def _plan_ring(self):
-        """Ring terms (rccsdt.py:540-596).
+    def _ring_blocks(self):
+        """Blocks that Xp and Xt hold for a ring product of a chunk (none without Z)."""
+        return self.ring_pairs * self.nocc if self.ring_fused else 0
 
-        G[r;pq] (the part-3 operator of the module docstring) is the same for the three parts; only
-        its placement differs (part 3 of target (r,p,q) is G[r;pq], part 4 of (p,r,q) is G[r;pq] with
-        (a,b) swapped, part 5 of (p,q,r) is G[r;pq] read as [c,a,b]).  So G is computed once for every
-        r into a scratch buffer Gs[pair][r][a,b,c] -- GEMMs with M = (r, x) over all o*v rows,
-        batched over pairs, plain strided output -- and then added into R by one S3 placement pass
-        per part.  Pairs are processed in chunks whose G fits ``ring_g_bytes``."""
+    def _plan_ring(self):
+        return self._plan_ring_products() if self.ring_fused else self._plan_ring_terms()
+
+    def _plan_ring_products(self):
+        """Ring terms (rccsdt.py:540-596) as three products per chunk of pairs, G0 into Gs, F1 into Xt and
+        F2 into Xp (module docstring), and one placement pass.  The two scratch buffers are idle here:
+        Xt after the T2 -> T3 and W_vvvv terms, Xp before the W_oooo/F_oo ones (one stream).  Every product
+        is written once, with rows of v^2 contiguous elements.  Accumulated into one G as the terms stand
+        (W_ovvo and W_ovov + W_ovvo as one product over twice the K) they were 4 units of flops against 3
+        here, and G was written, then read and rewritten twice: with the placement 58.5 ms at nocc=10,
+        nvir=90 in FP64 against 46.5 ms now, 72 against 54 ms at nocc=12, nvir=120 in split BF16."""
         o, v = self.nocc, self.nvir
         v2, v3 = v * v, v ** 3
         ov = o * v
         dt = self.dtype
-        pc = int(max(1, min(self.npairs, self.ring_g_bytes // max(1, o * v3 * dt.itemsize))))
+        pc = self.ring_pairs
+        shape = (pc, o, v, v, v)
+        self.Gs = DeviceArray(shape, dt)
+        F1 = DeviceArray(shape, dt, ptr=self.Xt.ptr, owner=False)
+        F2 = DeviceArray(shape, dt, ptr=self._xp_store.ptr, owner=False)
+        # name, weight, B, output, B maps of (l, d) and of the two N axes
+        products = [('ring WR3 M0', self.WR3a, self.Z, self.Gs, L.IdxMap(None, 0, 1, ov, 0, 0, v2),
+                     L.IdxMap(None, 0, 1, v2, 0, 0, 1)),
+                    ('ring WR1 M1', self.WR1, self.Y, F1, L.IdxMap(None, 0, o, v, 0, v3, v),
+                     L.IdxMap(None, 0, v, v, 0, v2, 1)),
+                    ('ring WR1 M2', self.WR1, self.Y, F2, L.IdxMap(None, 0, o, v, 0, v3, 1),
+                     L.IdxMap(None, 0, 1, v2, 0, 0, v))]
+        am, ak = L.IdxMap(None, 0, 1, ov, 0, 0, ov), L.IdxMap(None, 0, 1, ov, 0, 0, 1)
+        cm, cn = L.IdxMap(None, 0, 1, ov, 0, 0, v2), L.IdxMap(None, 0, 1, v2, 0, 0, 1)
+        # G = sum over the products of coefficient * product.transpose(q)
+        parts_of_g = [{(0, 1, 2): 1.0}, {(1, 0, 2): 1.0, (0, 1, 2): 0.5}, {(1, 2, 0): 1.0, (0, 2, 1): 0.5}]
+        launches = []
+        for c0 in range(0, self.npairs, pc):
+            chunk = list(enumerate(self.pairs))[c0:c0 + pc]
+            batches = [(0, pq * o * v3, (pq - c0) * o * v3, 0, ov) for pq, _ in chunk]
+            for name, W, B, C, bk, bn in products:
+                launches.append(GemmLaunch(name, ov, v2, ov, 1.0, 0.0, W, am, ak, B, bk, bn, C, cm, cn, batches, ov,
+                                           2.0 * len(chunk) * ov * v2 * ov))
+            jobs = []
+            for tq, lst in self._ring_targets(chunk, c0):
+                srcs = []
+                for perm, blk in lst:
+                    for buf, terms in enumerate(parts_of_g):
+                        # X.transpose(q).transpose(perm) = X.transpose(q[perm])
+                        srcs.append((buf, blk * v3, {tuple(q[n] for n in perm): c for q, c in terms.items()}))
+                jobs.append((tq * v3, srcs))
+            launches.append(S3PlaceLaunch('ring place', self.R, (self.Gs, F1, F2), v, jobs))
+        return launches
+
+    def _ring_targets(self, chunk, c0):
+        """[(target block, [(permutation of G, block of the chunk)])]: part 3 of target (r,p,q) is G[r;pq],
+        part 4 of (p,r,q) is G[r;pq] with (a,b) swapped, part 5 of (p,q,r) is G[r;pq] read as [c,a,b]."""
+        o = self.nocc
+        targets = {}
+        for pq, (p, q) in chunk:
+            for r in range(o):
+                blk = (pq - c0) * o + r
+                if r <= p:
+                    targets.setdefault(ijk_to_linear(r, p, q, o), []).append(((0, 1, 2), blk))
+                if p <= r <= q:
+                    targets.setdefault(ijk_to_linear(p, r, q, o), []).append(((1, 0, 2), blk))
+                if r >= q:
+                    targets.setdefault(ijk_to_linear(p, q, r, o), []).append(((1, 2, 0), blk))
+        return sorted(targets.items())
+
+    def _plan_ring_terms(self):
+        """Ring terms (rccsdt.py:540-596) without Z: G[r;pq] (the part-3 operator of the module docstring,
+        which the three parts only place differently) is accumulated term by term for every r into a
+        scratch buffer Gs[pair][r][a,b,c] -- GEMMs with M = (r, x) over all o*v rows, batched over pairs,
+        plain strided output -- and then added into R by one S3 gather pass.  Pairs are processed in
+        chunks whose G fits ``ring_g_bytes``."""
+        o, v = self.nocc, self.nvir
+        v2, v3 = v * v, v ** 3
+        ov = o * v
+        dt = self.dtype
+        pc = self.ring_pairs
         self.Gs = DeviceArray((pc, o, v, v, v), dt)
         Sg = (v2, v, 1)   # strides of [a,b,c] in a G block
-
-        def rows(part, p, q):
-            return {3: (0, p + 1), 4: (p, q + 1), 5: (q, o)}[part]
-
-        def target(part, r, p, q):
-            t = {3: (r, p, q), 4: (p, r, q), 5: (p, q, r)}[part]
-            return ijk_to_linear(t[0], t[1], t[2], o)
-
-        # placement of G[a,b,c] in the target block, as the S3 permutation of the source block
-        perm = {3: (0, 1, 2), 4: (1, 0, 2), 5: (1, 2, 0)}
         # term: (weight, G axis carried by M, N axes (outer, inner), B strides of d, n_outer, n_inner)
-        terms = []
-        if self.ring_fused:
-            # W_ovvo[l,a,d,r] Y[l][d,b,c] - 1/2(..) Z[l][d,b,c] as one GEMM over K = (term, l, d)
-            terms.append(('WR3', 0, (1, 2), v2, v, 1))
-        else:
-            terms += [
-                ('WR3a', 0, (1, 2), v2, v, 1),   #  W_ovvo[l,a,d,r] Y[l][d,b,c]
-                ('WR3b', 0, (1, 2), v, v2, 1),   # -1/2(..) Y[l][b,d,c]
-                ('WR3b', 0, (1, 2), 1, v, v2),   # -1/2(..) Y[l][c,b,d]
-            ]
-        terms += [
+        terms = [
+            ('WR3a', 0, (1, 2), v2, v, 1),   #  W_ovvo[l,a,d,r] Y[l][d,b,c]
+            ('WR3b', 0, (1, 2), v, v2, 1),   # -1/2(..) Y[l][b,d,c]
+            ('WR3b', 0, (1, 2), 1, v, v2),   # -1/2(..) Y[l][c,b,d]
             ('WR1', 1, (0, 2), v, v2, 1),    # -W_ovov[l,b,r,d] Y[l][a,d,c]
             ('WR1', 2, (0, 1), 1, v2, v),    # -W_ovov[l,c,r,d] Y[l][a,b,d]
         ]
@@ -775,36 +860,26 @@ class TriplesEngine:
             chunk = list(enumerate(self.pairs))[c0:c0 + pc]
             batches = [(0, pq * o * v3, (pq - c0) * o * v3, 0, ov) for pq, _ in chunk]
             for n, (wname, mx, (n0, n1), sd, sn0, sn1) in enumerate(terms):
-                W = getattr(self, wname)
-                nt = 2 if wname == 'WR3' else 1                  # terms fused along K
                 am = L.IdxMap(None, 0, 1, ov, 0, 0, ov)          # row (r,x) of the (ov x ov) weight
-                ak = L.IdxMap(None, 0, 1, ov, ov * ov, 0, 1)     # (term, (l,d))
-                zoff = self.npairs * o * v3                      # Z follows Y in one buffer
-                bk = L.IdxMap(None, 0, o, v, zoff, v3, sd)       # (term, l, d)
+                ak = L.IdxMap(None, 0, 1, ov, 0, 0, 1)           # (l, d)
+                bk = L.IdxMap(None, 0, o, v, 0, v3, sd)          # (l, d)
                 bn = L.IdxMap(None, 0, v, v, 0, sn0, sn1)        # (n_outer, n_inner)
                 cm = L.IdxMap(None, 0, o, v, 0, v3, Sg[mx])      # (r, x)
                 cn = L.IdxMap(None, 0, v, v, 0, Sg[n0], Sg[n1])
-                launches.append(GemmLaunch('ring %s M%d' % (wname, mx), ov, v2, nt * ov, 1.0,
-                                           0.0 if n == 0 else 1.0, W, am, ak, self.Y, bk, bn, self.Gs, cm, cn,
-                                           batches, ov, 2.0 * len(chunk) * ov * v2 * ov * nt))
+                launches.append(GemmLaunch('ring %s M%d' % (wname, mx), ov, v2, ov, 1.0, 0.0 if n == 0 else 1.0,
+                                           getattr(self, wname), am, ak, self.Y, bk, bn, self.Gs, cm, cn,
+                                           batches, ov, 2.0 * len(chunk) * ov * v2 * ov))
             # one gather pass: each target takes its (up to three) part contributions of this chunk
-            contrib = {}
-            for part in (3, 4, 5):
-                pidx = TP_T3.index(perm[part])
-                for pq, (p, q) in chunk:
-                    r0, r1 = rows(part, p, q)
-                    for r in range(r0, r1):
-                        contrib.setdefault(target(part, r, p, q), []).append((pidx, ((pq - c0) * o + r) * v3))
             jobs = []
-            for tq, lst in sorted(contrib.items()):
+            for tq, lst in self._ring_targets(chunk, c0):
                 srcs, coef = [0] * 6, np.zeros(6)
-                for pidx, off in lst:
+                for perm, blk in lst:
+                    pidx = TP_T3.index(perm)
                     assert coef[pidx] == 0.0   # the three parts use three different permutations
-                    srcs[pidx], coef[pidx] = off, 1.0
+                    srcs[pidx], coef[pidx] = blk * v3, 1.0
                 jobs.append((tq * v3, srcs, coef))
             launches.append(S3GatherLaunch('ring place', self.R, self.Gs, v, 1.0, jobs))
         return launches
-
 
     # ------------------------------------------------- T3 -> r1/r2 and T3 -> W
     def _setup_lower(self, z_budget_bytes=16 << 30):

@@ -216,6 +216,29 @@ int dcc_s3_gather_f32(float *out, const float *src, int64_t nvir, double beta,
                       const dcc_s3_gather_job *jobs, int64_t njobs, dcc_stream_t stream);
 
 /*
+ * Placement of permuted blocks: each job adds to the out block at dst, for its `count` sources from
+ * srcs[first], sum_p coef[p] * (block at off of buffer buf).transpose(p) (buf: 0 src0, 1 src1, 2 src2;
+ * permutations as in dcc_s3_job; FP64 sums).  Used for the ring operator, whose three products land in
+ * up to three parts of a target with two permutations of two of them (distr_cc/rccsdt.py:540-596).
+ * Jobs of one call must have distinct dst blocks; out must not overlap the sources.
+ */
+typedef struct dcc_s3_place_src {
+    int64_t off;
+    int64_t buf;
+    double coef[6];
+} dcc_s3_place_src;
+typedef struct dcc_s3_place_job {
+    int64_t dst;
+    int32_t first, count;
+} dcc_s3_place_job;
+int dcc_s3_place_f64(double *out, const double *src0, const double *src1, const double *src2, int64_t nvir,
+                     const dcc_s3_place_job *jobs, int64_t njobs, const dcc_s3_place_src *srcs,
+                     dcc_stream_t stream);
+int dcc_s3_place_f32(float *out, const float *src0, const float *src1, const float *src2, int64_t nvir,
+                     const dcc_s3_place_job *jobs, int64_t njobs, const dcc_s3_place_src *srcs,
+                     dcc_stream_t stream);
+
+/*
  * Fused end of the triples update (distr_cc/rccsdt.py:947-971):
  *   r = (R - (1/6) sum_p R.transpose(p)) / (eia[i,a] + eia[j,b] + eia[k,c])
  *   t3 += r;  optionally r3_out = r;

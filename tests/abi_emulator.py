@@ -567,6 +567,33 @@ class Emulator:
             o[...] = ((beta * o.astype(np.float64) if beta != 0.0 else 0.0) + val).astype(dt)
         return 0
 
+    def dcc_s3_place_f64(self, *a):
+        return self._s3_place(np.float64, *a)
+
+    def dcc_s3_place_f32(self, *a):
+        return self._s3_place(np.float32, *a)
+
+    def _s3_place(self, dt, out, src0, src1, src2, nvir, jobs, njobs, srcs, stream):
+        v = int(nvir)
+        O = self.dev.view(_ptr(out), dt)
+        S = [self.dev.view(_ptr(x), dt) for x in (src0, src1, src2)]
+        sdt = np.dtype([("off", np.int64), ("buf", np.int64), ("coef", np.float64, (6,))])
+        jdt = np.dtype([("dst", np.int64), ("first", np.int32), ("count", np.int32)])
+        jb = self.dev.view(_ptr(jobs), np.uint8, int(njobs) * jdt.itemsize).view(jdt)
+        assert len(set(int(d) for d in jb["dst"])) == len(jb), "S3 jobs of one call share a destination"
+        ns = int((jb["first"] + jb["count"]).max())
+        sr = self.dev.view(_ptr(srcs), np.uint8, ns * sdt.itemsize).view(sdt)
+        for j in jb:
+            o = O[int(j["dst"]): int(j["dst"]) + v ** 3].reshape(v, v, v)
+            val = o.astype(np.float64)
+            for s in sr[int(j["first"]): int(j["first"]) + int(j["count"])]:
+                x = S[int(s["buf"])][int(s["off"]): int(s["off"]) + v ** 3].reshape(v, v, v).astype(np.float64)
+                for c, p in zip(s["coef"], _PERMS):
+                    if c != 0.0:
+                        val = val + c * x.transpose(p)
+            o[...] = val.astype(dt)
+        return 0
+
     def dcc_r3_finalize_f64(self, *a):
         return self._finalize(np.float64, *a)
 

@@ -163,6 +163,50 @@ def test_s3_gather_multi_source(dev, v, dt, shift):
         assert abs(out[q] - ref).max() < tol * max(1.0, abs(ref).max()), (q, v)
 
 
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("v", [1, 7, 16, 18, 33, 50])
+def test_s3_place(dev, v, dt, shift):
+    """dcc_s3_place_*: sources of three buffers with several permutations each, a job without sources, a
+    source without coefficients; ``shift`` = 1 moves every block one element off alignment.  Sums are FP64,
+    so the tolerance is a rounding of the result (f32) or of each of up to 9 terms (f64)."""
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    _say("s3 place v=%d %s shift %d" % (v, dt, shift))
+    rng = np.random.default_rng(60 + v)
+    typ = np.float64 if dt == "f64" else np.float32
+    X = [rng.normal(size=(2, v, v, v)).astype(typ) for _ in range(3)]
+    O0 = rng.normal(size=(4, v, v, v)).astype(typ)
+    perms = ((0, 1, 2), (0, 2, 1), (1, 0, 2), (1, 2, 0), (2, 0, 1), (2, 1, 0))
+    v3 = v ** 3
+    jobs = [(2, [(0, 0, [1.0, 0, 0, 0, 0, 0]), (1, 1, [0.5, 0, 1.0, 0, 0, 0]), (2, 0, [0, 0.5, 0, 1.0, 0, 0])]),
+            (0, [(1, 0, [0, 0, 0, 0, 0, 0]), (2, 1, [0, 0, 0, 0, -2.0, 3.0])]), (3, []),
+            (1, [(0, 1, [1.0, -1.0, 0.5, 2.0, -0.25, 3.0])])]
+    job = np.zeros(len(jobs), dtype=L.S3PLACE_JOB_DTYPE)
+    src = np.zeros(sum(len(j[1]) for j in jobs), dtype=L.S3PLACE_SRC_DTYPE)
+    n = 0
+    for x, (q, lst) in zip(job, jobs):
+        x['dst'], x['first'], x['count'] = q * v3 + shift, n, len(lst)
+        for buf, blk, coef in lst:
+            src[n]['buf'], src[n]['off'], src[n]['coef'] = buf, blk * v3 + shift, coef
+            n += 1
+    pad = np.zeros(shift, typ)
+    dX = [DeviceArray.from_host(np.concatenate([pad, x.ravel()])) for x in X]
+    dO = DeviceArray.from_host(np.concatenate([pad, O0.ravel()]))
+    dj, ds = DeviceArray.from_host(job), DeviceArray.from_host(src)
+    L.call("dcc_s3_place_" + dt, dO.vp, dX[0].vp, dX[1].vp, dX[2].vp, v, dj.vp, len(jobs), ds.vp, None)
+    outf = dO.download()
+    assert np.all(outf[:shift] == 0)
+    out = outf[shift:].reshape(O0.shape).astype(np.float64)
+    tol = 1e-13 if dt == "f64" else 1e-6
+    for q, lst in jobs:
+        ref = O0[q].astype(np.float64)
+        for buf, blk, coef in lst:
+            for c, p in zip(coef, perms):
+                ref = ref + c * X[buf][blk].astype(np.float64).transpose(p)
+        assert abs(out[q] - ref).max() < tol * max(1.0, abs(ref).max()), (q, v)
+
+
 @pytest.mark.parametrize("prec", ["fp64", "bf16x3"])
 def test_residual_chunked_vs_oracle(dev, prec):
     """Residual with the memory-bounded paths of large systems at nocc=10, nvir=9 (220 blocks): ring

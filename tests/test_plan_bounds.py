@@ -109,3 +109,26 @@ def test_residual_plan_in_bounds(monkeypatch, o, v, prec, gbytes):
             assert g.buf.size >= 2 * g.nb * v * (kp if g.kpad is not None else nS), g.name
     if (o, v, gbytes) == (16, 160, 16):
         assert big >= 2 ** 31      # the case where 32-bit offset arithmetic would wrap
+
+
+@pytest.mark.parametrize("o,v,gbytes", [(10, 90, 8 << 30), (10, 90, 2 << 30), (16, 160, 8 << 30), (3, 5, 1), (4, 5, 48000)])
+def test_ring_products_in_bounds(monkeypatch, o, v, gbytes):
+    """The ring products kept in the T2 -> T3 and W_oooo/F_oo scratch, and their placement, stay inside it."""
+    allocs = _fake_device(monkeypatch)
+    from distr_cc.t3_engine import S3PlaceLaunch, TriplesEngine
+    eng = TriplesEngine(o, v, ring_fused=True, ring_g_bytes=gbytes)
+    v3 = v ** 3
+    place = [g for g in eng.launches if isinstance(g, S3PlaceLaunch)]
+    assert len(place) == -(-eng.npairs // eng.ring_pairs)
+    for g in place:
+        job, src = g.jobs._host, g.srcs._host
+        assert (job["dst"] >= 0).all() and (job["dst"] + v3 <= eng.R.size).all()
+        assert (job["first"] + job["count"] <= len(src)).all()
+        assert (src["buf"] >= 0).all() and (src["buf"] < 3).all()
+        for n, b in enumerate(g.bufs):
+            off = src["off"][src["buf"] == n]
+            s, nb = _owner(allocs, b.ptr)
+            assert (off >= 0).all() and b.ptr + 8 * (int(off.max()) + v3) <= s + nb
+    for g in eng.launches:
+        if g.name.startswith("ring W"):
+            _check_gemm(g, allocs, 8)
