@@ -61,6 +61,39 @@ __global__ void oooo_prefactors_kernel(const T *__restrict__ W, const T *__restr
     for (int u = 0; u < 6; ++u) pfs[u * nn + t] = (T)s[u];
 }
 
+// Weights of the W_oooo / F_oo terms over pairs: with the F_oo terms folded in,
+//   W'[l,m,x,y] = W_oooo[l,m,x,y] - 1/2 F_oo[l,x] d_my - 1/2 F_oo[m,y] d_lx
+// (each target has three pairs, so every F_oo term is met twice), out[(l<=m)][(s, x<=y)] is
+//   s = 0: W'[l,m,x,y],  s = 1: W'[m,l,x,y] for l < m, else 0.
+// Pairs count as (0,0), (0,1), .., (0,o-1), (1,1), ...
+template <typename T>
+__global__ void oooo_pairs_kernel(const T *__restrict__ W, const T *__restrict__ F, int no, T *__restrict__ out) {
+    const int np = no * (no + 1) / 2;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 2 * np * np) return;
+    auto pair = [&](int n, int &x, int &y) {
+        x = 0;
+        while (n >= no - x) n -= no - x++;
+        y = x + n;
+    };
+    const int s = t % (2 * np) / np;
+    int l, m, x, y;
+    pair(t / (2 * np), l, m);
+    pair(t % np, x, y);
+    double w = 0.0;
+    if (s == 0 || l < m) {
+        if (s) {
+            const int u = l;
+            l = m;
+            m = u;
+        }
+        w = (double)W[(((int64_t)l * no + m) * no + x) * no + y];
+        if (m == y) w -= 0.5 * (double)F[l * no + x];
+        if (l == x) w -= 0.5 * (double)F[m * no + y];
+    }
+    out[t] = (T)w;
+}
+
 // Weight matrices of the ring terms, all (o*v) x (o*v) with rows (r, x) and
 // columns (l, d):
 //   WR1[r,x,l,d]  = -W_ovov[l,x,r,d]
@@ -99,6 +132,18 @@ int oooo_prefactors(const T *W_oooo, const T *F_oo, int64_t nocc, const int32_t 
 }
 
 template <typename T>
+int oooo_pairs(const T *W_oooo, const T *F_oo, int64_t nocc, T *out, dcc_stream_t stream) {
+    DCC_CHECK(nocc >= 0 && nocc <= 128, "nocc outside 0..128");
+    if (nocc == 0) return 0;
+    DCC_CHECK(W_oooo && F_oo && out, "null pointer");
+    const int64_t np = nocc * (nocc + 1) / 2, total = 2 * np * np;
+    hipLaunchKernelGGL(oooo_pairs_kernel<T>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                       dcc::as_stream(stream), W_oooo, F_oo, (int)nocc, out);
+    DCC_LAUNCH_CHECK();
+    return 0;
+}
+
+template <typename T>
 int ring_weights(const T *W_ovov, const T *W_ovvo, int64_t nocc, int64_t nvir, T *WR1, T *WR3a, T *WR3b,
                  dcc_stream_t stream) {
     DCC_CHECK(nocc >= 0 && nvir >= 0, "negative extent");
@@ -123,6 +168,14 @@ int dcc_oooo_prefactors_f64(const double *W_oooo, const double *F_oo, int64_t no
 int dcc_oooo_prefactors_f32(const float *W_oooo, const float *F_oo, int64_t nocc, const int32_t *blk_ijk,
                             int64_t nblk, float *pfs, dcc_stream_t stream) {
     return oooo_prefactors<float>(W_oooo, F_oo, nocc, blk_ijk, nblk, pfs, stream);
+}
+
+int dcc_oooo_pairs_f64(const double *W_oooo, const double *F_oo, int64_t nocc, double *out, dcc_stream_t stream) {
+    return oooo_pairs<double>(W_oooo, F_oo, nocc, out, stream);
+}
+
+int dcc_oooo_pairs_f32(const float *W_oooo, const float *F_oo, int64_t nocc, float *out, dcc_stream_t stream) {
+    return oooo_pairs<float>(W_oooo, F_oo, nocc, out, stream);
 }
 
 int dcc_ring_weights_f64(const double *W_ovov, const double *W_ovvo, int64_t nocc, int64_t nvir, double *WR1,

@@ -135,6 +135,8 @@ _SIGS = {
     "dcc_ring_weights_f64": ([c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp], ctypes.c_int),
     "dcc_ring_weights_f32": ([c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp], ctypes.c_int),
     "dcc_oooo_prefactors_f32": ([c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp], ctypes.c_int),
+    "dcc_oooo_pairs_f64": ([c_vp, c_vp, c_i64, c_vp, c_vp], ctypes.c_int),
+    "dcc_oooo_pairs_f32": ([c_vp, c_vp, c_i64, c_vp, c_vp], ctypes.c_int),
     "dcc_t3_to_abc_f64": ([c_vp, c_i64, c_i64, c_i64, c_vp, c_vp], ctypes.c_int),
     "dcc_t3_tri_to_abc_packed_f64": ([c_vp, c_i64, c_i64, c_vp, c_vp], ctypes.c_int),
     "dcc_t3_abc_packed_to_dense_f64": ([c_vp, c_i64, c_i64, c_i64, c_vp, c_vp], ctypes.c_int),

@@ -9,11 +9,11 @@ Data in HBM (FP64, C order):
   Gs             (pairs per chunk, o, v, v, v)  ring products of row x = (r,a) before their placement
                                    (with Z three such buffers, two of them views of Xt and Xp)
   Xt             (i per chunk, o, o, v, v, v)   T2->T3 base term X over ordered (i,j,k)
-  pfs            (6, n3, n3)       W_oooo/F_oo prefactors
+  Woo            (npairs, 2, npairs)  W_oooo/F_oo weights over pairs
   W1             (v, v, v, v)      W_vvvv with the F_vv terms folded in
   Wp             (nS + nA, kpad)   pair-symmetric weights from W1 (vvvv_pairs); Tp / Up, the split T3
                                    and the products of a chunk of blocks, are views of Xt / Gs
-  Xp             (5, targets per chunk, v, v, v)  W_oooo/F_oo terms s = 1..5 before their permutation
+  Xp             (5, targets per chunk, v, v, v)  scratch: W_oooo/F_oo products before their permutation
   intermediates  shapes of distr_cc/rccsdt.py:380,445,625
 
 The residual follows distr_cc/rccsdt.py:368-433 term by term, grouped into
@@ -37,9 +37,9 @@ batched gather-GEMMs (dcc_contract_f64):
         G[a,b,c] = G0[a,b,c] + F1[b,a,c] + 1/2 F1[a,b,c] + F2[c,a,b] + 1/2 F2[a,c,b]
     and one placement pass adds the permuted blocks (all three parts of a target at once).  Without Z
     the five terms are accumulated as they stand into one G;
-  * W_oooo/F_oo x T3 (rccsdt.py:616-732): 6 GEMMs M = n3 targets, K = n3 sources,
-    N = v^3, with the prefactors built on the device; term 0 goes straight into R, terms
-    1..5 into Xp per chunk of targets and are added, permuted, by one S3 gather pass.
+  * W_oooo/F_oo x T3 (rccsdt.py:616-732): one GEMM over the pairs l <= m per chunk of spectators,
+    both orders of (l,m) as rows, into Xp, added, permuted, by one S3 gather pass (split BF16x3 with
+    nocc <= 5: over source blocks, with the prefactors built on the device).
 Then dcc_r3_finalize_f64 fuses rccsdt.py:947-971.
 
 T3 -> r1/r2 (rccsdt.py:253-321) and T3 -> W_vooo/W_vvvo (rccsdt.py:323-366)
@@ -528,10 +528,14 @@ class TriplesEngine:
         w3 = (o * v) ** 2 * dt.itemsize
         self.WR3a = DeviceArray((o, v, o, v), dt, ptr=self.WR3.ptr, owner=False)
         self.WR3b = DeviceArray((o, v, o, v), dt, ptr=self.WR3.ptr + w3, owner=False)
-        self.pfs = DeviceArray((6, n3, n3), dt)
-        # W_oooo/F_oo terms s = 1..5 before their permutation, for a chunk of target blocks (the GEMMs'
-        # M); a chunk is rounded up to a multiple of 64 rows when that stays within 5/4 of the bound,
-        # so the GEMM tiles are not partly empty (e.g. 52 -> 64 at nocc=16, nvir=160 in FP64)
+        # W_oooo/F_oo weights over pairs, or prefactors of the source blocks (see _plan_oooo_blocks)
+        self.oooo_blocks = contract == "bf16x3" and self.npairs <= 16
+        if self.oooo_blocks:
+            self.pfs = DeviceArray((6, n3, n3), dt)
+        else:
+            self.Woo = DeviceArray((self.npairs, 2, self.npairs), dt)
+        # scratch of the W_oooo/F_oo products before their permutation, as 5 blocks per target for as many
+        # targets as the bound allows; rounded up to a multiple of 64 targets when that stays within 5/4 of it
         per_target = max(1, 5 * v3 * dt.itemsize)
         qc = ring_g_bytes // per_target
         if qc >= 32 and -(-qc // 64) * 64 * per_target * 4 <= 5 * ring_g_bytes:
@@ -539,7 +543,9 @@ class TriplesEngine:
         qc = int(max(1, min(n3, qc)))
         # pairs per chunk of the ring; with Z, Xp and Xt (plan_t2t3) each also hold one of its products
         self.ring_pairs = int(max(1, min(self.npairs, ring_g_bytes // max(1, o * v3 * dt.itemsize))))
-        self._xp_store = DeviceArray((max(5 * qc, self._ring_blocks()), v, v, v), dt)
+        # (where all targets fit, so do all products over pairs, at most 6/5 of that)
+        xp_blocks = max(5 * qc, self._ring_blocks(), 2 * self.npairs * o if qc == n3 else 0)
+        self._xp_store = DeviceArray((xp_blocks, v, v, v), dt)
         self.Xp = DeviceArray((5, qc, v, v, v), dt, ptr=self._xp_store.ptr, owner=False)
         self.eia = DeviceArray((o, v))
         self._eia_host = None    # what it holds
@@ -600,7 +606,8 @@ class TriplesEngine:
         Y and Z are packed in place (they are rebuilt from T3 for every residual and read by nothing
         else), by writing them as packed words in the first place; the others get packed copies.
         Returns the (source, packed, count) passes to run."""
-        sources = [self.t3, self.Yz, self.W1, self.W_ovvv, self.W_oovo, self.t2, self.WR1, self.WR3, self.pfs]
+        sources = [self.t3, self.Yz, self.W1, self.W_ovvv, self.W_oovo, self.t2, self.WR1, self.WR3,
+                   self.pfs if self.oooo_blocks else self.Woo]
         # the pair-symmetric W_vvvv operands are written as packed words by their own kernels
         in_place = [self.Wp, self.Tp] if self.vvvv_pairs else []
         sources += in_place
@@ -655,10 +662,8 @@ class TriplesEngine:
     def _plan_residual(self):
         o, v, n3 = self.nocc, self.nvir, self.n3
         ext = {x: v for x in 'abcdexyz'}
-        ext.update({'l': o, 'm': o, 'r': o, 'B': n3, 'p': n3, 'q': n3})
-        T = Operand(self.t3, 'Bxyz', (n3, v, v, v))
+        ext.update({'B': n3})
         launches = []
-        blocks = [dict(I=i, J=j, K=k, B=n) for n, (i, j, k) in enumerate(self.triples)]
         # T2 -> T3 (rccsdt.py:388-399)
         Rb = Operand(self.R, 'Babc', (n3, v, v, v))
         launches += self._plan_t2t3()
@@ -675,7 +680,17 @@ class TriplesEngine:
                 B = Operand(self.t3, tl, (n3, v, v, v))
                 launches.append(plan_term('W_vvvv ' + sub, sub, A, B, Rb, 1.0, 1.0, one, ext))
         launches += ring
-        # W_oooo / F_oo (rccsdt.py:726-731).  The abc permutation of each of the six terms commutes
+        launches += self._plan_oooo()
+        return launches
+
+    def _plan_oooo_blocks(self):
+        """W_oooo / F_oo terms (rccsdt.py:726-731) summed over source blocks: for a split-BF16x3 engine of so few
+        pairs (nocc <= 5) that the product over pairs would run on FP32 (K <= 16) and read Y, which is packed."""
+        v, n3 = self.nvir, self.n3
+        ext = {x: v for x in 'abc'}
+        ext.update({'p': n3, 'q': n3})
+        launches = []
+        # The abc permutation of each of the six terms commutes
         # with the sum over source blocks p, so every term is the same natural GEMM
         # X_s[q] = sum_p pfs[s][p][q] T[p] (coalesced in and out) followed, for s > 0, by R[q] +=
         # X_s[q] transposed by the term's permutation (an S3 gather pass).
@@ -705,6 +720,50 @@ class TriplesEngine:
                     srcs[p], coef[p] = ((s - 1) * qc + q - q0) * v3, 1.0
                 jobs.append((q * v3, srcs, coef))
             launches.append(S3GatherLaunch('W_oooo/F_oo add', self.R, self.Xp, v, 1.0, jobs))
+        return launches
+
+    def _plan_oooo(self):
+        if self.oooo_blocks:
+            return self._plan_oooo_blocks()
+        return self._plan_oooo_pairs()
+
+    def _plan_oooo_pairs(self):
+        """W_oooo / F_oo terms (rccsdt.py:616-732) over pairs: P[s,xy;z][c,a,b] = sum_(l<=m) Woo[lm][s,xy]
+        Y[lm][z][c,a,b] for a range of spectators z is one plain GEMM (N = (z,c,a,b), K = the pairs l <= m, Y as
+        the ring reads it), and one gather pass adds, for every target, the two products s of each of its three
+        pairs, whose permutations are the six of the group.  Summed over source blocks instead, six GEMMs of
+        n3 x n3 per element, these terms were 4.8 (nocc=10) to 5.6 (nocc=12) times the flops."""
+        o, v = self.nocc, self.nvir
+        v3, npr = v ** 3, self.npairs
+        blocks = self._xp_store.size // v3
+        zc = max(1, min(o, blocks // (2 * npr), ((1 << 31) - 1) // v3))  # spectators per chunk
+        pc = npr if 2 * npr * zc <= blocks else max(1, blocks // 2)     # and pairs, where one does not fit
+        index = {p: n for n, p in enumerate(self.pairs)}
+        launches = []
+        for z0 in range(0, o, zc):
+            nz = min(zc, o - z0)
+            for p0 in range(0, npr, pc):
+                n = min(pc, npr - p0)
+                am, ak = L.IdxMap(None, 0, 2, n, 0, npr, 1), L.IdxMap(None, 0, 1, npr, 0, 0, 2 * npr)
+                bk, bn = L.IdxMap(None, 0, 1, npr, 0, 0, o * v3), L.IdxMap(None, 0, 1, nz * v3, 0, 0, 1)
+                cm, cn = L.IdxMap(None, 0, 1, 2 * n, 0, 0, nz * v3), L.IdxMap(None, 0, 1, nz * v3, 0, 0, 1)
+                launches.append(GemmLaunch('W_oooo/F_oo pairs', 2 * n, nz * v3, npr, 1.0, 0.0, self.Woo, am, ak,
+                                           self.Y, bk, bn, self._xp_store, cm, cn, [(p0, z0 * v3, 0, 0, 2 * n)], 2 * n,
+                                           2.0 * 2 * n * nz * v3 * npr))
+                jobs = []
+                for q, (i, j, k) in enumerate(self.triples):
+                    srcs, coef = [0] * 6, np.zeros(6)
+                    for pair, z, perms in (((i, j), k, ((1, 2, 0), (2, 1, 0))), ((i, k), j, ((1, 0, 2), (2, 0, 1))),
+                                           ((j, k), i, ((0, 1, 2), (0, 2, 1)))):
+                        row = index[(int(pair[0]), int(pair[1]))] - p0
+                        if not (0 <= row < n and z0 <= z < z0 + nz):
+                            continue
+                        for s, perm in enumerate(perms):
+                            p = TP_T3.index(perm)
+                            srcs[p], coef[p] = ((s * n + row) * nz + int(z) - z0) * v3, 1.0
+                    if coef.any():
+                        jobs.append((q * v3, srcs, coef))
+                launches.append(S3GatherLaunch('W_oooo/F_oo add', self.R, self._xp_store, v, 1.0, jobs))
         return launches
 
     def _pair_scratch(self):
@@ -1029,8 +1088,11 @@ class TriplesEngine:
             L.call(fn, self.W1.vp, v, self.pair_dims[2], self.Wp.vp, s)
         L.call("dcc_ring_weights_" + self.sfx, self.W_ovov.vp, self.W_ovvo.vp, o, v, self.WR1.vp, self.WR3a.vp,
                self.WR3b.vp, s)
-        L.call("dcc_oooo_prefactors_" + self.sfx, self.W_oooo.vp, self.F_oo.vp, o, self.blk_ijk.vp, self.n3,
-               self.pfs.vp, s)
+        if self.oooo_blocks:
+            L.call("dcc_oooo_prefactors_" + self.sfx, self.W_oooo.vp, self.F_oo.vp, o, self.blk_ijk.vp, self.n3,
+                   self.pfs.vp, s)
+        else:
+            L.call("dcc_oooo_pairs_" + self.sfx, self.W_oooo.vp, self.F_oo.vp, o, self.Woo.vp, s)
 
     def _build_z(self, c):
         jobs, njobs = self._lower['chunks'][c][:2]

@@ -291,6 +291,16 @@ int dcc_oooo_prefactors_f32(const float *W_oooo, const float *F_oo, int64_t nocc
                             int64_t nblk, float *pfs, dcc_stream_t stream);
 
 /*
+ * Weights of the same terms over pairs (nocc <= 128): with W'[l,m,x,y] = W_oooo[l,m,x,y]
+ * - 1/2 F_oo[l,x] d_my - 1/2 F_oo[m,y] d_lx and np pairs (0,0), (0,1), .., (1,1), ..,
+ *   out[(l<=m)][s][(x<=y)] = W'[l,m,x,y] for s = 0, W'[m,l,x,y] (0 where l = m) for s = 1,
+ * an np x 2 np matrix.  X_s[xy;z] = sum_(l<=m) out[lm][s][xy] T[z,l,m] then holds every term of target
+ * blocks with pair (x,y) and spectator z: X_0[c,a,b] + X_1[c,b,a] (distr_cc/rccsdt.py:616-732).
+ */
+int dcc_oooo_pairs_f64(const double *W_oooo, const double *F_oo, int64_t nocc, double *out, dcc_stream_t stream);
+int dcc_oooo_pairs_f32(const float *W_oooo, const float *F_oo, int64_t nocc, float *out, dcc_stream_t stream);
+
+/*
  * Ring-term weight matrices ((nocc*nvir) x (nocc*nvir), rows (r,x), cols (l,d)):
  *   WR1 = -W_ovov[l,x,r,d], WR3a = W_ovvo[l,x,d,r],
  *   WR3b = -(W_ovov[l,x,r,d] + W_ovvo[l,x,d,r]) / 2

@@ -637,6 +637,24 @@ class Emulator:
     def dcc_oooo_prefactors_f32(self, *a):
         return self._pfs(np.float32, *a)
 
+    def dcc_oooo_pairs_f64(self, *a):
+        return self._oooo_pairs(np.float64, *a)
+
+    def dcc_oooo_pairs_f32(self, *a):
+        return self._oooo_pairs(np.float32, *a)
+
+    def _oooo_pairs(self, dt, W, F, nocc, out, stream):
+        o = int(nocc)
+        Wd = self.dev.view(_ptr(W), dt, o ** 4).reshape(o, o, o, o).astype(np.float64)
+        Fd = self.dev.view(_ptr(F), dt, o * o).reshape(o, o).astype(np.float64)
+        I = np.eye(o)
+        Wp = Wd - 0.5 * np.einsum('lx,my->lmxy', Fd, I) - 0.5 * np.einsum('my,lx->lmxy', Fd, I)
+        x, y = np.triu_indices(o)
+        A = Wp[x, y][:, x, y]
+        B = Wp[y, x][:, x, y] * (x < y)[:, None]
+        self.dev.view(_ptr(out), dt, 2 * len(x) ** 2)[:] = np.stack([A, B], axis=1).ravel().astype(dt)
+        return 0
+
     def _pfs(self, dt, W, F, nocc, blk_ijk, nblk, pfs, stream):
         o, n3 = int(nocc), int(nblk)
         Wv = self.dev.view(_ptr(W), dt, o ** 4).reshape(o, o, o, o).astype(np.float64)

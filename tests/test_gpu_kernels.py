@@ -163,6 +163,30 @@ def test_s3_gather_multi_source(dev, v, dt, shift):
         assert abs(out[q] - ref).max() < tol * max(1.0, abs(ref).max()), (q, v)
 
 
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("o", [1, 2, 5, 12])
+def test_oooo_pairs(dev, o, dt):
+    """dcc_oooo_pairs_*: the weights of both orders of (l,m) with F_oo folded in, against NumPy; at most three
+    terms each, so a few roundings."""
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    _say("oooo pairs o=%d %s" % (o, dt))
+    rng = np.random.default_rng(o)
+    typ = np.float64 if dt == "f64" else np.float32
+    W, F = rng.normal(size=(o,) * 4).astype(typ), rng.normal(size=(o, o)).astype(typ)
+    dW, dF = DeviceArray.from_host(W), DeviceArray.from_host(F)
+    npr = o * (o + 1) // 2
+    out = DeviceArray((npr, 2, npr), typ)
+    L.call("dcc_oooo_pairs_" + dt, dW.vp, dF.vp, o, out.vp, None)
+    I = np.eye(o)
+    W, F = W.astype(np.float64), F.astype(np.float64)
+    Wp = W - 0.5 * np.einsum('lx,my->lmxy', F, I) - 0.5 * np.einsum('my,lx->lmxy', F, I)
+    x, y = np.triu_indices(o)
+    ref = np.stack([Wp[x, y][:, x, y], Wp[y, x][:, x, y] * (x < y)[:, None]], axis=1)
+    eps = np.finfo(typ).eps
+    assert abs(out.download() - ref).max() <= 4 * eps * abs(ref).max()
+
+
 @pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("dt", ["f64", "f32"])
 @pytest.mark.parametrize("v", [1, 7, 16, 18, 33, 50])
