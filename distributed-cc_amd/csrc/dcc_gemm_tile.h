@@ -193,8 +193,9 @@ __device__ __forceinline__ void contract_tile(const ContractArgs<T> &p, int64_t 
     // STAGES = 2: two register sets hold the tiles k+1 and k+2 while tile k is multiplied out of LDS,
     // so every global load has two K steps of MFMA work (plus the other resident waves) to hide
     // behind; STAGES = 1 keeps one set (fewer registers, more resident waves).
-    // Loads are branch-free: rows/columns outside the operand read its offset 0 (they only feed
-    // outputs that are never stored), and k beyond K reads offset 0 and is replaced by zero.
+    // Rows/columns outside the operand read its offset 0 (they only feed outputs that are never stored); k
+    // beyond K reads offset 0 and is replaced by zero, in a branch of the last K tile only: the select waits
+    // for its load, which then hides behind nothing.
     typedef T T2 __attribute__((ext_vector_type(2)));
     T a_reg[STAGES][SA::NR][SA::NK], b_reg[STAGES][SB::NR][SB::NK];
     // K offsets of this thread's k values, advanced by one K tile after every load (tiles are loaded
@@ -205,7 +206,7 @@ __device__ __forceinline__ void contract_tile(const ContractArgs<T> &p, int64_t 
 #pragma unroll
     for (int j = 0; j < SB::NIT; ++j) b_it[j] = dcc::kiter(p.bk, (uint32_t)SB::kidx(tid, j));
     // one operand: X with row offsets rows[], K map km and iterators it[], into reg[NR][NK]
-    auto load_op = [&](const T *X, const int64_t *rows, const KMap &km, dcc::KIter *it, int k0, bool vfull,
+    auto load_op = [&](const T *X, const int64_t *rows, const KMap &km, dcc::KIter *it, int k0, bool full, bool vfull,
                        auto &reg, auto kfast_tag, auto geom) {
         typedef decltype(geom) G;
         if constexpr (decltype(kfast_tag)::value) {
@@ -234,17 +235,23 @@ __device__ __forceinline__ void contract_tile(const ContractArgs<T> &p, int64_t 
             }
             dcc::kstep(km, it[0]);
         } else {
+            if (vfull) {
 #pragma unroll
-            for (int j = 0; j < G::NK; ++j) {
-                const uint32_t k = (uint32_t)(k0 + G::kidx(tid, j));
-                const bool ok = k < (uint32_t)p.K;
-                const int64_t o = ok ? it[j].off : 0;
-                dcc::kstep(km, it[j]);
-                if (vfull) {
-                    const T2 x = *reinterpret_cast<const T2 *>(X + rows[0] + o);
+                for (int j = 0; j < G::NK; ++j) {
+                    const T2 x = *reinterpret_cast<const T2 *>(X + rows[0] + it[j].off);
                     reg[0][j] = x[0];
                     reg[1][j] = x[1];
-                } else {
+                }
+            } else if (full) {
+#pragma unroll
+                for (int j = 0; j < G::NK; ++j)
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) reg[r][j] = X[rows[r] + it[j].off];
+            } else {
+#pragma unroll
+                for (int j = 0; j < G::NK; ++j) {
+                    const bool ok = (uint32_t)(k0 + G::kidx(tid, j)) < (uint32_t)p.K;
+                    const int64_t o = ok ? it[j].off : 0;
 #pragma unroll
                     for (int r = 0; r < 2; ++r) {
                         const T x = X[rows[r] + o];
@@ -252,12 +259,14 @@ __device__ __forceinline__ void contract_tile(const ContractArgs<T> &p, int64_t 
                     }
                 }
             }
+#pragma unroll
+            for (int j = 0; j < G::NK; ++j) dcc::kstep(km, it[j]);
         }
     };
     auto load_tiles = [&](int s, int k0) {
-        const bool vfull = vec && k0 + kBK <= p.K;   // the last, partial K tile loads per element
-        load_op(p.A, a_row, p.ak, a_it, k0, vfull, a_reg[s], std::integral_constant<bool, A_KFAST>{}, SA{});
-        load_op(p.B, b_col, p.bk, b_it, k0, vfull, b_reg[s], std::integral_constant<bool, !B_NFAST>{}, SB{});
+        const bool full = k0 + kBK <= p.K, vfull = vec && full;   // the last, partial K tile loads per element
+        load_op(p.A, a_row, p.ak, a_it, k0, full, vfull, a_reg[s], std::integral_constant<bool, A_KFAST>{}, SA{});
+        load_op(p.B, b_col, p.bk, b_it, k0, full, vfull, b_reg[s], std::integral_constant<bool, !B_NFAST>{}, SB{});
     };
     auto store_tiles = [&](int s, int buf) {
 #pragma unroll
