@@ -481,6 +481,99 @@ __global__ __launch_bounds__(kOrbitThreads) void s3_place_kernel(T *__restrict__
     else s3_place_orbit<T, false>(lds, out + jb.dst, bufs, nvir, src, jb.count, A, B, C);
 }
 
+// Copy and sum: out[dst0] = src.transpose(p0) and out[dst1] = sum_p c[p] src.transpose(p) in one pass over
+// the source.  A workgroup does a tile orbit of one job as in the placement; the copies are stored as their
+// source tile is staged, the sums stay in registers.  Jobs come in groups of three of one source (empty ones
+// have dst0 < 0) whose workgroups for an orbit are neighbours, so it is read from HBM once for all of them.
+// As two transforms, three tiles read per tile of the sum, the ring operands took 10.6 ms at nocc=12, nvir=120
+// (packed), against 7.0 ms here, where HBM bounds it (15.5 GB); 0.89 against 0.50 ms at nocc=8, nvir=67 in FP32.
+template <typename T, typename O, bool PAIR, bool AB, bool BC>
+__device__ __forceinline__ void s3_copy_sum_orbit(T (*lds)[kLdsTile], O *out, const T *__restrict__ src, int nvir,
+                                                  const dcc_s3_copy_sum_job &jb, int A, int B, int C) {
+    typedef OwnOrbit<PAIR> W;
+    constexpr int NT = AB && BC ? 1 : AB || BC ? 3 : 6;
+    constexpr int AHEAD = NT < 3 ? NT : 3;
+    const W w;
+    auto coords = [&](int s) { return I3{pick3(kPc[s][0], A, B, C), pick3(kPc[s][1], A, B, C), pick3(kPc[s][2], A, B, C)}; };
+    auto store = [&](int64_t dst, int t, const double *x) {
+        O y[W::PER];
+#pragma unroll
+        for (int k = 0; k < W::PER; ++k) {
+            if constexpr (std::is_same<O, T>::value) {
+                y[k] = (T)x[k];
+            } else {
+                float f = (float)x[k];
+                asm("" : "+v"(f));   // rounded to float first: the compiler rounds a double to BF16 in one step
+                y[k] = dcc::pack_bf16x3(f);
+            }
+        }
+        store_rows<O, PAIR>(out + dst, nvir, coords(kTile(AB, BC, t)), w, y);
+    };
+    double acc[NT][W::PER] = {};
+    T v[AHEAD][W::PER];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) load_rows<T, PAIR>(src, nvir, coords(kTile(AB, BC, i)), w, v[i]);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        T *tile = lds[i & 1];
+        stage_rows<T, PAIR>(tile, w, v[i % AHEAD]);
+        __syncthreads();
+        if (i + AHEAD < NT) load_rows<T, PAIR>(src, nvir, coords(kTile(AB, BC, i + AHEAD)), w, v[i % AHEAD]);
+#pragma unroll
+        for (int p = 0; p < 6; ++p) {
+            const double c = jb.coef[p];
+            const bool copy = jb.perm0 == p, sum = (__double_as_longlong(c) << 1) != 0;   // uniform
+            if (!copy && !sum) continue;
+            const int s0 = kPc[p][0] == 0 ? kSX : kPc[p][0] == 1 ? kSY : 1;
+            const int s1 = kPc[p][1] == 0 ? kSX : kPc[p][1] == 1 ? kSY : 1;
+            const int s2 = kPc[p][2] == 0 ? kSX : kPc[p][2] == 1 ? kSY : 1;
+            const T *at = tile + w.x0 * s0 + w.y * s1 + w.z0 * s2;
+            double x[W::PER];
+#pragma unroll
+            for (int k = 0; k < W::PER; ++k) x[k] = (double)at[w.dx(k) * s0 + w.dz(k) * s2];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                if (kRep(AB, BC, kMul(kTile(AB, BC, t), p)) != kTile(AB, BC, i)) continue;
+                if (copy) store(jb.dst0, t, x);
+                if (!sum) continue;   // no zero times an infinity
+#pragma unroll
+                for (int k = 0; k < W::PER; ++k) acc[t][k] += c * x[k];
+            }
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t) store(jb.dst1, t, acc[t]);
+}
+
+template <typename T, typename O, bool PAIR>
+__device__ __forceinline__ void s3_copy_sum_orbit(T (*lds)[kLdsTile], O *out, const T *src, int nvir,
+                                                  const dcc_s3_copy_sum_job &jb, int A, int B, int C) {
+    if (A == B && B == C) s3_copy_sum_orbit<T, O, PAIR, true, true>(lds, out, src, nvir, jb, A, B, C);
+    else if (A == B) s3_copy_sum_orbit<T, O, PAIR, true, false>(lds, out, src, nvir, jb, A, B, C);
+    else if (B == C) s3_copy_sum_orbit<T, O, PAIR, false, true>(lds, out, src, nvir, jb, A, B, C);
+    else s3_copy_sum_orbit<T, O, PAIR, false, false>(lds, out, src, nvir, jb, A, B, C);
+}
+
+template <typename T, typename O, bool PAIR>
+__global__ __launch_bounds__(kOrbitThreads) void s3_copy_sum_kernel(O *__restrict__ out, const T *__restrict__ src,
+                                                                    int nvir,
+                                                                    const dcc_s3_copy_sum_job *__restrict__ jobs,
+                                                                    int nt, int nso) {
+    __shared__ T lds[2][kLdsTile];
+    const int64_t b = dcc_gemm::xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t group = b / (24 * (int64_t)nso);
+    const int r3 = (int)(b - group * 24 * (int64_t)nso), r = r3 / 3;
+    const dcc_s3_copy_sum_job &jb = jobs[3 * group + r3 % 3];
+    if (jb.dst0 < 0) return;
+    int SA, SB, SC;
+    decode_orbit(r / 8, SA, SB, SC);
+    const int A = 2 * SA + ((r >> 2) & 1), B = 2 * SB + ((r >> 1) & 1), C = 2 * SC + (r & 1);
+    if (!(A >= B && B >= C && A < nt)) return;
+    if (PAIR && ((jb.dst0 | jb.dst1 | jb.src) & 1) == 0)
+        s3_copy_sum_orbit<T, O, true>(lds, out, src + jb.src, nvir, jb, A, B, C);
+    else s3_copy_sum_orbit<T, O, false>(lds, out, src + jb.src, nvir, jb, A, B, C);
+}
+
 // The fused projection/update keeps the 8x8x8 tile orbits: one workgroup reads the six tiles of an
 // orbit of R from HBM once and writes the six output tiles.  In the per-output-tile form above the
 // six tiles of an orbit each re-read all six source tiles through L2, one after another, and the
@@ -787,6 +880,25 @@ int s3_place(T *out, const T *src0, const T *src1, const T *src2, int64_t nvir, 
     return 0;
 }
 
+template <typename T, typename O>
+int s3_copy_sum(O *out, const T *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs, int64_t ngroups,
+                dcc_stream_t stream) {
+    DCC_CHECK(nvir >= 0 && ngroups >= 0, "negative extent");
+    if (nvir == 0 || ngroups == 0) return 0;
+    DCC_CHECK(out != nullptr && src != nullptr && jobs != nullptr, "null pointer");
+    const int64_t nt = (nvir + E - 1) / E, nso = n_orbits((nt + 1) / 2);
+    DCC_CHECK(24 * nso * ngroups * kOrbitThreads < ((int64_t)1 << 32), "grid too large");
+    const dim3 grid((unsigned)(24 * nso * ngroups));
+    if (pair_ok(nvir, out, src))
+        hipLaunchKernelGGL((s3_copy_sum_kernel<T, O, true>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream),
+                           out, src, (int)nvir, jobs, (int)nt, (int)nso);
+    else
+        hipLaunchKernelGGL((s3_copy_sum_kernel<T, O, false>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream),
+                           out, src, (int)nvir, jobs, (int)nt, (int)nso);
+    DCC_LAUNCH_CHECK();
+    return 0;
+}
+
 template <typename T, typename O = T>
 int s3_transform(O *out, const T *src, int64_t nvir, double beta, const dcc_s3_job *jobs, int64_t njobs,
                  dcc_stream_t stream) {
@@ -890,6 +1002,21 @@ int dcc_s3_place_f32(float *out, const float *src0, const float *src1, const flo
                      const dcc_s3_place_job *jobs, int64_t njobs, const dcc_s3_place_src *srcs,
                      dcc_stream_t stream) {
     return s3_place<float>(out, src0, src1, src2, nvir, jobs, njobs, srcs, stream);
+}
+
+int dcc_s3_copy_sum_f64(double *out, const double *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs,
+                        int64_t ngroups, dcc_stream_t stream) {
+    return s3_copy_sum<double, double>(out, src, nvir, jobs, ngroups, stream);
+}
+
+int dcc_s3_copy_sum_f32(float *out, const float *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs,
+                        int64_t ngroups, dcc_stream_t stream) {
+    return s3_copy_sum<float, float>(out, src, nvir, jobs, ngroups, stream);
+}
+
+int dcc_s3_copy_sum_pack_f32(uint32_t *out, const float *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs,
+                             int64_t ngroups, dcc_stream_t stream) {
+    return s3_copy_sum<float, uint32_t>(out, src, nvir, jobs, ngroups, stream);
 }
 
 int64_t dcc_r3_finalize_tiles(int64_t nvir) {

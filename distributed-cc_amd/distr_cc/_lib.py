@@ -57,6 +57,8 @@ BATCH_DTYPE = np.dtype([("a_off", np.int64), ("b_off", np.int64), ("c_off", np.i
 S3JOB_DTYPE = np.dtype([("dst", np.int64), ("src", np.int64), ("coef", np.float64, (6,))])
 S3GATHER_DTYPE = np.dtype([("dst", np.int64), ("src", np.int64, (6,)), ("coef", np.float64, (6,))])
 S3PLACE_SRC_DTYPE = np.dtype([("off", np.int64), ("buf", np.int64), ("coef", np.float64, (6,))])
+S3COPYSUM_DTYPE = np.dtype([("dst0", np.int64), ("dst1", np.int64), ("src", np.int64), ("perm0", np.int64),
+                            ("coef", np.float64, (6,))])
 S3PLACE_JOB_DTYPE = np.dtype([("dst", np.int64), ("first", np.int32), ("count", np.int32)])
 # dcc_combine_term, dcc_combine_job, dcc_dot_job
 TERM_DTYPE = np.dtype([("src", np.int64), ("stride", np.int64, (4,)), ("coef", np.float64), ("count", np.int64),
@@ -122,6 +124,9 @@ _SIGS = {
     "dcc_s3_gather_f64": ([c_vp, c_vp, c_i64, c_dbl, c_vp, c_i64, c_vp], ctypes.c_int),
     "dcc_s3_gather_f32": ([c_vp, c_vp, c_i64, c_dbl, c_vp, c_i64, c_vp], ctypes.c_int),
     "dcc_s3_place_f64": ([c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp], ctypes.c_int),
+    "dcc_s3_copy_sum_f64": ([c_vp, c_vp, c_i64, c_vp, c_i64, c_vp], ctypes.c_int),
+    "dcc_s3_copy_sum_f32": ([c_vp, c_vp, c_i64, c_vp, c_i64, c_vp], ctypes.c_int),
+    "dcc_s3_copy_sum_pack_f32": ([c_vp, c_vp, c_i64, c_vp, c_i64, c_vp], ctypes.c_int),
     "dcc_s3_place_f32": ([c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_i64, c_vp, c_vp], ctypes.c_int),
     "dcc_r3_finalize_tiles": ([c_i64], c_i64),
     "dcc_r3_finalize_f64": ([c_vp, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp],

@@ -552,28 +552,25 @@ class TriplesEngine:
         self.norb = int(L._lib.dcc_r3_finalize_tiles(v))
         self.partials = DeviceArray((n3 * self.norb, 2))
         self.norms = DeviceArray((2,))
-        # --- Y materialization jobs: Y[(p,q)][l] = T[l,p,q] ---
-        jobs = []
+        # --- Y[(p,q)][l] = T[l,p,q] and Z[(p,q)][l] = Y - 1/2 (Y.transpose(1,0,2) + Y.transpose(2,1,0)), from T ---
+        jobs = {}   # (Y/Z block, permutation of Y) by source block; up to three each
         for pq, (p, q) in enumerate(self.pairs):
             for l in range(o):
                 case, (ci, cj, ck) = canonical_case(l, p, q)
-                coef = np.zeros(6)
-                coef[case] = 1.0
-                jobs.append(((pq * o + l) * v3, ijk_to_linear(ci, cj, ck, o) * v3, coef))
-        self.y_jobs = DeviceArray.from_host(s3_jobs_array(jobs))
-        self.n_y_jobs = len(jobs)
-        # --- Z jobs: Z[(p,q)][l] = Y - 1/2 (Y.transpose(1,0,2) + Y.transpose(2,1,0)), from T ---
+                jobs.setdefault(ijk_to_linear(ci, cj, ck, o), []).append((pq * o + l, case))
         if self.ring_fused:
-            jobs = []
-            for pq, (p, q) in enumerate(self.pairs):
-                for l in range(o):
-                    case, (ci, cj, ck) = canonical_case(l, p, q)
+            arr = np.zeros((len(jobs), 3), dtype=L.S3COPYSUM_DTYPE)
+            arr['dst0'] = -1
+            for group, (src, lst) in zip(arr, sorted(jobs.items())):
+                for j, (blk, case) in zip(group, lst):
+                    j['dst0'], j['dst1'], j['src'], j['perm0'] = blk * v3, ysize + blk * v3, src * v3, case
                     a = TP_T3[case]
-                    coef = np.zeros(6)
                     for b, x in (((0, 1, 2), 1.0), ((1, 0, 2), -0.5), ((2, 1, 0), -0.5)):
-                        coef[TP_T3.index((a[b[0]], a[b[1]], a[b[2]]))] += x
-                    jobs.append(((pq * o + l) * v3, ijk_to_linear(ci, cj, ck, o) * v3, coef))
-            self.z_jobs = DeviceArray.from_host(s3_jobs_array(jobs))
+                        j['coef'][TP_T3.index((a[b[0]], a[b[1]], a[b[2]]))] += x
+            self.y_jobs, self.n_y_jobs = DeviceArray.from_host(arr.ravel()), len(jobs)
+        else:
+            lst = [(blk * v3, src * v3, np.eye(6)[case]) for src, l in sorted(jobs.items()) for blk, case in l]
+            self.y_jobs, self.n_y_jobs = DeviceArray.from_host(s3_jobs_array(lst)), len(lst)
         # --- pair-symmetric W_vvvv: weights [nS + nA][kpad], split T3 and products for a chunk of blocks
         # (the split T3 and the products of a chunk of blocks live in the T2 -> T3 and ring scratch
         # buffers, idle during the W_vvvv terms: only the weights take memory of their own)
@@ -1203,15 +1200,14 @@ class TriplesEngine:
     def materialize_y(self):
         """Y (and Z) from T3; in the split-BF16x3 engine written directly as packed words."""
         s = self.stream.handle if self.stream is not None else None
-        if self._yz_direct:
-            call = lambda dst, jobs: L.call("dcc_s3_transform_pack_f32", dst.vp, self.t3.vp, self.nvir, jobs.vp,
-                                            self.n_y_jobs, s)
-        else:
-            call = lambda dst, jobs: L.call("dcc_s3_transform_" + self.sfx, dst.vp, self.t3.vp, self.nvir, 0.0,
-                                            jobs.vp, self.n_y_jobs, s)
-        call(self.Y, self.y_jobs)
+        sfx = "pack_f32" if self._yz_direct else self.sfx
         if self.ring_fused:
-            call(self.Z, self.z_jobs)
+            L.call("dcc_s3_copy_sum_" + sfx, self.Yz.vp, self.t3.vp, self.nvir, self.y_jobs.vp, self.n_y_jobs, s)
+        elif self._yz_direct:
+            L.call("dcc_s3_transform_pack_f32", self.Y.vp, self.t3.vp, self.nvir, self.y_jobs.vp, self.n_y_jobs, s)
+        else:
+            L.call("dcc_s3_transform_" + self.sfx, self.Y.vp, self.t3.vp, self.nvir, 0.0, self.y_jobs.vp,
+                   self.n_y_jobs, s)
 
     def residual(self, timer=None):
         """R <- r3 of distr_cc/rccsdt.py:368-433 for the current t3 and intermediates.

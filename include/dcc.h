@@ -239,6 +239,23 @@ int dcc_s3_place_f32(float *out, const float *src0, const float *src1, const flo
                      dcc_stream_t stream);
 
 /*
+ * Copy and sum: for each job, out[dst0] = X.transpose(perm0) and out[dst1] = sum_p coef[p] X.transpose(p), X the
+ * block at src (permutations as in dcc_s3_job, perm0 its index; FP64 sums), reading X once: the ring operands of
+ * a T3 block.  Jobs come in groups of three, best of one source block; dst0 < 0 skips a job.  All dst blocks are
+ * distinct; out and src must not overlap.  _pack_f32 writes split-BF16x3 words of the float results.
+ */
+typedef struct dcc_s3_copy_sum_job {
+    int64_t dst0, dst1, src, perm0;
+    double coef[6];
+} dcc_s3_copy_sum_job;
+int dcc_s3_copy_sum_f64(double *out, const double *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs,
+                        int64_t ngroups, dcc_stream_t stream);
+int dcc_s3_copy_sum_f32(float *out, const float *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs,
+                        int64_t ngroups, dcc_stream_t stream);
+int dcc_s3_copy_sum_pack_f32(uint32_t *out, const float *src, int64_t nvir, const dcc_s3_copy_sum_job *jobs,
+                             int64_t ngroups, dcc_stream_t stream);
+
+/*
  * Fused end of the triples update (distr_cc/rccsdt.py:947-971):
  *   r = (R - (1/6) sum_p R.transpose(p)) / (eia[i,a] + eia[j,b] + eia[k,c])
  *   t3 += r;  optionally r3_out = r;

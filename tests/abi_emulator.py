@@ -530,6 +530,35 @@ class Emulator:
             self.dcc_pack_bf16x3(_ptr(out) + 4 * int(dst), _ptr(out) + 4 * int(dst), v3, stream)
         return 0
 
+    def dcc_s3_copy_sum_f64(self, *a):
+        return self._s3_copy_sum(np.float64, False, *a)
+
+    def dcc_s3_copy_sum_f32(self, *a):
+        return self._s3_copy_sum(np.float32, False, *a)
+
+    def dcc_s3_copy_sum_pack_f32(self, *a):
+        return self._s3_copy_sum(np.float32, True, *a)
+
+    def _s3_copy_sum(self, dt, pack, out, src, nvir, jobs, ngroups, stream):
+        v = int(nvir)
+        v3 = v ** 3
+        O = self.dev.view(_ptr(out), dt)
+        S = self.dev.view(_ptr(src), dt)
+        jdt = np.dtype([("dst0", np.int64), ("dst1", np.int64), ("src", np.int64), ("perm0", np.int64),
+                        ("coef", np.float64, (6,))])
+        jb = self.dev.view(_ptr(jobs), np.uint8, 3 * int(ngroups) * jdt.itemsize).view(jdt)
+        jb = jb[jb["dst0"] >= 0]
+        dst = [int(d) for d in jb["dst0"]] + [int(d) for d in jb["dst1"]]
+        assert len(set(dst)) == len(dst), "S3 jobs of one call share a destination"
+        for j in jb:
+            x = S[int(j["src"]): int(j["src"]) + v3].reshape(v, v, v).astype(np.float64)
+            val = sum(c * x.transpose(p) for c, p in zip(j["coef"], _PERMS) if c != 0.0) + np.zeros((v, v, v))
+            for d, y in ((int(j["dst0"]), x.transpose(_PERMS[int(j["perm0"])])), (int(j["dst1"]), val)):
+                O[d: d + v3] = y.astype(dt).ravel()
+                if pack:
+                    self.dcc_pack_bf16x3(_ptr(out) + 4 * d, _ptr(out) + 4 * d, v3, stream)
+        return 0
+
     def _s3(self, dt, out, src, nvir, beta, jobs, njobs, stream):
         v = int(nvir)
         O = self.dev.view(_ptr(out), dt)

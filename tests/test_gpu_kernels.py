@@ -188,6 +188,50 @@ def test_oooo_pairs(dev, o, dt):
 
 
 @pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("dt", ["f64", "f32", "pack_f32"])
+@pytest.mark.parametrize("v", [1, 7, 16, 18, 33, 50])
+def test_s3_copy_sum(dev, v, dt, shift):
+    """dcc_s3_copy_sum_*: every permutation as the copy (exact), sums of none to six terms, empty jobs; packed
+    words as dcc_pack_bf16x3 of the float results.  ``shift`` = 1 moves every block one element off alignment.
+    Sums are FP64: a rounding of the result (f32) or of each of six terms (f64)."""
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    _say("s3 copy sum v=%d %s shift %d" % (v, dt, shift))
+    rng = np.random.default_rng(70 + v)
+    typ = np.float64 if dt == "f64" else np.float32
+    X = rng.normal(size=(2, v, v, v)).astype(typ)
+    perms = ((0, 1, 2), (0, 2, 1), (1, 0, 2), (1, 2, 0), (2, 0, 1), (2, 1, 0))
+    coefs = [[1, 0, -0.5, 0, 0, -0.5], [0] * 6, [0, 0, 0, 2.0, 0, 0], [1, -1, 0.5, 2, -0.25, 3], [0, 1, 0, 0, -1, 0]]
+    v3 = v ** 3
+    arr = np.zeros(6, dtype=L.S3COPYSUM_DTYPE)
+    arr['dst0'] = -1
+    for n, c in enumerate(coefs):
+        j = arr[n if n < 2 else n + 1]
+        j['dst0'], j['dst1'], j['src'], j['perm0'], j['coef'] = (2 * n * v3 + shift, (2 * n + 1) * v3 + shift,
+                                                                 n % 2 * v3 + shift, (n + 1) % 6, c)
+    pad = np.zeros(shift, typ)
+    dX = DeviceArray.from_host(np.concatenate([pad, X.ravel()]))
+    dO = DeviceArray.zeros((shift + 2 * len(coefs) * v3,), typ)
+    dj = DeviceArray.from_host(arr)
+    L.call("dcc_s3_copy_sum_" + dt, dO.vp, dX.vp, v, dj.vp, 2, None)
+    out = dO.download()
+    assert np.all(out[:shift] == 0)
+    out = out[shift:].reshape(len(coefs), 2, v, v, v)
+    f = DeviceArray.zeros((shift + 2 * len(coefs) * v3,), typ)
+    if dt == "pack_f32":
+        L.call("dcc_s3_copy_sum_f32", f.vp, dX.vp, v, dj.vp, 2, None)
+        L.call("dcc_pack_bf16x3", f.vp, f.vp, f.size, None)
+        assert np.array_equal(dO.download().view(np.uint32), f.download().view(np.uint32))
+        return
+    tol = 1e-13 if dt == "f64" else 1e-6
+    for n, c in enumerate(coefs):
+        x = X[n % 2]
+        assert np.array_equal(out[n, 0], x.transpose(perms[(n + 1) % 6])), n
+        ref = sum(y * x.astype(np.float64).transpose(p) for y, p in zip(c, perms) if y != 0) + np.zeros((v, v, v))
+        assert abs(out[n, 1] - ref).max() <= tol * max(1.0, abs(ref).max()), n
+
+
+@pytest.mark.parametrize("shift", [0, 1])
 @pytest.mark.parametrize("dt", ["f64", "f32"])
 @pytest.mark.parametrize("v", [1, 7, 16, 18, 33, 50])
 def test_s3_place(dev, v, dt, shift):
