@@ -96,7 +96,9 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
     }
 
     typedef T T2 __attribute__((ext_vector_type(2)));
-    // 4 values of every fragment, zero beyond K: at k .. k+3, or with one wave k, k+4, k+8, k+12
+    // 4 values of every fragment: at k .. k+3, or with one wave k, k+4, k+8, k+12.  Beyond K offset 0 is read;
+    // mul zeroes those values (a select here would wait for the load, and the stage ahead would not be ahead:
+    // a cycle at nocc=8, nvir=38 took 4.84 ms that way and takes 4.73 ms)
     constexpr int KS = W == 1 ? 4 : 1;
     auto load = [&](auto &reg, const T *const *ptr, const KMap &km, dcc::KIter &it, uint32_t k, bool vec, bool step,
                     auto nf) {
@@ -109,8 +111,8 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
 #pragma unroll
                 for (int f = 0; f < NF; ++f) {
                     const T2 v = *reinterpret_cast<const T2 *>(ptr[f] + o);
-                    reg[f][h] = ok ? v[0] : T(0);
-                    reg[f][h + 1] = ok ? v[1] : T(0);
+                    reg[f][h] = v[0];
+                    reg[f][h + 1] = v[1];
                 }
             }
         } else {
@@ -119,10 +121,7 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
                 const bool ok = k + KS * s < (uint32_t)p.K;
                 const int64_t o = !ok ? 0 : s == 0 ? it.off : step ? it.off + KS * s * km.s2 : koff(km, k + KS * s);
 #pragma unroll
-                for (int f = 0; f < NF; ++f) {
-                    const T v = ptr[f][o];
-                    reg[f][s] = ok ? v : T(0);
-                }
+                for (int f = 0; f < NF; ++f) reg[f][s] = ptr[f][o];
             }
         }
         dcc::kstep(km, it);
@@ -143,15 +142,28 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
             k += 16 * W;
         }
     };
-    auto mul = [&](int s) {
+    // block 0 of the stage is the wave's block kb of 16 * W k values
+    auto mul = [&](int s, int kb) {
 #pragma unroll
-        for (int b = 0; b < KB; ++b)
+        for (int b = 0; b < KB; ++b) {
+            const uint32_t first = 16u * (uint32_t)(w + W * (kb + b));   // of this block
+            if (first + 16 > (uint32_t)p.K) {   // uniform
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool ok = first + (uint32_t)(W == 1 ? lk + 4 * e : 4 * lk + e) < (uint32_t)p.K;
+#pragma unroll
+                    for (int i = 0; i < FX; ++i) xr[s][b][i][e] = ok ? xr[s][b][i][e] : T(0);
+#pragma unroll
+                    for (int j = 0; j < FY; ++j) yr[s][b][j][e] = ok ? yr[s][b][j][e] : T(0);
+                }
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int i = 0; i < FX; ++i)
 #pragma unroll
                     for (int j = 0; j < FY; ++j) acc[i][j] = MF::step(xr[s][b][i][e], yr[s][b][j][e], acc[i][j]);
+        }
     };
     const int nblk = (p.K + 15) / 16;
     const int mine = nblk > w ? (nblk - w + W - 1) / W : 0;   // blocks of this wave
@@ -159,9 +171,9 @@ __device__ __forceinline__ void skinny_tile(const SkinnyArgs<T> &p, int64_t batc
         stage(0);
         for (int b = 0; b < mine; b += 2 * KB) {
             stage(1);
-            mul(0);
+            mul(0, b);
             stage(0);
-            mul(1);
+            mul(1, b + KB);
         }
     }
     // partial tiles: [wave][fragment][r][lane]

@@ -867,16 +867,21 @@ int s3_place(T *out, const T *src0, const T *src1, const T *src2, int64_t nvir, 
     if (nvir == 0 || njobs == 0) return 0;
     DCC_CHECK(out && src0 && src1 && src2 && jobs && srcs, "null pointer");
     const int64_t nt = (nvir + E - 1) / E, nso = n_orbits((nt + 1) / 2);
-    DCC_CHECK(8 * nso * njobs * kOrbitThreads < ((int64_t)1 << 32), "grid too large");
     const PlaceBufs<T> bufs{{src0, src1, src2}};
-    const dim3 grid((unsigned)(8 * nso * njobs));
-    if (pair_ok(nvir, out, src0) && pair_ok(nvir, src1, src2))
-        hipLaunchKernelGGL((s3_place_kernel<T, true>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream), out, bufs,
-                           (int)nvir, jobs, srcs, (int)nt, (int)nso);
-    else
-        hipLaunchKernelGGL((s3_place_kernel<T, false>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream), out, bufs,
-                           (int)nvir, jobs, srcs, (int)nt, (int)nso);
-    DCC_LAUNCH_CHECK();
+    const bool pair = pair_ok(nvir, out, src0) && pair_ok(nvir, src1, src2);
+    // a grid holds less than 2^32 threads
+    const int64_t most = ((int64_t)1 << 32) / (8 * nso * kOrbitThreads + 1);
+    DCC_CHECK(most > 0, "grid too large");
+    for (int64_t j = 0; j < njobs; j += most) {
+        const dim3 grid((unsigned)(8 * nso * (njobs - j < most ? njobs - j : most)));
+        if (pair)
+            hipLaunchKernelGGL((s3_place_kernel<T, true>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream), out,
+                               bufs, (int)nvir, jobs + j, srcs, (int)nt, (int)nso);
+        else
+            hipLaunchKernelGGL((s3_place_kernel<T, false>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream), out,
+                               bufs, (int)nvir, jobs + j, srcs, (int)nt, (int)nso);
+        DCC_LAUNCH_CHECK();
+    }
     return 0;
 }
 
@@ -887,15 +892,19 @@ int s3_copy_sum(O *out, const T *src, int64_t nvir, const dcc_s3_copy_sum_job *j
     if (nvir == 0 || ngroups == 0) return 0;
     DCC_CHECK(out != nullptr && src != nullptr && jobs != nullptr, "null pointer");
     const int64_t nt = (nvir + E - 1) / E, nso = n_orbits((nt + 1) / 2);
-    DCC_CHECK(24 * nso * ngroups * kOrbitThreads < ((int64_t)1 << 32), "grid too large");
-    const dim3 grid((unsigned)(24 * nso * ngroups));
-    if (pair_ok(nvir, out, src))
-        hipLaunchKernelGGL((s3_copy_sum_kernel<T, O, true>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream),
-                           out, src, (int)nvir, jobs, (int)nt, (int)nso);
-    else
-        hipLaunchKernelGGL((s3_copy_sum_kernel<T, O, false>), grid, dim3(kOrbitThreads), 0, dcc::as_stream(stream),
-                           out, src, (int)nvir, jobs, (int)nt, (int)nso);
-    DCC_LAUNCH_CHECK();
+    const bool pair = pair_ok(nvir, out, src);
+    const int64_t most = ((int64_t)1 << 32) / (24 * nso * kOrbitThreads + 1);   // as s3_place
+    DCC_CHECK(most > 0, "grid too large");
+    for (int64_t g = 0; g < ngroups; g += most) {
+        const dim3 grid((unsigned)(24 * nso * (ngroups - g < most ? ngroups - g : most)));
+        if (pair)
+            hipLaunchKernelGGL((s3_copy_sum_kernel<T, O, true>), grid, dim3(kOrbitThreads), 0,
+                               dcc::as_stream(stream), out, src, (int)nvir, jobs + 3 * g, (int)nt, (int)nso);
+        else
+            hipLaunchKernelGGL((s3_copy_sum_kernel<T, O, false>), grid, dim3(kOrbitThreads), 0,
+                               dcc::as_stream(stream), out, src, (int)nvir, jobs + 3 * g, (int)nt, (int)nso);
+        DCC_LAUNCH_CHECK();
+    }
     return 0;
 }
 
