@@ -472,8 +472,9 @@ inline bool tile_shape_of(int64_t id, int &bm, int &bn, int &stages) {
 // tiles take, times the tile's area over its rate.  Rates are relative to the 64x64 one-stage tile at
 // equal padding and depend on the layouts (which operand is staged K-contiguous), measured on the launches
 // of one residual: FP64 at nocc=10, nvir=90 and nocc=8, nvir=38, FP32 at nocc=8, nvir=67.  The taller tile
-// pays where A is K-contiguous (ring GEMM 28.4 -> 27.5 ms in FP64 although 900 rows pad to 1024, 3.27 ->
-// 2.96 ms in FP32), the wider one where A is row-contiguous (W_oooo 9.1 -> 8.2 ms), 128x128 where both are
+// pays where A is K-contiguous (a ring product over K = 2 o v, 28.4 -> 27.5 ms in FP64 although 900 rows pad
+// to 1024, 3.27 -> 2.96 ms in FP32), the wider one where A is row-contiguous (1100 x 729000 x 220, 9.1 -> 8.2
+// ms), 128x128 where both are
 // K-contiguous and K is long (W_vvvv pairs 22.7 -> 20.6 ms); short K and few rounds stay on 64x64, whose
 // one-stage form keeps four workgroups per CU (T2->T3 at K = 46: 201 -> 154 us against two stages).
 struct TileChoice {
