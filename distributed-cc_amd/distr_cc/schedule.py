@@ -257,7 +257,7 @@ class LowerSchedule:
                           [term(oovv, "jkbc"), term(gv("jkcb"), "jkbc", -0.5)], {})]
             diag.append((Operand.strided(lo["Ecomb"], {"l": o * o * v + o * v, "p": v, "a": 1}), "lpa", [o, o, v],
                          [term(Operand.strided(e.Fd, {"l": 0, "p": n, "a": 1}, o), "lpa", 0.5)], {"beta": 1.0}))
-            build.append(Step(lambda _s, tr=tr: tr._build_z(0)))
+            build.append(Step(lambda _s, tr=tr: self._build_z(tr)))
             _, _, a2, a3 = lo["chunks"][0]
             ein = {g.name.split(" q0")[0]: g for g in a2 + a3 if isinstance(g, GemmLaunch)}
             # the E_ooov term as a partial of its own, after the o slices of the E_vovv term
@@ -287,6 +287,13 @@ class LowerSchedule:
                      (e.r2s, e.r2s, None, e.scal.ptr + 8, e.r2s.size, 0, 0)]
         upload_tables([g for _, g in gemms])
         return ([Combine(operands), Combine(diag)] + build + self._contractions(gemms) + [Combine(final), Dots(dots)])
+
+    @staticmethod
+    def _build_z(tr):
+        """Z of the current T3.  The launches that follow reuse the buffer of the W_vvvo terms, so terms kept there
+        by an earlier t3_to_r1r2 are no longer those of t3_to_w(reuse_z=True)."""
+        tr._lower["dw_valid"] = False
+        tr._build_z(0)
 
     def energies(self):
         """The energy dot products of every engine as one launch (into scal[2:4])."""

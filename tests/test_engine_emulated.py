@@ -504,3 +504,25 @@ def test_lower_schedule_matches_programs(monkeypatch, o, v, shift):
         assert np.allclose(res[0], res[1], rtol=1e-12, atol=1e-15)
         for x, y in zip(engs[0].get_amplitudes(), engs[1].get_amplitudes()):
             assert abs(x - y).max() <= 1e-13 * max(abs(y).max(), 1e-30)
+
+
+def test_schedule_drops_kept_t3_terms(monkeypatch):
+    """t3_to_w(reuse_z=True) after t3_to_r1r2 and then a scheduled iteration computes the T3 terms of W_vooo and
+    W_vvvo from the new T3: the iteration has overwritten what t3_to_r1r2 kept."""
+    abi_emulator.install(monkeypatch)
+    from ccsdt_cases import molecule_like, random_amplitudes
+    from distr_cc.rccsdt_engine import RCCSDTEngine
+    o, v = 3, 4
+    F, g, e, _ = molecule_like(o, v, 7)
+    res = []
+    for schedule in (True, False):
+        eng = RCCSDTEngine(o, v, F, g, e, schedule=schedule)
+        assert (eng.sched is not None) == schedule
+        eng.set_amplitudes(*random_amplitudes(o, v, 6))
+        eng.tr.set_t1_dressed_device(eng.G0, eng.F0, o + v)
+        eng.tr.t3_to_r1r2()
+        eng.update_amps()
+        eng.tr.t3_to_w(reuse_z=True)
+        res.append(eng.tr.get_w_t3_adjusted())
+    for x, y in zip(*res):
+        assert abs(x - y).max() <= 1e-13 * abs(y).max()
