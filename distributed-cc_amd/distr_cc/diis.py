@@ -100,8 +100,15 @@ class DeviceDIIS:
         return np.linalg.solve(h, g)
 
     def extrapolate(self, nd):
-        """The extrapolated vector of the first ``nd`` history vectors (a new DeviceArray)."""
-        return self._combine(nd, self._copy(self._xprev))
+        """The extrapolated vector of the first ``nd`` history vectors (a new DeviceArray); nothing is kept."""
+        c = self.coefficients(nd)[1:]
+        xnew = DeviceArray((self.size,))
+        lay = L.Strided()
+        lay.ndim, lay.shape[0], lay.dst_stride[0], lay.src_stride[0] = 1, self.size, 1, 1
+        for i, ci in enumerate(c):
+            L.call("dcc_tensor_axpby_f64", xnew.vp, self.xs[i].vp, ctypes.byref(lay), float(ci), 0.0 if i == 0 else 1.0,
+                   self._h())
+        return xnew
 
     def _combine(self, nd, xprev):
         """The extrapolated vector, which also replaces ``xprev``; keeps the norm of the change."""

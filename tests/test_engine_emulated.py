@@ -526,3 +526,28 @@ def test_schedule_drops_kept_t3_terms(monkeypatch):
         res.append(eng.tr.get_w_t3_adjusted())
     for x, y in zip(*res):
         assert abs(x - y).max() <= 1e-13 * abs(y).max()
+
+
+def test_diis_extrapolate_keeps_nothing(monkeypatch):
+    """DeviceDIIS.extrapolate only forms the vector: the norm of the last update, the previous iterate and the
+    vector that the next update returns are as without the call."""
+    abi_emulator.install(monkeypatch)
+    from distr_cc.device import DeviceArray
+    from distr_cc.diis import DeviceDIIS
+    from oracle.diis import DIIS
+    n, steps = 9, 5
+    xs = np.random.default_rng(2).standard_normal((steps, n))
+    plain, asked, od = DeviceDIIS(n, space=4), DeviceDIIS(n, space=4), DIIS(space=4)
+    for k, x in enumerate(xs):
+        ref = od.update(x.copy())
+        got = plain.update(DeviceArray.from_host(x)).download()
+        assert np.array_equal(asked.update(DeviceArray.from_host(x)).download(), got)
+        assert np.abs(got - ref).max() <= 1e-9 * np.abs(ref).max()
+        nd = sum(v is not None for v in asked.xs)
+        for m in range(1, nd + 1):
+            y = asked.extrapolate(m).download()
+            c = asked.coefficients(m)[1:]
+            want = sum(ci * v.download() for ci, v in zip(c, asked.xs))
+            assert np.abs(y - want).max() <= 1e-12 * np.abs(c).max() * np.abs(xs).max()
+        assert asked.last_delta_norm_sq == plain.last_delta_norm_sq
+        assert np.array_equal(asked._xprev.download(), plain._xprev.download())
