@@ -113,7 +113,8 @@ def _suffix(dtype):
     return {np.dtype(np.float64): "f64", np.dtype(np.float32): "f32"}[np.dtype(dtype)]
 
 
-# the library's own choice of an FP64/FP32 launch as an autotuner result (its skinny tiles have no tile shape)
+# the library's own choice of an FP64/FP32 launch as an autotuner result (its skinny tiles have no tile shape);
+# of a split-BF16x3 launch 8 is a tile like any other
 LIBRARY_TILE = 8
 
 
@@ -138,7 +139,9 @@ class GemmLaunch:
         self.max_rows = int(max_rows)
         self.flops = float(flops)
         self.keep = keep  # device tables referenced by maps
-        self.tile = -1    # -1, LIBRARY_TILE: library default; 0..7: dcc_contract_tiled_* tile_shape (autotuned)
+        # -1: library default; else the tile_shape of dcc_contract_tiled_* (autotuned): 0..7, LIBRARY_TILE the default
+        # again, or 0..13 for split BF16x3
+        self.tile = -1
 
     def __call__(self, stream):
         self.run(stream)
@@ -153,7 +156,7 @@ class GemmLaunch:
         s = stream.handle if stream is not None else None
         if self.fn == "dcc_contract_packed_bf16x3":
             L.call(self.fn, *self.args, self.batches.vp, self.nbatch, self.max_rows, self.tile, s)
-        elif 0 <= self.tile != LIBRARY_TILE:
+        elif self.tile >= 0 and (self.tile != LIBRARY_TILE or self.fn == "dcc_contract_f32_bf16x3"):
             L.call(self.fn.replace("contract_", "contract_tiled_"), *self.args, self.batches.vp, self.nbatch,
                    self.max_rows, self.tile, s)
         else:

@@ -551,3 +551,29 @@ def test_diis_extrapolate_keeps_nothing(monkeypatch):
             assert np.abs(y - want).max() <= 1e-12 * np.abs(c).max() * np.abs(xs).max()
         assert asked.last_delta_norm_sq == plain.last_delta_norm_sq
         assert np.array_equal(asked._xprev.download(), plain._xprev.download())
+
+
+def test_tile_8_of_split_bf16x3_and_plain_launches(monkeypatch):
+    """Tile 8 is 256x256 with direct-to-LDS staging for a split-BF16x3 launch, packed or not, and the library's own
+    choice for an FP64 or FP32 one."""
+    abi_emulator.install(monkeypatch)
+    from distr_cc import _lib as L
+    from distr_cc.t3_engine import GemmLaunch, TriplesEngine
+    eng = TriplesEngine(3, 6, dtype=np.float32, contract="bf16x3", ring_fused=True)
+    eng._setup_lower()
+    plain = TriplesEngine(3, 6, ring_fused=True)
+    launches = [g for e in (eng, plain) for g in e._tunable() if isinstance(g, GemmLaunch)]
+    seen, calls = set(), []
+    monkeypatch.setattr(L, "call", lambda name, *a: calls.append((name, a)))
+    for g in launches:
+        g.tile = 8
+        del calls[:]
+        g.run(None)
+        name, args = [c for c in calls if c[0].startswith("dcc_contract")][0]
+        seen.add(g.fn)
+        if g.fn.endswith("bf16x3"):
+            assert name == {"dcc_contract_f32_bf16x3": "dcc_contract_tiled_f32_bf16x3"}.get(g.fn, g.fn), g.name
+            assert args[-2] == 8
+        else:
+            assert name == g.fn, g.name
+    assert {"dcc_contract_f32_bf16x3", "dcc_contract_packed_bf16x3", "dcc_contract_f64"} <= seen
