@@ -11,6 +11,8 @@ launch takes the same contraction of every system.  Divisions by the
 denominators, the amplitude update and the T3 terms ride along as further terms of those sums; dot products
 are one launch of many (dcc_dots_f64). 
 """
+import itertools
+
 import numpy as np
 
 from distr_cc import _lib as L
@@ -194,7 +196,8 @@ class LowerSchedule:
 
     def _contractions(self, gemms):
         """Launches of independent contractions [(engine, GemmLaunch)].  One engine: the small ones together,
-        a large one alone.  An ensemble: the n-th of every engine together, which fills the chip already."""
+        a large one alone.  An ensemble: the n-th of every engine that has so many together, which fills the chip
+        already."""
         if len(self.engines) == 1:
             small = [g for _, g in gemms if _small(g)]
             steps = [small[0]] if len(small) == 1 else [self._group(small, True)] if small else []
@@ -202,7 +205,7 @@ class LowerSchedule:
         per = {}
         for k, g in gemms:
             per.setdefault(k, []).append(g)
-        return [self._group(list(gs), False) for gs in zip(*per.values())]
+        return [self._group([g for g in gs if g is not None], False) for gs in itertools.zip_longest(*per.values())]
 
     def _group(self, launches, small):
         ph = _GroupedPhase(launches, small)

@@ -577,3 +577,23 @@ def test_tile_8_of_split_bf16x3_and_plain_launches(monkeypatch):
         else:
             assert name == g.fn, g.name
     assert {"dcc_contract_f32_bf16x3", "dcc_contract_packed_bf16x3", "dcc_contract_f64"} <= seen
+
+
+def test_schedule_groups_unequal_engines(monkeypatch):
+    """An ensemble whose systems have different numbers of contractions in a stage: every one is issued once, in a
+    group with at most one of each system."""
+    abi_emulator.install(monkeypatch)
+    from ccsdt_cases import molecule_like
+    from distr_cc.rccsdt_engine import RCCSDTEngine
+    from distr_cc.schedule import LowerSchedule
+    from distr_cc.t3_engine import GemmLaunch
+    engines = []
+    for o, v in ((2, 3), (1, 2), (2, 4)):
+        F, g, e, _ = molecule_like(o, v, 5)
+        engines.append(RCCSDTEngine(o, v, F, g, e, schedule=False))
+    sched = LowerSchedule(engines, None)
+    gemms = [(k, [s for s in e.prog["dress"].steps if isinstance(s, GemmLaunch)]) for k, e in enumerate(engines)]
+    gemms = [(k, g) for k, gs in gemms for g in gs[:(4, 1, 2)[k]]]
+    groups = [ph.launches for ph in sched._contractions(gemms)]
+    assert sorted(map(len, groups)) == [1, 1, 2, 3]
+    assert sorted(id(g) for gs in groups for g in gs) == sorted(id(g) for _, g in gemms)
