@@ -90,6 +90,15 @@ class Step:
         self.run = fn
 
 
+class NotSchedulable(ValueError):
+    """A program whose operations cannot run stage by stage."""
+
+
+def _need(ok, why):
+    if not ok:
+        raise NotSchedulable("program cannot be scheduled: " + why)
+
+
 def _small(g):
     M, N = g.args[:2]
     return -(-M // 64) * -(-N // 64) * g.nbatch <= SMALL_TILES
@@ -130,30 +139,42 @@ class LowerSchedule:
         Z, partials within MAX_PARTIAL_BYTES, tensors below 2^31 elements."""
         if eng.mixed or len(eng.tr._lower["chunks"]) != 1 or eng.nmo ** 4 >= 1 << 31:
             return False
-        return all(LowerSchedule._targets(eng, n)[1].used * 8 <= MAX_PARTIAL_BYTES for n in ("r1r2", "imds3"))
+        try:
+            return all(LowerSchedule._targets(eng, n)[1].used * 8 <= MAX_PARTIAL_BYTES for n in ("r1r2", "imds3"))
+        except NotSchedulable:
+            return False
 
     # ------------------------------------------------------------------ programs
     @staticmethod
     def _targets(eng, name):
         """The tensors a program accumulates into, in order: {id(buffer): [Operand, letters, level, parts]} with
-        parts ("ein", offset of the partial, op, stage) or ("src", op); and the partials' sizes."""
-        out, part = {}, _Partials()
-        level = lambda op: out[id(op.buf)][2] if id(op.buf) in out else 0
+        parts ("ein", offset of the partial, op, stage) or ("src", op); and the partials' sizes.  A tensor's stage is
+        known when it is read, so every contribution to it must come before."""
+        out, part, read = {}, _Partials(), set()
+
+        def level(op):
+            read.add(id(op.buf))
+            return out[id(op.buf)][2] if id(op.buf) in out else 0
+
         for op in eng.prog[name].ops:
+            _need(op[0] in ("axpby", "ein"), "a step that is no contraction or copy")
+            dst = op[1] if op[0] == "axpby" else op[5]
             if op[0] == "axpby":
-                _, dst, src, letters, alpha, beta = op
-                assert sorted(letters) == sorted(dst.letters)
+                _, _, src, letters, alpha, beta = op
+                _need(sorted(letters) == sorted(dst.letters), "a copy that broadcasts into its target")
                 if beta == 0.0:
-                    assert id(dst.buf) not in out and dst.shape is not None
+                    _need(id(dst.buf) not in out and dst.shape is not None, "a tensor that is set twice")
                     out[id(dst.buf)] = [dst, dst.letters, 0, []]
-                t, at, entry = out[id(dst.buf)], level(src), ("src", op)
-            elif op[0] == "ein":
-                _, _, sub, A, B, C, alpha, beta = op
-                t, at = out[id(C.buf)], max(level(A), level(B))
-                assert C.strides == t[0].strides and C.base == t[0].base and beta == 1.0
-                entry = ("ein", part.size(t[0]), op, at)
+                at, entry = level(src), ("src", op)
             else:
-                raise ValueError("program %s has a step that is no contraction or copy" % name)
+                _, _, sub, A, B, C, alpha, beta = op
+                at = max(level(A), level(B))
+            t = out.get(id(dst.buf))
+            _need(t is not None, "an accumulation into a tensor that is not set first")
+            _need(id(dst.buf) not in read, "a tensor that is read before its last contribution")
+            if op[0] == "ein":
+                _need(C.strides == t[0].strides and C.base == t[0].base and beta == 1.0, "a contraction into a view")
+                entry = ("ein", part.size(t[0]), op, at)
             t[2] = max(t[2], at + 1)
             t[3].append(entry)
         return out, part

@@ -597,3 +597,46 @@ def test_schedule_groups_unequal_engines(monkeypatch):
     groups = [ph.launches for ph in sched._contractions(gemms)]
     assert sorted(map(len, groups)) == [1, 1, 2, 3]
     assert sorted(id(g) for gs in groups for g in gs) == sorted(id(g) for _, g in gemms)
+
+
+def _with_op(monkeypatch, name, add):
+    """Engines whose program ``name`` gets one more operation from add(engine, program)."""
+    from distr_cc.rccsdt_engine import RCCSDTEngine
+    build = RCCSDTEngine._build_program
+
+    def changed(self):
+        steps = build(self)
+        add(self, steps[name])
+        return steps
+
+    monkeypatch.setattr(RCCSDTEngine, "_build_program", changed)
+
+
+@pytest.mark.parametrize("case", ["read before complete", "set after read", "not set"])
+def test_schedule_refuses_order_it_cannot_keep(monkeypatch, case):
+    """A program that reads a tensor before its last contribution, or sets or accumulates out of order, runs one by
+    one (no schedule) and gives what its order says."""
+    abi_emulator.install(monkeypatch)
+    from ccsdt_cases import molecule_like, random_amplitudes
+    from distr_cc.rccsdt_engine import RCCSDTEngine
+    from distr_cc.t3_engine import Operand
+    o, v = 2, 3
+    F, g, e, _ = molecule_like(o, v, 11)
+
+    def add(eng, p):
+        h, W = eng.nview(eng.h_ovvo, "ladi"), eng.nview(eng.imd["W_ovvo"], "ladi")
+        if case == "read before complete":    # W_ovvo has been formed from h by now
+            p.axpby(h, eng.gview(eng.G, "ladi"), "ladi", 0.5, 1.0)
+        elif case == "set after read":        # t2 is read by every contraction before
+            p.axpby(Operand(eng.t2, "ijab", (o, o, v, v)), eng.gview(eng.G, "ijab"), "ijab", 1.0, 0.0)
+        else:                                 # accumulates into the result of another program
+            p.axpby(eng.nview(eng.Foo1, "ki"), eng.gview(eng.Fd, "ki"), "ki", 1.0, 1.0)
+
+    _with_op(monkeypatch, "imds3", add)
+    engs = [RCCSDTEngine(o, v, F, g, e, schedule=s) for s in (True, False)]
+    assert engs[0].sched is None
+    for eng in engs:
+        eng.set_amplitudes(*random_amplitudes(o, v, 6))
+        eng.update_amps()
+    for x, y in zip(engs[0].get_amplitudes(), engs[1].get_amplitudes()):
+        assert np.array_equal(x, y)
