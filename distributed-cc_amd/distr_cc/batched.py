@@ -205,7 +205,8 @@ class BatchedRCCSDT(_Grouped):
         self._group_lower(group_lower)
 
     def _group_lower(self, group):
-        """Operation q of every engine's issue_lower (RCCSDTEngine.lower_ops): when each engine's
+        """The schedule of all systems (LowerSchedule) where it fits; otherwise operation q of every engine's
+        issue_lower (RCCSDTEngine.lower_ops): when each engine's
         operation starts with an FP64 contraction, those contractions run as one grouped persistent
         launch, followed by the rest of every engine's operation (split-K sums, ...).  Operations
         without a contraction run engine by engine.  If the engines' operation lists differ in length
@@ -213,7 +214,7 @@ class BatchedRCCSDT(_Grouped):
         from distr_cc.schedule import LowerSchedule
         self.lower_phases = []
         self.sched = self.energy_dots = None
-        if group and all(LowerSchedule.fits(e) for e in self.engines):
+        if group and LowerSchedule.fits(self.engines):
             # the operations of all systems side by side, stage by stage
             self.sched = LowerSchedule(self.engines, self.stream)
             self.lower_phases = self.sched.grouped

@@ -245,7 +245,7 @@ class RCCSDTEngine:
         self.sched = None
         if schedule:
             from distr_cc.schedule import LowerSchedule
-            if LowerSchedule.fits(self):
+            if LowerSchedule.fits([self]):
                 self.sched = LowerSchedule([self], stream)
                 self._eprog = self.sched.energies()
             else:

@@ -17,7 +17,7 @@ import numpy as np
 
 from distr_cc import _lib as L
 from distr_cc.batched import _GroupedPhase
-from distr_cc.device import DeviceArray
+from distr_cc.device import DeviceArray, mem_get_info
 from distr_cc.t3_engine import GemmLaunch, LIBRARY_TILE, Operand, plan_einsum, upload_tables
 
 # 64x64 tiles below which a contraction does not fill the chip and joins its stage's grouped launch
@@ -134,15 +134,23 @@ class LowerSchedule:
                        "update12": self._plan_update(), "imds3": self._plan_program("imds3", targets["imds3"])}
 
     @staticmethod
-    def fits(eng):
-        """Whether the engine's lower-order part is worth and able to run this way: FP64 triples, one chunk of
-        Z, partials within MAX_PARTIAL_BYTES, tensors below 2^31 elements."""
-        if eng.mixed or len(eng.tr._lower["chunks"]) != 1 or eng.nmo ** 4 >= 1 << 31:
-            return False
-        try:
-            return all(LowerSchedule._targets(eng, n)[1].used * 8 <= MAX_PARTIAL_BYTES for n in ("r1r2", "imds3"))
-        except NotSchedulable:
-            return False
+    def fits(engines):
+        """Whether the lower-order part of every engine is worth and able to run this way: FP64 triples, one chunk
+        of Z, partials within MAX_PARTIAL_BYTES, tensors below 2^31 elements; and whether the partials of all of
+        them leave as much of the device's free memory as they take (the one-by-one programs need next to none, so
+        an ensemble that fills the device runs on those)."""
+        total = 0
+        for e in engines:
+            if e.mixed or len(e.tr._lower["chunks"]) != 1 or e.nmo ** 4 >= 1 << 31:
+                return False
+            try:
+                used = 8 * max(LowerSchedule._targets(e, n)[1].used for n in ("r1r2", "imds3"))
+            except NotSchedulable:
+                return False
+            if used > MAX_PARTIAL_BYTES:
+                return False
+            total += used + 8 * (e.nocc * e.nvir) ** 2    # and the E_ooov partial of _plan_update
+        return 2 * total <= mem_get_info()[0]
 
     # ------------------------------------------------------------------ programs
     @staticmethod

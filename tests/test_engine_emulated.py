@@ -640,3 +640,47 @@ def test_schedule_refuses_order_it_cannot_keep(monkeypatch, case):
         eng.update_amps()
     for x, y in zip(engs[0].get_amplitudes(), engs[1].get_amplitudes()):
         assert np.array_equal(x, y)
+
+
+def test_ensemble_schedule_leaves_room(monkeypatch):
+    """The partial results of an ensemble's schedule are allocated only where they leave as much free memory as they
+    take, over all systems; without room the ensemble and a single engine run operation by operation, to the same
+    result."""
+    emu = abi_emulator.install(monkeypatch)
+    from ccsdt_cases import molecule_like, random_amplitudes
+    from distr_cc.batched import BatchedRCCSDT
+    from distr_cc.device import Stream
+    from distr_cc.rccsdt_engine import RCCSDTEngine
+    from distr_cc.schedule import LowerSchedule
+    st = Stream.__new__(Stream)
+    st.handle, st._own = None, False
+    monkeypatch.setattr(Stream, "synchronize", lambda self: None)
+    systems = []
+    for o, v in ((2, 4), (3, 4), (2, 3)):
+        F, g, e, _ = molecule_like(o, v, 21)
+        systems.append((o, v, F, g, e))
+
+    free = [288 << 30]
+
+    def info(pfree, ptotal):
+        pfree._obj.value, ptotal._obj.value = free[0], 288 << 30
+        return 0
+
+    monkeypatch.setattr(emu, "dcc_mem_get_info", info)
+    one = RCCSDTEngine(*systems[0])
+    used = [8 * (max(LowerSchedule._targets(e, n)[1].used for n in ("r1r2", "imds3")) + (e.nocc * e.nvir) ** 2)
+            for e in (RCCSDTEngine(*s, schedule=False) for s in systems)]
+    res = []
+    # room for all; for each of them but not for all; for none
+    for free[0], all_fit, one_fits in ((2 * sum(used), True, True), (2 * sum(used) - 1, False, True), (0, False, False)):
+        bt = BatchedRCCSDT(systems, st)
+        assert (bt.sched is not None) == all_fit
+        for k, (o, v, *_) in enumerate(systems):
+            bt.set_amplitudes(k, *random_amplitudes(o, v, 6 + k))
+        bt.issue_step()
+        res.append([bt.energies()] + [x for e in bt.engines for x in e.get_amplitudes()])
+        one = RCCSDTEngine(*systems[1])
+        assert (one.sched is not None) == one_fits
+    for other in res[1:]:
+        for x, y in zip(res[0], other):
+            assert np.allclose(x, y, rtol=1e-12, atol=1e-15)
