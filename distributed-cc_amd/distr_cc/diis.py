@@ -31,7 +31,9 @@ class _Iterate(DeviceArray):
         diis = self._diis()
         if self.ptr and diis is not None and diis._spare is None:
             L.call("dcc_device_synchronize")
-            diis._spare, self.ptr = self.ptr, 0
+            # another iterate may have been freed during the wait (by a thread, or by the garbage collector): its
+            # memory is in this one's hands then
+            self.ptr, diis._spare = diis._spare or 0, self.ptr
         super().free()
 
 

@@ -684,3 +684,35 @@ def test_ensemble_schedule_leaves_room(monkeypatch):
     for other in res[1:]:
         for x, y in zip(res[0], other):
             assert np.allclose(x, y, rtol=1e-12, atol=1e-15)
+
+
+@pytest.mark.parametrize("nested", [1, 3])
+def test_diis_iterates_freed_during_a_wait(monkeypatch, nested):
+    """Iterates freed while another one waits for the device in its free(): each piece of memory is either kept as
+    the one spare vector or released, once, and nothing is left when the DIIS goes."""
+    emu = abi_emulator.install(monkeypatch)
+    from distr_cc.device import DeviceArray
+    from distr_cc.diis import DeviceDIIS
+    n = 33
+    dd = DeviceDIIS(n, space=3)
+    rng = np.random.default_rng(1)
+    its = [dd.update(DeviceArray.from_host(rng.standard_normal(n))) for _ in range(nested + 2)][1:]
+    ptrs = [y.ptr for y in its]
+    assert len(set(ptrs)) == nested + 1
+    freed, waiting = [], its[1:]
+    monkeypatch.setattr(emu, "dcc_free", lambda p: freed.append(p.value if p.value in ptrs else None) or 0)
+
+    def wait():
+        if waiting:
+            waiting.pop().free()
+        return 0
+
+    monkeypatch.setattr(emu, "dcc_device_synchronize", wait, raising=False)
+    its[0].free()
+    assert not waiting
+    assert sorted([p for p in freed if p] + [dd._spare]) == sorted(ptrs)
+    for y in its:
+        assert y.ptr == 0
+        y.free()
+    y = dd.update(DeviceArray.from_host(rng.standard_normal(n)))
+    assert y.ptr in ptrs and dd._spare is None   # the spare is used again
