@@ -600,6 +600,30 @@ int contract_skinny(const ContractArgs<T> &g, const dcc_idxmap &ak, const dcc_id
     });
 }
 
+// Tile of a launch without one: a skinny variant (kSkinnyBase + variant) where skinny_variant gives one, the
+// shape of TileChoice elsewhere -- except for FP64 products of a short K added into C.  Those are bound by
+// reading and writing C, whose rows come in runs of nocc to a few hundred elements, so what counts is workgroups
+// in flight to hide that, not the area of a tile: the one-stage 64x64 tile keeps four on a CU.  Where C is
+// contiguous along neither index the two-stage tile is the better one.  Measured on the z4 and t4 contractions
+// of (Q) at nocc = 10..15 (K = nocc or nvir up to 25, 874 launches): 570 ms in all, 668 ms with the shapes of
+// TileChoice, 608 ms with 64x64 two-stage; launches of this kind in the iteration and the adjoint (K to 40)
+// change by less than 1 %.
+template <typename T>
+int default_tile(int64_t max_rows, int64_t N, int64_t K, int64_t nbatch, double beta, const dcc_idxmap &cm,
+                 const dcc_idxmap &cn, bool a_kfast, bool b_nfast) {
+    constexpr int64_t kShortK = 40;
+    constexpr bool f64 = std::is_same<T, double>::value;
+    SkinnySize z;
+    if (inner_stride(cn) != 1) z.add(N, max_rows, K, nbatch);
+    else z.add(max_rows, N, K, nbatch);
+    const int v = skinny_variant(z);
+    if (v >= 0) return kSkinnyBase + v;
+    if (f64 && beta != 0.0 && K <= kShortK) return inner_stride(cm) == 1 || inner_stride(cn) == 1 ? 4 : 0;
+    TileChoice tc;
+    tc.add(max_rows, N, K, nbatch);
+    return tc.pick(f64, a_kfast, b_nfast);
+}
+
 template <typename T>
 int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, const T *A, dcc_idxmap am,
                    dcc_idxmap ak, const T *B, dcc_idxmap bk, dcc_idxmap bn, T *C, dcc_idxmap cm, dcc_idxmap cn,
@@ -643,8 +667,7 @@ int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, c
     hipStream_t s = dcc::as_stream(stream);
     // Workgroup tile: tile_shape 0..3 = 64x64, 128x64, 64x128, 128x128 with the two-stage register
     // prefetch, 4..7 = the same shapes with one stage; -1 = DCC_CONTRACT_TILE (e.g. "128x64" or
-    // "64x64s1") when set, otherwise a skinny variant where skinny_variant gives one and the shape of
-    // TileChoice elsewhere.
+    // "64x64s1") when set, otherwise default_tile's.
     static const char *tile_env = getenv("DCC_CONTRACT_TILE");
     int tbm = 64, tbn = 64, stages = 2;
     if (tile_shape >= 0) {
@@ -658,14 +681,10 @@ int contract_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, c
         }
         stages = st == 1 ? 1 : 2;
     } else {
-        SkinnySize z;
-        if (c_mfast) z.add(N, max_rows, K, nbatch);
-        else z.add(max_rows, N, K, nbatch);
-        const int v = skinny_variant(z);
-        if (v >= 0) return contract_skinny<T>(args, ak, bk, c_mfast, nbatch, max_rows, v, s);
-        TileChoice tc;
-        tc.add(max_rows, N, K, nbatch);
-        tile_shape_of(tc.pick(std::is_same<T, double>::value, a_kfast, b_nfast), tbm, tbn, stages);
+        const int id = default_tile<T>(max_rows, N, K, nbatch, beta, cm, cn, a_kfast, b_nfast);
+        if (id >= kSkinnyBase)
+            return contract_skinny<T>(args, ak, bk, c_mfast, nbatch, max_rows, id - kSkinnyBase, s);
+        tile_shape_of(id, tbm, tbn, stages);
     }
     if (tbm == 128 && tbn == 128) return launch<T, 128, 128>(args, max_rows, a_kfast, b_nfast, c_mfast, stages, s);
     if (tbm == 128 && tbn == 64) return launch<T, 128, 64>(args, max_rows, a_kfast, b_nfast, c_mfast, stages, s);
@@ -825,6 +844,24 @@ int contract_bf16x3_entry(int64_t M, int64_t N, int64_t K, double alpha, double 
 }
 
 }  // namespace
+
+extern "C" int64_t dcc_contract_default_tile(int32_t kind, int64_t N, int64_t K, double beta, const void *A,
+                                             dcc_idxmap am, dcc_idxmap ak, const void *B, dcc_idxmap bk,
+                                             dcc_idxmap bn, dcc_idxmap cm, dcc_idxmap cn, int64_t nbatch,
+                                             int64_t max_rows) {
+    const bool a_kfast = inner_stride(ak) == 1 || inner_stride(am) != 1;
+    const bool b_nfast = inner_stride(bn) == 1 || inner_stride(bk) != 1;
+    switch (kind) {
+        case 0: return default_tile<double>(max_rows, N, K, nbatch, beta, cm, cn, a_kfast, b_nfast);
+        case 1: return default_tile<float>(max_rows, N, K, nbatch, beta, cm, cn, a_kfast, b_nfast);
+        case 2: return pick_bf16x3(max_rows, N, K, nbatch, false);
+        case 3:
+            return pick_bf16x3(max_rows, N, K, nbatch,
+                               vectors_contiguous(A, am, ak, a_kfast, 0, 4, 16) &&
+                                   vectors_contiguous(B, bn, bk, !b_nfast, N, 4, 16));
+    }
+    return -1;
+}
 
 extern "C" int dcc_contract_f32_bf16x3(int64_t M, int64_t N, int64_t K, double alpha, double beta,
                                        const float *A, dcc_idxmap am, dcc_idxmap ak, const float *B,

@@ -216,6 +216,8 @@ inline int skinny_flags(const void *X, const dcc_idxmap &xm, const dcc_idxmap &x
            (k_pairs(Y, ym, yk, K, esize) ? kSkinnyPairY : 0);
 }
 
+constexpr int64_t kSkinnyBase = 64;   // numbers of tiles: shapes below, skinny variants from here
+
 // The variants: fragments of X and Y per tile and waves that split K.
 struct SkinnyVariant {
     int fx, fy, w;

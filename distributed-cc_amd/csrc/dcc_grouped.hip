@@ -19,8 +19,7 @@ namespace {
 
 using namespace dcc_gemm;
 
-constexpr int64_t kSkinnyBase = 64;   // launch variants below: tile shape | flags << 3; from here: skinny ones
-
+// variant of a launch: below kSkinnyBase tile shape | flags << 3, from there a skinny one.
 // flags of a prepared problem: bits 0..2 the loader/epilogue choice of the launch (A K-contiguous,
 // B N-contiguous, C written along m; the same for every problem of a launch), bits 3..4 the pair
 // vector loads allowed for A and B of this problem under that choice.

@@ -102,6 +102,8 @@ _SIGS = {
                                 c_vp, IdxMap, IdxMap, c_vp, c_i64, c_i64, c_i64, c_vp], ctypes.c_int),
     "dcc_contract_f32_bf16x3": ([c_i64, c_i64, c_i64, c_dbl, c_dbl, c_vp, IdxMap, IdxMap, c_vp, IdxMap, IdxMap,
                                  c_vp, IdxMap, IdxMap, c_vp, c_i64, c_i64, c_vp], ctypes.c_int),
+    "dcc_contract_default_tile": ([ctypes.c_int32, c_i64, c_i64, c_dbl, c_vp, IdxMap, IdxMap, c_vp, IdxMap, IdxMap, IdxMap,
+                                   IdxMap, c_i64, c_i64], c_i64),
     "dcc_pack_bf16x3": ([c_vp, c_vp, c_i64, c_vp], ctypes.c_int),
     "dcc_t2t3_operands_f64": ([c_vp] * 5 + [c_i64] * 4 + [c_vp], ctypes.c_int),
     "dcc_t2t3_operands_f32": ([c_vp] * 5 + [c_i64] * 4 + [c_vp], ctypes.c_int),

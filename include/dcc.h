@@ -164,6 +164,14 @@ int dcc_contract_tiled_f32_bf16x3(int64_t M, int64_t N, int64_t K, double alpha,
                                   float *C, dcc_idxmap cm, dcc_idxmap cn, const dcc_batch *batches, int64_t nbatch,
                                   int64_t max_rows, int64_t tile_shape, dcc_stream_t stream);
 
+/* Host side: the tile that a contraction without one runs on (dcc_contract_f64 for kind 0, _f32 for 1,
+ * _f32_bf16x3 for 2, _packed_bf16x3 with tile_shape -1 for 3): a tile_shape of its _tiled form, or 64 and above one
+ * of the tiles for few or narrow outputs; -1 for another kind.  Arguments as there; nothing is launched, and A
+ * and B are looked at for their alignment only.  No reference counterpart. */
+int64_t dcc_contract_default_tile(int32_t kind, int64_t N, int64_t K, double beta, const void *A, dcc_idxmap am,
+                                  dcc_idxmap ak, const void *B, dcc_idxmap bk, dcc_idxmap bn, dcc_idxmap cm,
+                                  dcc_idxmap cn, int64_t nbatch, int64_t max_rows);
+
 /* ---------------------------------------- S3 block transforms (HBM-bound) */
 
 /*
