@@ -745,22 +745,58 @@ int run_bf16x3(ContractArgs<float> &args, int64_t nbatch, int64_t max_rows, bool
     return 0;
 }
 
-// Tile shape of a split-BF16x3 launch without one: rounds of resident workgroups times area over rate, as
-// TileChoice.  Rates relative to 128x128 at equal padding, from the launches of one residual at nocc=12,
-// nvir=120 and nocc=9, nvir=71: 256x256 gains most where operands load as 16-byte vectors or K is long
-// (W_vvvv pairs 28.5 -> 22.4 ms, ring 31.1 -> 27.5 ms) and little on short, unaligned K (K = 639: 1.95 ms
-// against 2.19 with the padding of 639 rows); 256x128 suits one side of at most 128 (t3 -> W_vvvo 642 ->
-// 534 us).
-int pick_bf16x3(int64_t rows, int64_t N, int64_t K, int64_t nbatch, bool quads) {
+// How the operands of a split-BF16x3 launch are loaded, as far as it decides the tile: unpacked ones (split by every
+// tile that reads them) or packed ones in quads (16 bytes), pairs (8) or single words.
+enum class Bf16x3Loads { kUnpackedPairs, kUnpacked, kQuads, kQuadsDma, kPairs, kSingle };
+
+// Tile shape of a split-BF16x3 launch without one: per candidate the rounds of resident workgroups its tiles take,
+// times the area of a round over the tile's rate.  Up to 16 rounds they are counted whole, with a last round of at
+// most one workgroup per CU as 0.65 of one for the tiles of which two fit (alone on its CU a workgroup runs faster
+// than half of two); beyond, as a fraction.  Rates are relative to 128x128 at equal padding and depend on how
+// operands load: the register-staged 256x256 tile gains most where every element is a load of its own (nvir odd: a
+// tile of four times the area has half the loads per product; W_vvvv at nocc=11, nvir=107: 31.1 ms against 47.7),
+// but with pairs 128x128 keeps its loads in flight and is the faster one (nvir even but no multiple of four:
+// nocc=11, nvir=50: 0.80 ms against 1.12); with quads 256x256 is ahead again (nocc=9, nvir=104: 5.0 against 6.4 ms).
+// A K of up to 128 against at most 256 rows or columns is bound by the long operand, which a tile across the whole
+// short side reads once (nocc=12, nvir=35, 156 x 514500 x 78: 216 us against 328).
+// Fitted to 2173 launches of 156 engines (nocc 2..12, nvir 10..120), each timed on every tile: in all 1443 ms on the
+// best tiles, 1451 with this rule, 1742 on 128x128 with 64 for a short side; 11 launches are more than 3 % slower
+// than on the latter, by 14 % at most.
+int pick_bf16x3(int64_t rows, int64_t N, int64_t K, int64_t nbatch, Bf16x3Loads loads) {
     static const int shapes[7][4] = {{0, 64, 64, 512},     {1, 128, 64, 512},  {2, 64, 128, 512}, {3, 128, 128, 512},
                                      {9, 256, 128, 256}, {10, 128, 256, 256}, {8, 256, 256, 256}};
-    const double rate[7] = {0.73, 0.8, 0.8, 1.0, 1.08, 1.03, quads || K >= 1024 ? 1.25 : 1.15};
+    // 64x64, 128x64, 64x128, 128x128, 256x128, 128x256, 256x256; 0: not a candidate
+    static const double unpacked[7] = {0.7, 0.79, 0.8, 1.0, 1.1, 0.0, 0.0};
+    static const double unpacked_pairs[7] = {0.7, 0.74, 0.8, 1.0, 0.0, 0.0, 0.0};
+    static const double quads[7] = {0.72, 0.0, 0.75, 1.0, 0.0, 0.0, 1.19};
+    static const double quads_dma[7] = {0.75, 0.0, 0.89, 1.0, 0.0, 0.0, 1.09};
+    static const double quads_short[7] = {0.68, 0.0, 0.76, 1.0, 0.0, 0.0, 0.0};
+    static const double stream[7] = {0.72, 0.0, 0.76, 1.0, 1.12, 1.06, 1.5};
+    static const double pairs[7] = {0.72, 0.74, 0.0, 1.0, 0.0, 0.0, 0.0};
+    static const double single_short[7] = {0.83, 0.0, 0.6, 1.0, 0.0, 0.0, 1.08};
+    static const double single[7] = {0.7, 0.0, 0.72, 1.0, 1.12, 1.03, 1.33};
+    static const double single_long[7] = {0.65, 0.0, 0.57, 1.0, 1.05, 0.95, 1.23};
+    const bool streams = K <= 128 && (rows < N ? rows : N) <= 256;
+    const double *rate = nullptr;
+    switch (loads) {
+        case Bf16x3Loads::kUnpackedPairs: rate = unpacked_pairs; break;
+        case Bf16x3Loads::kUnpacked: rate = unpacked; break;
+        case Bf16x3Loads::kQuads: rate = K <= 64 ? quads_short : quads; break;
+        case Bf16x3Loads::kQuadsDma: rate = K <= 64 ? quads_short : quads_dma; break;
+        case Bf16x3Loads::kPairs: rate = streams ? stream : pairs; break;
+        case Bf16x3Loads::kSingle:
+            rate = streams ? stream : K <= 128 ? single_short : K < 1500 ? single : single_long;
+            break;
+    }
     int best = 3;
     double least = 0.0;
     for (int c = 0; c < 7; ++c) {
+        if (rate[c] == 0.0) continue;
         const int64_t bm = shapes[c][1], bn = shapes[c][2], slots = shapes[c][3];
         const int64_t tiles = nbatch * ((rows + bm - 1) / bm) * ((N + bn - 1) / bn);
-        const double rounds = tiles < slots ? 1.0 : (double)tiles / (double)slots;
+        const int64_t full = tiles / slots, rem = tiles % slots;
+        double rounds = (double)tiles / (double)slots;
+        if (full < 16) rounds = (double)full + (rem == 0 ? 0.0 : slots == 512 && rem <= 256 ? 0.65 : 1.0);
         const double cost = rounds * (double)(slots * bm * bn) / rate[c];
         if (least == 0.0 || cost < least) {
             least = cost;
@@ -768,6 +804,13 @@ int pick_bf16x3(int64_t rows, int64_t N, int64_t K, int64_t nbatch, bool quads) 
         }
     }
     return best;
+}
+
+// The load class of a launch whose A and B both load in quads, or in pairs (of words; never quads if unpacked).
+Bf16x3Loads bf16x3_loads(bool packed, bool quads, bool pairs, bool a_kfast, bool b_nfast, int64_t K) {
+    if (!packed) return pairs ? Bf16x3Loads::kUnpackedPairs : Bf16x3Loads::kUnpacked;
+    if (quads) return a_kfast && !b_nfast && K % 64 == 0 ? Bf16x3Loads::kQuadsDma : Bf16x3Loads::kQuads;
+    return pairs ? Bf16x3Loads::kPairs : Bf16x3Loads::kSingle;
 }
 
 int contract_bf16x3_entry(int64_t M, int64_t N, int64_t K, double alpha, double beta, const float *A,
@@ -815,7 +858,9 @@ int contract_bf16x3_entry(int64_t M, int64_t N, int64_t K, double alpha, double 
     if (!c_mfast && vectors_contiguous(C, cm, cn, true, 0, 4, 16)) args.vec |= 4;
     hipStream_t s = dcc::as_stream(stream);
     int shape = (int)tile_shape;
-    if (shape < 0) shape = pick_bf16x3(max_rows, N, K, nbatch, mode == 2);
+    if (shape < 0)
+        shape = pick_bf16x3(max_rows, N, K, nbatch,
+                            bf16x3_loads(packed, quads, (args.vec & 3) == 3, a_kfast, b_nfast, K));
     // shapes 8..13: direct-to-LDS staging, for packed quads with both operands K-contiguous and K a
     // multiple of 32 x stages; otherwise the register-staged kernel of the same tile
     const int stages = (shape == 9 || shape == 10) ? 3 : 2;
@@ -854,11 +899,13 @@ extern "C" int64_t dcc_contract_default_tile(int32_t kind, int64_t N, int64_t K,
     switch (kind) {
         case 0: return default_tile<double>(max_rows, N, K, nbatch, beta, cm, cn, a_kfast, b_nfast);
         case 1: return default_tile<float>(max_rows, N, K, nbatch, beta, cm, cn, a_kfast, b_nfast);
-        case 2: return pick_bf16x3(max_rows, N, K, nbatch, false);
-        case 3:
-            return pick_bf16x3(max_rows, N, K, nbatch,
-                               vectors_contiguous(A, am, ak, a_kfast, 0, 4, 16) &&
-                                   vectors_contiguous(B, bn, bk, !b_nfast, N, 4, 16));
+        case 2:
+        case 3: {
+            const bool quads = kind == 3 && vectors_contiguous(A, am, ak, a_kfast, 0, 4, 16) &&
+                               vectors_contiguous(B, bn, bk, !b_nfast, N, 4, 16);
+            const bool pairs = pairs_contiguous(A, am, ak, a_kfast, 0, 8) && pairs_contiguous(B, bn, bk, !b_nfast, N, 8);
+            return pick_bf16x3(max_rows, N, K, nbatch, bf16x3_loads(kind == 3, quads, pairs, a_kfast, b_nfast, K));
+        }
     }
     return -1;
 }

@@ -157,7 +157,7 @@ int dcc_contract_packed_bf16x3(int64_t M, int64_t N, int64_t K, double alpha, do
  * accumulators) on 16x16x32 and 32x32x16, with operands staged by direct global -> LDS requests (two, three,
  * three, two, two and two stages) when both packed operands are K-contiguous in 16-byte quads and K is a
  * positive multiple of 32 x stages (otherwise the register-staged tile 6, 4, 5, 7, 6 or 7 runs); -1 picks
- * 128 on each side unless that side has at most 64 rows.
+ * one for the sizes and for how the operands load (dcc_contract_default_tile).
  * No reference counterpart (as dcc_contract_f32_bf16x3). */
 int dcc_contract_tiled_f32_bf16x3(int64_t M, int64_t N, int64_t K, double alpha, double beta, const float *A,
                                   dcc_idxmap am, dcc_idxmap ak, const float *B, dcc_idxmap bk, dcc_idxmap bn,

@@ -44,3 +44,40 @@ def test_few_outputs_stay_on_the_skinny_tiles():
     for kind in (0, 1):
         assert _tile(kind, 64, 64, 8, 1.0, am, ak, bk, bn, _map((64, 64)), _map((64, 1)), 1) >= 64
     assert _tile(9, 64, 64, 8, 1.0, am, ak, bk, bn, _map((64, 64)), _map((64, 1)), 1) == -1
+
+
+# split-BF16x3 launches by how their operands load: rows, N, K, batches, inner extent of B's K, best tiles (times in
+# us; the rule by areas alone took 8 or 9 for each of them but the last two)
+BF16X3 = [
+    # packed pairs, nvir = 50: 128x128 against 256x256, 804: 1123 and 842: 1398
+    ("pairs", 2500, 14300, 2500, 1, 2500, (3,)),
+    ("pairs", 2500, 14300, 2500, 1, 50, (3,)),
+    # ring at nocc=10, nvir=90: 3402: 4572
+    ("pairs", 900, 8100, 900, 55, 90, (3,)),
+    # packed pairs of a short K against 156 rows: one pass over the long operand, 216: 328
+    ("pairs", 156, 514500, 78, 1, 78, (8,)),
+    # packed quads, 360 tiles of 256x256: 150: 218
+    ("quads", 820, 11440, 832, 2, 832, (3,)),
+    ("quads", 5460, 17160, 5504, 2, 5504, (8,)),
+    # single words, nvir = 107: 31114: 47667; 1080 x 1080 x 102 over 1080 batches: 4607..4735
+    ("single", 11449, 30602, 11449, 1, 11449, (8,)),
+    ("single", 472, 472, 67, 472, 67, (3, 8)),
+    # operands split in the tile: t3 -> W_vvvo at nocc=9, nvir=73: 671: 827, nocc=6, nvir=88: 231: 326
+    ("unpacked", 47961, 73, 5913, 1, 73, (3, 9)),
+    ("unpacked pairs", 46464, 88, 3168, 1, 88, (3,)),
+    ("unpacked", 1440, 1, 14400, 144, 14400, (1,)),
+]
+
+
+@pytest.mark.parametrize("loads,rows,N,K,nbatch,ke,best", BF16X3)
+def test_split_bf16x3(loads, rows, N, K, nbatch, ke, best):
+    packed = not loads.startswith("unpacked")
+    step = {"quads": 4, "pairs": 2, "unpacked pairs": 2}.get(loads, 1)
+    assert K % step == 0 and N % step == 0
+    pad = (8, 6, 5)[(step == 2) + 2 * (step == 1)]     # the row stride decides what an aligned vector can hold
+    stride = -(-max(K, N) // 8) * 8 + pad
+    am, ak = _map((rows, stride)), _map((K, 1))
+    # B contiguous along K in runs of ke
+    bk = _map((K // ke, stride * N), (ke, 1)) if ke < K else _map((K, 1))
+    bn = _map((N, stride))
+    assert _tile(3 if packed else 2, rows, N, K, 0.0, am, ak, bk, bn, _map((rows, N)), _map((N, 1)), nbatch) in best
