@@ -14,10 +14,12 @@ Up to nocc = 9 one kernel (dcc_q_quads_f64) forms the z4_p and t4 of every
 the denominator, P4_444, the factor and both dot products (rccsdt_q.py:1131-1153),
 writing per-workgroup partials that are summed in a fixed order into one pair per
 chunk; the host reads the pairs once at the end.  For nocc > 9 (or ``finalize_ws``)
-the o^4 blocks do not fit LDS: each of the 24 z4_p and 24 t4 einsums of a task is one
+the o^4 blocks do not fit LDS, and for nocc <= 2 with many virtuals a kernel per
+quadruple does too little: there each of the 24 z4_p and 24 t4 einsums of a task is one
 batched gather-GEMM over a chunk of tasks into
   z4, t4   (ntask_chunk, bs, bs, bs, bs, o, o, o, o)
-and the finalize kernel keeps its intermediate in a workspace of the size of t4.
+and the finalize kernel keeps its intermediate in LDS, or for nocc > 9 in a workspace
+of the size of t4.
 """
 import numpy as np
 
@@ -99,7 +101,7 @@ class QEngine:
             raise ValueError("blksize must be positive")
         self.vp = -(-self.v // self.bs) * self.bs
         self.stream = stream
-        o, vp, bs = self.o, self.vp, self.bs
+        o, v, vp, bs = self.o, self.v, self.vp, self.bs
         per_task = bs ** 4 * o ** 4 * 8
         self.chunk = max(1, min(int(max_chunk_bytes // per_task), 4096))
         # a chunk of fused quadruples: one workgroup each, partials of two doubles
@@ -109,10 +111,20 @@ class QEngine:
         if w_mode not in ("dense", "task"):
             raise ValueError("w_mode must be 'dense' or 'task'")
         self.w_mode = w_mode
-        # z4 and t4 of a quadruple fit LDS up to nocc = 9; beyond, GEMMs and a finalize with a workspace
+        # z4 and t4 of a quadruple fit LDS up to nocc = 9; beyond, GEMMs and a finalize with a workspace (below, the
+        # finalize keeps its intermediate in LDS too, where GEMMs are used)
         self.finalize_ws = (o > 9) if finalize_ws is None else bool(finalize_ws)
         if o > 9 and not self.finalize_ws:
             raise ValueError("nocc > 9 needs the workspace form of the (Q) finalize")
+        # One workgroup per quadruple costs 60 to 100 ns of the chip however few occupied orbitals there are (some
+        # fifty barrier intervals), the batched GEMMs a time of their own per chunk and then less per quadruple for
+        # nocc <= 2: with blocks of three and more they are the faster ones from these nvir on (nocc=1, nvir=30,
+        # blksize 4: 1.75 ms against 3.00; nocc=2, nvir=48: 17.4 against 24.2; below, nocc=1, nvir=18: 0.88 against
+        # 0.67).  Blocks of one and two give GEMMs of a tile's corner (nocc=1, nvir=30, blksize 1: 20.5 against 2.3 ms),
+        # and from nocc = 3 the kernel is ahead (nocc=3, nvir=44: 17.2 ms; 20.8 ms with GEMMs on 64x64 tiles).
+        # (A block of seven and more has many quadruples without weight, and starts earlier.)
+        gemms_from = {1: (26, 24, 24), 2: (54, 34, 28)}.get(o, (v + 1,) * 3)[(bs > 3) + (bs > 6)] if bs > 2 else v + 1
+        self.fused = not self.finalize_ws and v < gemms_from
         self.dev = None
         self.wplans = None
         self.task_plans = {}
@@ -176,12 +188,14 @@ class QEngine:
         ext.update({'e': vp, 'f': vp})
         ext.update({x: o for x in 'ijklmn'})
         # chunks bound z4/t4 and the W_vvvvoo slots; with neither only the partials
-        size = self.quad_chunk if not self.finalize_ws and self.w_mode == "dense" else self.chunk
+        fused = self.fused
+        size = self.quad_chunk if fused and self.w_mode == "dense" else self.chunk
         nmax = min(size, len(tasks))
-        fused = not self.finalize_ws
         z4 = t4 = ws = None
         if not fused:
-            z4, t4, ws = (DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o)) for _ in range(3))
+            z4, t4 = (DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o)) for _ in range(2))
+        if self.finalize_ws:
+            ws = DeviceArray((nmax, bs, bs, bs, bs, o, o, o, o))
         part = DeviceArray((nmax * bs ** 4, 2))
         nchunk = -(-len(tasks) // size)
         tot = DeviceArray((max(nchunk, 1), 2))
@@ -269,14 +283,15 @@ class QEngine:
             for g in launches:
                 g.run(st)
             nwg = nt * bs ** 4
-            if ws is None:
+            if self.fused:
                 Wv = Ws if slots is not None else dev['Wv']
                 L.call("dcc_q_quads_f64", dev['T'].vp, dev['vvvo'].vp, dev['vooo'].vp, dev['vvoo'].vp, dev['t2'].vp,
                        Wv.vp, dev['Wo'].vp, slots.vp if slots is not None else None, tk.vp, nt, bs, o, v, vp,
                        dev['e_occ'].vp, dev['e_vir'].vp, part.vp, self._s())
             else:
                 L.call("dcc_q_finalize_f64", t4.vp, z4.vp, tk.vp, nt, bs, o, v, vp, dev['e_occ'].vp,
-                       dev['e_vir'].vp, dev['vvoo'].vp, dev['t2'].vp, ws.vp, part.vp, self._s())
+                       dev['e_vir'].vp, dev['vvoo'].vp, dev['t2'].vp, ws.vp if ws is not None else None, part.vp,
+                       self._s())
             L.call("dcc_reduce_pairs_f64", part.vp, nwg, tot.offset_ptr(2 * ci), self._s())
         pairs = tot.download(stream=st).reshape(-1, 2)[:len(chunks)]
         paren = bracket = 0.0

@@ -716,3 +716,40 @@ def test_diis_iterates_freed_during_a_wait(monkeypatch, nested):
         y.free()
     y = dd.update(DeviceArray.from_host(rng.standard_normal(n)))
     assert y.ptr in ptrs and dd._spare is None   # the spare is used again
+
+
+@pytest.mark.parametrize("o,v,bs,fused", [(1, 18, 4, True), (1, 23, 4, True), (1, 24, 4, False), (1, 25, 3, True),
+                                          (1, 26, 3, False), (1, 60, 2, True), (2, 33, 4, True), (2, 34, 6, False), (2, 30, 8, False),
+                                          (2, 48, 3, True), (2, 60, 3, False), (2, 60, 1, True), (3, 60, 4, True),
+                                          (9, 30, 4, True)])
+def test_q_form_by_sizes(monkeypatch, o, v, bs, fused):
+    """Which form of (Q) runs: the fused quadruples except for nocc <= 2 with many virtuals (both sides of the rule
+    were timed at these sizes)."""
+    abi_emulator.install(monkeypatch)
+    from distr_cc.q_engine import QEngine
+    assert QEngine(o, v, blksize=bs).fused == fused
+    assert not QEngine(o, v, blksize=bs, finalize_ws=True).fused
+
+
+@pytest.mark.parametrize("w_mode", ["dense", "task"])
+@pytest.mark.parametrize("o,v,bs", [(1, 5, 4), (2, 5, 3)])
+def test_q_engine_gemms_below_nocc_10(monkeypatch, o, v, bs, w_mode):
+    """The batched GEMMs with the finalize that needs no workspace == the fused quadruples == the oracle."""
+    emu = abi_emulator.install(monkeypatch)
+    from distr_cc.device import DeviceArray
+    from distr_cc.q_engine import QEngine
+    from distr_cc.synthetic import SyntheticSystem
+    from oracle import q_energy as Q
+    from oracle import t3_layout as TL
+    s = SyntheticSystem(o, v, naux=30, seed=500 + o * v, sigma_t3=1e-3)
+    pppp, t2, t3 = s.pppp(), s.t2(), s.t3_tri()
+    ref = Q.kernel(o, v, pppp, t2, TL.full_t3_from_tri(t3, o), s.mo_energy, blksize=bs)
+    for fused in (True, False):
+        eng = QEngine(o, v, blksize=bs, w_mode=w_mode)
+        assert eng.fused
+        eng.fused = fused
+        for _ in range(2):
+            got = eng.kernel(pppp, t2, DeviceArray.from_host(t3), s.mo_energy)
+            for x, y in zip(got, ref):
+                assert abs(x - y) <= 1e-12 * abs(y)
+    assert "dcc_q_quads_f64" in emu.calls and "dcc_q_finalize_f64" in emu.calls

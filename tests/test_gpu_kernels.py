@@ -987,3 +987,26 @@ def test_combine_and_dots(dev, shape):
     if rank2:
         y = ref + np.einsum("ia,jb->ijab", e, e)
         assert abs(got[1] - (a * y).sum()) <= 1e-13 * np.abs(a * y).sum()
+
+
+@pytest.mark.parametrize("o,v,bs,w_mode", [(1, 26, 4, "dense"), (1, 27, 3, "task"), (2, 35, 5, "dense"),
+                                           (2, 7, 4, "task"), (4, 5, 2, "dense"), (9, 5, 2, "task")])
+def test_q_gemms_with_lds_finalize_vs_oracle(dev, o, v, bs, w_mode):
+    """(Q) as batched GEMMs and the finalize without a workspace (both o^4 blocks in LDS, up to nocc = 9): the form
+    that nocc <= 2 with many virtuals takes by itself, elsewhere asked for.  Bound as test_q_energy_vs_oracle."""
+    from distr_cc.device import DeviceArray
+    from distr_cc.q_engine import QEngine
+    from distr_cc.synthetic import SyntheticSystem
+    from oracle import q_energy as Q
+    from oracle import t3_layout as TL
+    _say("(Q) GEMMs, LDS finalize o=%d v=%d blksize=%d %s" % (o, v, bs, w_mode))
+    s = SyntheticSystem(o, v, naux=30, seed=800 + o * v, sigma_t3=1e-3)
+    pppp, t2, t3 = s.pppp(), s.t2(), s.t3_tri()
+    ref = Q.kernel(o, v, pppp, t2, TL.full_t3_from_tri(t3, o), s.mo_energy, blksize=bs)
+    eng = QEngine(o, v, blksize=bs, w_mode=w_mode)
+    assert eng.fused == (v < 20)
+    eng.fused = False
+    for _ in range(2):
+        got = eng.kernel(pppp, t2, DeviceArray.from_host(t3), s.mo_energy)
+        for g, r in zip(got, ref):
+            assert abs(g - r) <= 1e-12 * abs(r)
