@@ -1,5 +1,6 @@
 """Device buffers, streams and events on top of libdcc (no torch)."""
 import ctypes
+import math
 
 import numpy as np
 
@@ -87,7 +88,7 @@ class DeviceArray:
     def __init__(self, shape, dtype=np.float64, ptr=None, owner=True):
         self.shape = tuple(int(s) for s in (shape if isinstance(shape, (tuple, list)) else (shape,)))
         self.dtype = np.dtype(dtype)
-        self.size = int(np.prod(self.shape)) if self.shape else 1
+        self.size = math.prod(self.shape)
         self.nbytes = self.size * self.dtype.itemsize
         if ptr is None:
             p = ctypes.c_void_p()

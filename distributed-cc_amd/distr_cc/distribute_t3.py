@@ -65,6 +65,16 @@ def canonical_case(i, j, k):
     return 5, tuple(s)
 
 
+def canonical_cases(i, j, k, nocc):
+    """canonical_case of arrays of triples (broadcast against each other): case numbers and linear indices of the
+    canonical triples."""
+    i, j, k = np.broadcast_arrays(i, j, k)
+    case = np.select([(i <= j) & (j <= k), (i <= k) & (k < j), (j < i) & (i <= k), (k < i) & (i <= j),
+                      (j <= k) & (k < i)], range(5), 5)
+    s = np.sort(np.stack([i, j, k]).astype(np.int64), axis=0)
+    return case, ijk_to_linear(s[0], s[1], s[2], nocc)
+
+
 def nocc3(nocc):
     return nocc * (nocc + 1) * (nocc + 2) // 6
 

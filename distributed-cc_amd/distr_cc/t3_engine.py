@@ -53,12 +53,25 @@ built by one S3 transform, with all ordered (p,q,r) covered exactly once:
 (E_* are slices of the T1-dressed <pq|rs>; r1 uses P3_422 = 2 P3_201 - (P3_201)^{acb}.)
 """
 import ctypes
+import math
 
 import numpy as np
 
 from distr_cc import _lib as L
 from distr_cc.device import DeviceArray, init as device_init
-from distr_cc.distribute_t3 import TP_T3, canonical_case, canonical_triples, ijk_to_linear, nocc3
+from distr_cc.distribute_t3 import TP_T3, canonical_cases, canonical_triples, ijk_to_linear, nocc3
+
+
+# _COMPOSED[p][q]: index of the permutation (P[q0], P[q1], P[q2]) with P = TP_T3[p], q = TP_T3[q]
+_COMPOSED = [[TP_T3.index(tuple(p[n] for n in q)) for q in TP_T3] for p in TP_T3]
+
+
+def _combination(case, terms):
+    """The six coefficients of sum_q terms[q] X.transpose(q) with X = Y.transpose(TP_T3[case]), in terms of Y."""
+    coef = np.zeros(6)
+    for q, c in terms.items():
+        coef[_COMPOSED[case][TP_T3.index(q)]] += c
+    return coef
 
 
 def c_strides(shape):
@@ -194,12 +207,12 @@ def _group_map(groups, ext, op):
     """dcc_idxmap of up to three fused groups (outermost first) into operand ``op``."""
     if not groups:
         return L.IdxMap(None, 0, 1, 1, 0, 0, 0), 1
-    exts = [int(np.prod([ext[x] for x in g])) for g in groups]
+    exts = [math.prod(ext[x] for x in g) for g in groups]
     strides = [op.strides[g[-1]] for g in groups]
     while len(exts) < 3:
         exts.insert(0, 1)
         strides.insert(0, 0)
-    return L.IdxMap(None, 0, exts[1], exts[2], strides[0], strides[1], strides[2]), int(np.prod(exts))
+    return L.IdxMap(None, 0, exts[1], exts[2], strides[0], strides[1], strides[2]), math.prod(exts)
 
 
 def plan_einsum(name, sub, A, B, C, alpha, beta, ext, batches, max_levels=3):
@@ -288,18 +301,14 @@ class S3Launch:
 
 
 class S3GatherLaunch:
-    """One dcc_s3_gather call: out[dst] = beta*out[dst] + sum_p coef[p] src[src_p]^{TP_T3[p]} per job."""
+    """One dcc_s3_gather call: out[dst] = beta*out[dst] + sum_p coef[p] src[src_p]^{TP_T3[p]} per job (``jobs`` an
+    array of L.S3GATHER_DTYPE)."""
 
     def __init__(self, name, out, src, nvir, beta, jobs):
         self.name, self.flops = name, 0.0
         self.fn = "dcc_s3_gather_" + _suffix(out.dtype)
         self.out, self.src, self.nvir, self.beta = out, src, int(nvir), float(beta)
-        arr = np.zeros(len(jobs), dtype=L.S3GATHER_DTYPE)
-        for n, (dst, srcs, coef) in enumerate(jobs):
-            arr[n]['dst'] = dst
-            arr[n]['src'] = srcs
-            arr[n]['coef'] = coef
-        self.jobs = DeviceArray.from_host(arr)
+        self.jobs = DeviceArray.from_host(jobs)
         self.njobs = len(jobs)
 
     def run(self, stream):
@@ -397,7 +406,7 @@ def plan_t2t3(o, v, R, t2, W_ovvv, W_oovo, scratch_bytes, packed=False, min_bloc
     ext = {'j': o, 'a': v, 'K': K2, 'k': o, 'c': v}
     # source-position permutations of (i,j,k); the abc permutation of the S3 job is its inverse
     pis = [(0, 1, 2), (0, 2, 1), (1, 0, 2), (1, 2, 0), (2, 0, 1), (2, 1, 0)]
-    triples = canonical_triples(o)
+    triples = np.asarray(canonical_triples(o), dtype=np.int64)   # the offsets pass 2^31 for large chunks
     launches = []
     for i0 in range(0, o, ic):
         n = min(ic, o - i0)
@@ -411,18 +420,15 @@ def plan_t2t3(o, v, R, t2, W_ovvv, W_oovo, scratch_bytes, packed=False, min_bloc
             g.fn = "dcc_contract_packed_bf16x3"
         launches.append(g)
         # one gather pass: target q takes sum_pi X[pi(ijk)]^{pi^-1} over the sources in this chunk
-        jobs = []
-        for q, t in enumerate(triples):
-            t = tuple(int(x) for x in t)   # Python integers: the offsets pass 2^31 for large chunks
-            srcs, coef = [0] * 6, np.zeros(6)
-            for pos in pis:
-                src = (t[pos[0]], t[pos[1]], t[pos[2]])
-                if i0 <= src[0] < i0 + n:
-                    p = TP_T3.index(tuple(pos.index(u) for u in range(3)))
-                    srcs[p] = (((src[0] - i0) * o + src[1]) * o + src[2]) * v3
-                    coef[p] = 1.0
-            if coef.any():
-                jobs.append((q * v3, srcs, coef))
+        jobs = np.zeros(len(triples), dtype=L.S3GATHER_DTYPE)
+        jobs['dst'] = np.arange(len(triples)) * v3
+        for pos in pis:
+            src = triples[:, pos]
+            here = (src[:, 0] >= i0) & (src[:, 0] < i0 + n)
+            p = TP_T3.index(tuple(pos.index(u) for u in range(3)))
+            jobs['src'][here, p] = ((((src[:, 0] - i0) * o + src[:, 1]) * o + src[:, 2]) * v3)[here]
+            jobs['coef'][here, p] = 1.0
+        jobs = jobs[jobs['coef'].any(axis=1)]
         launches.append(S3GatherLaunch('T2T3: symmetrise', R, Xt, v, 1.0, jobs))
     return Xt, launches
 
@@ -437,24 +443,14 @@ def s3_jobs_array(jobs):
 
 
 class S3PlaceLaunch:
-    """One dcc_s3_place call: out[dst] += sum of src.transpose(TP_T3[p]) * coef[p] over a job's sources
-    (buffer index, offset, {permutation: coefficient})."""
+    """One dcc_s3_place call: out[dst] += sum over a job's sources of sum_p coef[p] src.transpose(TP_T3[p]) (``jobs``
+    and ``srcs`` arrays of L.S3PLACE_JOB_DTYPE and L.S3PLACE_SRC_DTYPE)."""
 
-    def __init__(self, name, out, bufs, nvir, jobs):
+    def __init__(self, name, out, bufs, nvir, jobs, srcs):
         self.name, self.flops = name, 0.0
         self.fn = "dcc_s3_place_" + _suffix(out.dtype)
         self.out, self.bufs, self.nvir, self.njobs = out, tuple(bufs), int(nvir), len(jobs)
-        job = np.zeros(len(jobs), dtype=L.S3PLACE_JOB_DTYPE)
-        src = np.zeros(sum(len(lst) for _, lst in jobs), dtype=L.S3PLACE_SRC_DTYPE)
-        n = 0
-        for j, (dst, lst) in zip(job, jobs):
-            j['dst'], j['first'], j['count'] = dst, n, len(lst)
-            for buf, off, coef in lst:
-                src[n]['buf'], src[n]['off'] = buf, off
-                for p, c in coef.items():
-                    src[n]['coef'][TP_T3.index(p)] += c
-                n += 1
-        self.jobs, self.srcs = DeviceArray.from_host(job), DeviceArray.from_host(src)
+        self.jobs, self.srcs = DeviceArray.from_host(jobs), DeviceArray.from_host(srcs)
 
     def run(self, stream):
         L.call(self.fn, self.out.vp, *(b.vp for b in self.bufs), self.nvir, self.jobs.vp, self.njobs, self.srcs.vp,
@@ -556,24 +552,25 @@ class TriplesEngine:
         self.partials = DeviceArray((n3 * self.norb, 2))
         self.norms = DeviceArray((2,))
         # --- Y[(p,q)][l] = T[l,p,q] and Z[(p,q)][l] = Y - 1/2 (Y.transpose(1,0,2) + Y.transpose(2,1,0)), from T ---
-        jobs = {}   # (Y/Z block, permutation of Y) by source block; up to three each
-        for pq, (p, q) in enumerate(self.pairs):
-            for l in range(o):
-                case, (ci, cj, ck) = canonical_case(l, p, q)
-                jobs.setdefault(ijk_to_linear(ci, cj, ck, o), []).append((pq * o + l, case))
+        # by source block, up to three (Y/Z block, permutation of Y) each
+        pq = np.array(self.pairs, dtype=np.int64).reshape(-1, 2)
+        case, src = canonical_cases(np.arange(o), pq[:, :1], pq[:, 1:], o)
+        order = np.argsort(src, axis=None, kind='stable')
+        case, src, blk = case.ravel()[order], src.ravel()[order], order
         if self.ring_fused:
-            arr = np.zeros((len(jobs), 3), dtype=L.S3COPYSUM_DTYPE)
+            first = np.searchsorted(src, src)                  # every canonical block is a source
+            arr = np.zeros((n3, 3), dtype=L.S3COPYSUM_DTYPE)
             arr['dst0'] = -1
-            for group, (src, lst) in zip(arr, sorted(jobs.items())):
-                for j, (blk, case) in zip(group, lst):
-                    j['dst0'], j['dst1'], j['src'], j['perm0'] = blk * v3, ysize + blk * v3, src * v3, case
-                    a = TP_T3[case]
-                    for b, x in (((0, 1, 2), 1.0), ((1, 0, 2), -0.5), ((2, 1, 0), -0.5)):
-                        j['coef'][TP_T3.index((a[b[0]], a[b[1]], a[b[2]]))] += x
-            self.y_jobs, self.n_y_jobs = DeviceArray.from_host(arr.ravel()), len(jobs)
+            job = np.zeros(len(blk), dtype=L.S3COPYSUM_DTYPE)
+            job['dst0'], job['dst1'], job['src'], job['perm0'] = blk * v3, ysize + blk * v3, src * v3, case
+            job['coef'] = np.array([_combination(c, {(0, 1, 2): 1.0, (1, 0, 2): -0.5, (2, 1, 0): -0.5})
+                                    for c in range(6)])[case]
+            arr[src, np.arange(len(blk)) - first] = job
+            self.y_jobs, self.n_y_jobs = DeviceArray.from_host(arr.ravel()), n3
         else:
-            lst = [(blk * v3, src * v3, np.eye(6)[case]) for src, l in sorted(jobs.items()) for blk, case in l]
-            self.y_jobs, self.n_y_jobs = DeviceArray.from_host(s3_jobs_array(lst)), len(lst)
+            arr = np.zeros(len(blk), dtype=L.S3JOB_DTYPE)
+            arr['dst'], arr['src'], arr['coef'] = blk * v3, src * v3, np.eye(6)[case]
+            self.y_jobs, self.n_y_jobs = DeviceArray.from_host(arr), len(arr)
         # --- pair-symmetric W_vvvv: weights [nS + nA][kpad], split T3 and products for a chunk of blocks
         # (the split T3 and the products of a chunk of blocks live in the T2 -> T3 and ring scratch
         # buffers, idle during the W_vvvv terms: only the weights take memory of their own)
@@ -712,13 +709,12 @@ class TriplesEngine:
             Aq = Operand.strided(self.pfs, {'S': n3 * n3, 'p': n3, 'q': 1}, base=n3 * n3 + q0)
             X = Operand.strided(self.Xp, {'S': qc * v3, 'q': v3, 'a': v * v, 'b': v, 'c': 1})
             launches.append(plan_term('W_oooo/F_oo s1-5', 'pSq,pabc->Sqabc', Aq, B, X, 1.0, 0.0, [dict()], ext_c))
-            jobs = []
-            for q in range(q0, q0 + nq):
-                srcs, coef = [0] * 6, np.zeros(6)
-                for s in range(1, 6):
-                    p = TP_T3.index(perm[s])
-                    srcs[p], coef[p] = ((s - 1) * qc + q - q0) * v3, 1.0
-                jobs.append((q * v3, srcs, coef))
+            q = np.arange(nq)
+            jobs = np.zeros(nq, dtype=L.S3GATHER_DTYPE)
+            jobs['dst'] = (q0 + q) * v3
+            for s in range(1, 6):
+                p = TP_T3.index(perm[s])
+                jobs['src'][:, p], jobs['coef'][:, p] = ((s - 1) * qc + q) * v3, 1.0
             launches.append(S3GatherLaunch('W_oooo/F_oo add', self.R, self.Xp, v, 1.0, jobs))
         return launches
 
@@ -738,7 +734,7 @@ class TriplesEngine:
         blocks = self._xp_store.size // v3
         zc = max(1, min(o, blocks // (2 * npr), ((1 << 31) - 1) // v3))  # spectators per chunk
         pc = npr if 2 * npr * zc <= blocks else max(1, blocks // 2)     # and pairs, where one does not fit
-        index = {p: n for n, p in enumerate(self.pairs)}
+        ijk = np.asarray(self.triples, dtype=np.int64)
         launches = []
         for z0 in range(0, o, zc):
             nz = min(zc, o - z0)
@@ -750,19 +746,18 @@ class TriplesEngine:
                 launches.append(GemmLaunch('W_oooo/F_oo pairs', 2 * n, nz * v3, npr, 1.0, 0.0, self.Woo, am, ak,
                                            self.Y, bk, bn, self._xp_store, cm, cn, [(p0, z0 * v3, 0, 0, 2 * n)], 2 * n,
                                            2.0 * 2 * n * nz * v3 * npr))
-                jobs = []
-                for q, (i, j, k) in enumerate(self.triples):
-                    srcs, coef = [0] * 6, np.zeros(6)
-                    for pair, z, perms in (((i, j), k, ((1, 2, 0), (2, 1, 0))), ((i, k), j, ((1, 0, 2), (2, 0, 1))),
-                                           ((j, k), i, ((0, 1, 2), (0, 2, 1)))):
-                        row = index[(int(pair[0]), int(pair[1]))] - p0
-                        if not (0 <= row < n and z0 <= z < z0 + nz):
-                            continue
-                        for s, perm in enumerate(perms):
-                            p = TP_T3.index(perm)
-                            srcs[p], coef[p] = ((s * n + row) * nz + int(z) - z0) * v3, 1.0
-                    if coef.any():
-                        jobs.append((q * v3, srcs, coef))
+                jobs = np.zeros(len(ijk), dtype=L.S3GATHER_DTYPE)
+                jobs['dst'] = np.arange(len(ijk)) * v3
+                for x, y, z, perms in ((0, 1, 2, ((1, 2, 0), (2, 1, 0))), (0, 2, 1, ((1, 0, 2), (2, 0, 1))),
+                                       (1, 2, 0, ((0, 1, 2), (0, 2, 1)))):
+                    x, y, z = ijk[:, x], ijk[:, y], ijk[:, z] - z0
+                    row = x * o - x * (x - 1) // 2 + (y - x) - p0      # of the pair x <= y
+                    here = (row >= 0) & (row < n) & (z >= 0) & (z < nz)
+                    for s, perm in enumerate(perms):
+                        p = TP_T3.index(perm)
+                        jobs['src'][here, p] = (((s * n + row) * nz + z) * v3)[here]
+                        jobs['coef'][here, p] = 1.0
+                jobs = jobs[jobs['coef'].any(axis=1)]
                 launches.append(S3GatherLaunch('W_oooo/F_oo add', self.R, self._xp_store, v, 1.0, jobs))
         return launches
 
@@ -859,6 +854,9 @@ class TriplesEngine:
         cm, cn = L.IdxMap(None, 0, 1, ov, 0, 0, v2), L.IdxMap(None, 0, 1, v2, 0, 0, 1)
         # G = sum over the products of coefficient * product.transpose(q)
         parts_of_g = [{(0, 1, 2): 1.0}, {(1, 0, 2): 1.0, (0, 1, 2): 0.5}, {(1, 2, 0): 1.0, (0, 2, 1): 0.5}]
+        # X.transpose(q).transpose(perm) = X.transpose(q[perm]): coefficients by permutation of G and buffer
+        coefs = np.array([[_combination(0, {tuple(q[n] for n in perm): c for q, c in terms.items()})
+                           for terms in parts_of_g] for perm in TP_T3])
         launches = []
         for c0 in range(0, self.npairs, pc):
             chunk = list(enumerate(self.pairs))[c0:c0 + pc]
@@ -866,32 +864,29 @@ class TriplesEngine:
             for name, W, B, C, bk, bn in products:
                 launches.append(GemmLaunch(name, ov, v2, ov, 1.0, 0.0, W, am, ak, B, bk, bn, C, cm, cn, batches, ov,
                                            2.0 * len(chunk) * ov * v2 * ov))
-            jobs = []
-            for tq, lst in self._ring_targets(chunk, c0):
-                srcs = []
-                for perm, blk in lst:
-                    for buf, terms in enumerate(parts_of_g):
-                        # X.transpose(q).transpose(perm) = X.transpose(q[perm])
-                        srcs.append((buf, blk * v3, {tuple(q[n] for n in perm): c for q, c in terms.items()}))
-                jobs.append((tq * v3, srcs))
-            launches.append(S3PlaceLaunch('ring place', self.R, (self.Gs, F1, F2), v, jobs))
+            tq, perm, blk = self._ring_targets(chunk, c0)
+            srcs = np.zeros((len(tq), 3), dtype=L.S3PLACE_SRC_DTYPE)
+            srcs['buf'], srcs['off'], srcs['coef'] = np.arange(3), blk[:, None] * v3, coefs[perm]
+            target, first, count = np.unique(tq, return_index=True, return_counts=True)
+            jobs = np.zeros(len(target), dtype=L.S3PLACE_JOB_DTYPE)
+            jobs['dst'], jobs['first'], jobs['count'] = target * v3, 3 * first, 3 * count
+            launches.append(S3PlaceLaunch('ring place', self.R, (self.Gs, F1, F2), v, jobs, srcs.ravel()))
         return launches
 
     def _ring_targets(self, chunk, c0):
-        """[(target block, [(permutation of G, block of the chunk)])]: part 3 of target (r,p,q) is G[r;pq],
-        part 4 of (p,r,q) is G[r;pq] with (a,b) swapped, part 5 of (p,q,r) is G[r;pq] read as [c,a,b]."""
+        """Target blocks in ascending order, each with the permutation (its index) and the block of the chunk of a part
+        of G that goes there: part 3 of target (r,p,q) is G[r;pq], part 4 of (p,r,q) is G[r;pq] with (a,b) swapped,
+        part 5 of (p,q,r) is G[r;pq] read as [c,a,b]."""
         o = self.nocc
-        targets = {}
-        for pq, (p, q) in chunk:
-            for r in range(o):
-                blk = (pq - c0) * o + r
-                if r <= p:
-                    targets.setdefault(ijk_to_linear(r, p, q, o), []).append(((0, 1, 2), blk))
-                if p <= r <= q:
-                    targets.setdefault(ijk_to_linear(p, r, q, o), []).append(((1, 0, 2), blk))
-                if r >= q:
-                    targets.setdefault(ijk_to_linear(p, q, r, o), []).append(((1, 2, 0), blk))
-        return sorted(targets.items())
+        pq = np.array([x for _, x in chunk], dtype=np.int64)
+        p, q, r = pq[:, :1], pq[:, 1:], np.arange(o)
+        blk = (np.array([n for n, _ in chunk])[:, None] - c0) * o + r
+        ok = np.stack([r <= p, (p <= r) & (r <= q), r >= q], axis=-1)
+        tq = np.stack([ijk_to_linear(r, p, q, o), ijk_to_linear(p, r, q, o), ijk_to_linear(p, q, r, o)], axis=-1)[ok]
+        part = np.array([TP_T3.index(x) for x in ((0, 1, 2), (1, 0, 2), (1, 2, 0))])
+        perm, blk = np.broadcast_to(part, ok.shape)[ok], np.broadcast_to(blk[..., None], ok.shape)[ok]
+        order = np.argsort(tq, kind='stable')
+        return tq[order], perm[order], blk[order]
 
     def _plan_ring_terms(self):
         """Ring terms (rccsdt.py:540-596) without Z: G[r;pq] (the part-3 operator of the module docstring,
@@ -929,14 +924,12 @@ class TriplesEngine:
                                            getattr(self, wname), am, ak, self.Y, bk, bn, self.Gs, cm, cn,
                                            batches, ov, 2.0 * len(chunk) * ov * v2 * ov))
             # one gather pass: each target takes its (up to three) part contributions of this chunk
-            jobs = []
-            for tq, lst in self._ring_targets(chunk, c0):
-                srcs, coef = [0] * 6, np.zeros(6)
-                for perm, blk in lst:
-                    pidx = TP_T3.index(perm)
-                    assert coef[pidx] == 0.0   # the three parts use three different permutations
-                    srcs[pidx], coef[pidx] = blk * v3, 1.0
-                jobs.append((tq * v3, srcs, coef))
+            tq, perm, blk = self._ring_targets(chunk, c0)
+            target, of = np.unique(tq, return_inverse=True)
+            jobs = np.zeros(len(target), dtype=L.S3GATHER_DTYPE)
+            jobs['dst'] = target * v3
+            jobs['src'][of, perm], jobs['coef'][of, perm] = blk * v3, 1.0
+            assert int(jobs['coef'].sum()) == len(tq)   # the three parts use three different permutations
             launches.append(S3GatherLaunch('ring place', self.R, self.Gs, v, 1.0, jobs))
         return launches
 
@@ -973,21 +966,15 @@ class TriplesEngine:
         ext.update({'p': o, 'r': o, 'l': o, 'm': o, 'i': o, 'k': o, 'Q': qc, 'X': 1})
         Zs = (qc, o, o, v, v, v)
         Z = lambda letters: Operand(lo['Z'], letters, Zs)
+        z_coef = np.array([_combination(c, {(0, 1, 2): 2.0, (2, 1, 0): -1.0, (1, 0, 2): -1.0}) for c in range(6)])
         chunks = []
         for q0 in range(0, o, qc):
             nq = min(qc, o - q0)
             ext_c = dict(ext, Q=nq)
-            jobs = []
-            for Q in range(nq):
-                for p in range(o):
-                    for r in range(o):
-                        case, (ci, cj, ck) = canonical_case(p, q0 + Q, r)
-                        P = TP_T3[case]
-                        coef = np.zeros(6)
-                        for c, Qp in ((2.0, (0, 1, 2)), (-1.0, (2, 1, 0)), (-1.0, (1, 0, 2))):
-                            comp = (P[Qp[0]], P[Qp[1]], P[Qp[2]])
-                            coef[TP_T3.index(comp)] += c
-                        jobs.append((((Q * o + p) * o + r) * v3, ijk_to_linear(ci, cj, ck, o) * v3, coef))
+            Q, p, r = np.ogrid[:nq, :o, :o]
+            case, src = canonical_cases(p, q0 + Q, r, o)
+            jobs = np.zeros(case.size, dtype=L.S3JOB_DTYPE)
+            jobs['dst'], jobs['src'], jobs['coef'] = np.arange(case.size) * v3, src.ravel() * v3, z_coef[case.ravel()]
             # --- T3 -> r2, r1 ---
             a2 = []
             e_split = [({'p': p}, {'p': p}, {'S': p}) for p in range(o)]
@@ -1016,7 +1003,7 @@ class TriplesEngine:
                                   Operand(lo['dWovvv'], 'Qabd', (o, v, v, v)), -1.0, 1.0, ext_c,
                                   [({}, {}, {'Q': q0})]))
             self._retarget([g for g in a2 + a3 if isinstance(g, GemmLaunch)])
-            chunks.append((DeviceArray.from_host(s3_jobs_array(jobs)), len(jobs), a2, a3))
+            chunks.append((DeviceArray.from_host(jobs), len(jobs), a2, a3))
         lo['chunks'] = chunks
         upload_tables([g for ch in chunks for g in ch[2] + ch[3]])
         lo['dw_valid'] = False
