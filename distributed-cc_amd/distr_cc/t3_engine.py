@@ -603,8 +603,9 @@ class TriplesEngine:
         Y and Z are packed in place (they are rebuilt from T3 for every residual and read by nothing
         else), by writing them as packed words in the first place; the others get packed copies.
         Returns the (source, packed, count) passes to run."""
-        sources = [self.t3, self.Yz, self.W1, self.W_ovvv, self.W_oovo, self.t2, self.WR1, self.WR3,
-                   self.pfs if self.oooo_blocks else self.Woo]
+        # (with Z, nothing reads WR3b)
+        sources = [self.t3, self.Yz, self.W1, self.W_ovvv, self.W_oovo, self.t2, self.WR1,
+                   self.WR3a if self.ring_fused else self.WR3, self.pfs if self.oooo_blocks else self.Woo]
         # the pair-symmetric W_vvvv operands are written as packed words by their own kernels
         in_place = [self.Wp, self.Tp] if self.vvvv_pairs else []
         sources += in_place

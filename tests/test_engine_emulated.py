@@ -792,3 +792,28 @@ def test_planning_builds_tables_with_array_operations(monkeypatch, kw):
         counts.append((n[0], sum(g.nbatch for g in launches)))
     calls, entries = (y - x for x, y in zip(*counts))
     assert entries < 1200 and calls < 15 * entries, counts
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_packed_operands_are_read(monkeypatch, fused):
+    """Every tensor that a split-BF16x3 engine packs for a residual is read, to its end, by a product."""
+    abi_emulator.install(monkeypatch)
+    from distr_cc.t3_engine import GemmLaunch, TriplesEngine
+    eng = TriplesEngine(4, 6, dtype=np.float32, contract="bf16x3", ring_fused=fused)
+    assert eng._packs
+    for src, dst, n in eng._packs:
+        assert n == src.size == dst.size
+        last = -1
+        for g in eng.launches:
+            if not isinstance(g, GemmLaunch) or g.fn != "dcc_contract_packed_bf16x3":
+                continue
+            M, N, K, _, _, A, am, ak, B, bk, bn = g.args[:11]
+            for ptr, field, rows, k, nrow in ((A, "a_off", am, ak, None), (B, "b_off", bn, bk, N)):
+                if not dst.ptr <= ptr.value < dst.ptr + dst.nbytes:
+                    continue
+                at = lambda m, x: (x // (m.e1 * m.e2) * m.s0 + x // m.e2 % m.e1 * m.s1 + x % m.e2 * m.s2).max()
+                for b in g.table:
+                    nr = int(b["m_end"]) if nrow is None else nrow
+                    off = (ptr.value - dst.ptr) // 4 + int(b[field])
+                    last = max(last, off + int(at(rows, np.arange(nr)) + at(k, np.arange(K))))
+        assert last == n - 1, (src.shape, last)
