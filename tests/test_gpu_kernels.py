@@ -1010,3 +1010,85 @@ def test_q_gemms_with_lds_finalize_vs_oracle(dev, o, v, bs, w_mode):
         got = eng.kernel(pppp, t2, DeviceArray.from_host(t3), s.mo_energy)
         for g, r in zip(got, ref):
             assert abs(g - r) <= 1e-12 * abs(r)
+
+
+# (variant, small, extents (x, y, K) of the problems): x walks the rows of a tile, y its columns
+SKINNY_GROUPS = [
+    (9, 0, [(33, 40, 64), (7, 9, 17), (16, 16, 1), (20, 31, 50)]),
+    (0, 0, [(33, 40, 100), (5, 70, 65), (17, 1, 97), (16, 16, 383)]),
+    (1, 0, [(33, 40, 400), (16, 17, 385), (1, 5, 384), (40, 40, 70)]),
+    (2, 0, [(5, 5, 1805), (33, 40, 768), (17, 18, 900), (3, 50, 66)]),
+    (0, 0, [(100, 150, 100), (19, 33, 70), (33, 40, 383)]),
+    (1, 0, [(100, 150, 400), (19, 33, 70), (33, 41, 385)]),
+    (3, 0, [(66, 500, 70), (33, 40, 97), (1, 35, 3)]),
+    (4, 0, [(500, 66, 70), (40, 33, 97), (35, 1, 3)]),
+    (5, 0, [(5, 9001, 66), (16, 70, 128), (1, 64, 100)]),
+    (6, 0, [(15, 9000, 130), (16, 70, 401), (1, 65, 64)]),
+    (7, 0, [(9001, 5, 66), (70, 16, 128), (64, 1, 100)]),
+    (8, 0, [(9000, 15, 130), (70, 16, 401), (65, 1, 64)]),
+    (3, 1, [(400, 1500, 66), (33, 40, 97), (2, 7, 5)]),
+    (9, 1, [(700, 900, 33), (16, 40, 64), (2, 7, 5)]),
+]
+
+
+@pytest.mark.parametrize("variant,small,sizes", SKINNY_GROUPS)
+def test_grouped_skinny_variants(dev, variant, small, sizes):
+    """dcc_grouped_prepare_auto and the grouped skinny kernel: each of the ten variants with problems that differ in
+    size, in which index of C is contiguous, in operand layouts, in K maps of one and two levels (odd and even
+    inner extents) and in odd batch offsets and row ranges, and with problems without rows and without K, on the
+    default grid and on seven persistent workgroups.  Bound: K rounding errors of the sum of magnitudes."""
+    import ctypes
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    _say("grouped skinny variant %d small=%d" % (variant, small))
+    rng = np.random.default_rng(1000 * variant + small)
+    lin = lambda s: L.IdxMap(None, 0, 1, 1 << 20, 0, 0, s)
+    two = lambda e, s: L.IdxMap(None, 0, 1, e, e * s, 0, s)      # the same offsets through two levels
+    cases = []
+    for n, (x, y, K) in enumerate(sizes + [(0, 16, 30), (6, 7, 0)]):
+        swap = n % 2 == 1                      # C contiguous along m: columns walk m
+        M, N = (y, x) if swap else (x, y)
+        for a_k, b_n in ((1, 1), (0, 0)) if n % 3 else ((1, 0), (0, 1)):
+            cases.append((M, N, K, a_k, b_n, not swap, (None, 5, 4)[(n + a_k) % 3]))
+    probs = (L.GemmProblem * len(cases))()
+    host, keep = [], []
+    for p, (M, N, K, a_k, b_n, c_n, inner) in zip(probs, cases):
+        A = rng.standard_normal((2, M, K) if a_k else (2, K, M))
+        B = rng.standard_normal((2, K, N) if b_n else (2, N, K))
+        C = rng.standard_normal((2, M, N) if c_n else (2, N, M))
+        one = np.zeros(1)
+        dA, dB, dC = (DeviceArray.from_host(np.concatenate([x[0].ravel(), one, x[1].ravel(), one])) for x in (A, B, C))
+        km = lin if inner is None else (lambda s: two(inner, s))
+        bt = np.zeros(2, dtype=L.BATCH_DTYPE)
+        bt["a_off"], bt["b_off"], bt["c_off"] = (0, M * K + 1), (0, K * N + 1), (0, M * N + 1)
+        bt["m_begin"], bt["m_end"] = (0, M // 4), (M, M - M // 3)
+        db = DeviceArray.from_host(bt)
+        p.N, p.K, p.alpha, p.beta = N, K, -0.5, (1.0, 0.0, 0.25)[(M + N) % 3]
+        p.A, p.B, p.C = dA.ptr, dB.ptr, dC.ptr
+        p.am, p.ak = (lin(K), km(1)) if a_k else (lin(1), km(M))
+        p.bk, p.bn = (km(N), lin(1)) if b_n else (km(1), lin(K))
+        p.cm, p.cn = (lin(N), lin(1)) if c_n else (lin(1), lin(M))
+        p.batches, p.nbatch, p.max_rows = db.ptr, 2, M
+        host.append((A, B, C, bt, p.beta))
+        keep.append((dA, dB, dC, db))
+    total, var = ctypes.c_int64(), ctypes.c_int64()
+    L.call("dcc_grouped_prepare_auto", ctypes.cast(probs, ctypes.c_void_p), len(cases), small, ctypes.byref(total),
+           ctypes.byref(var))
+    assert var.value == 64 + variant
+    dp = DeviceArray.from_host(np.frombuffer(bytes(probs), dtype=np.uint8).copy())
+    for grid in (0, 7):
+        for (A, B, C, bt, beta), (_, _, dC, _) in zip(host, keep):
+            dC.upload(np.concatenate([C[0].ravel(), [0.0], C[1].ravel(), [0.0]]))
+        L.call("dcc_contract_grouped_f64", dp.vp, len(cases), total.value, var.value, grid, None)
+        for (M, N, K, a_k, b_n, c_n, inner), (A, B, C, bt, beta), (_, _, dC, _) in zip(cases, host, keep):
+            out = dC.download()
+            for b in range(2):
+                at, lo, hi = int(bt["c_off"][b]), int(bt["m_begin"][b]), int(bt["m_end"][b])
+                got = out[at:at + M * N].reshape(C.shape[1:])
+                c, got = (C[b], got) if c_n else (C[b].T, got.T)
+                a, bb = A[b] if a_k else A[b].T, B[b] if b_n else B[b].T
+                ref = c.copy()
+                ref[lo:hi] = beta * c[lo:hi] - 0.5 * (a[lo:hi] @ bb)
+                bound = np.finfo(np.float64).eps * (max(K, 1) * (np.abs(a) @ np.abs(bb)) + np.abs(ref) + np.abs(c))
+                assert (np.abs(got - ref) <= bound).all(), (M, N, K, a_k, b_n, c_n, inner, grid)
+            assert out[M * N] == 0.0 and out[-1] == 0.0
