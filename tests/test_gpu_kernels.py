@@ -1092,3 +1092,38 @@ def test_grouped_skinny_variants(dev, variant, small, sizes):
                 bound = np.finfo(np.float64).eps * (max(K, 1) * (np.abs(a) @ np.abs(bb)) + np.abs(ref) + np.abs(c))
                 assert (np.abs(got - ref) <= bound).all(), (M, N, K, a_k, b_n, c_n, inner, grid)
             assert out[M * N] == 0.0 and out[-1] == 0.0
+
+
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("o", [1, 2, 3, 6])
+def test_oooo_prefactors(dev, o, dt):
+    """dcc_oooo_prefactors_*: applied to the blocks of a T3 they give the W_oooo and F_oo terms of the full tensors
+    (which of the permutations that leave a block unchanged carries a coefficient is free).  The coefficients are
+    FP64 sums of a few terms, rounded once; the products are formed on the host in FP64."""
+    from distr_cc import _lib as L
+    from distr_cc.device import DeviceArray
+    from distr_cc.distribute_t3 import canonical_triples
+    from distr_cc.synthetic import SyntheticSystem
+    from oracle import t3_layout as TL
+    _say("oooo prefactors o=%d %s" % (o, dt))
+    v = 3
+    rng = np.random.default_rng(30 + o)
+    typ = np.float64 if dt == "f64" else np.float32
+    W, F = rng.normal(size=(o,) * 4), rng.normal(size=(o, o)).astype(typ)
+    W = (W + W.transpose(1, 0, 3, 2)).astype(typ)
+    ijk = np.ascontiguousarray(canonical_triples(o), dtype=np.int32)
+    n3 = len(ijk)
+    t3 = SyntheticSystem(o, v, naux=20, seed=9, sigma_t3=1.0).t3_tri()
+    out = DeviceArray((6, n3, n3), typ)
+    dW, dF, dB = DeviceArray.from_host(W), DeviceArray.from_host(F), DeviceArray.from_host(ijk)
+    L.call("dcc_oooo_prefactors_" + dt, dW.vp, dF.vp, o, dB.vp, n3, out.vp, None)
+    pfs = out.download().astype(np.float64)
+    got = sum(np.einsum(f, c, t3) for f, c in zip(("pq,pabc->qabc", "pq,pacb->qabc", "pq,pbac->qabc", "pq,pabc->qcab",
+                                                   "pq,pabc->qbca", "pq,pabc->qcba"), pfs))
+    T, W, F = TL.full_t3_from_tri(t3, o), W.astype(np.float64), F.astype(np.float64)
+    full = (np.einsum("lmij,lmkabc->ijkabc", W, T) + np.einsum("lmik,lmjacb->ijkabc", W, T) +
+            np.einsum("lmjk,lmibca->ijkabc", W, T) - np.einsum("li,ljkabc->ijkabc", F, T) -
+            np.einsum("lj,ilkabc->ijkabc", F, T) - np.einsum("lk,ijlabc->ijkabc", F, T))
+    ref = np.array([full[tuple(x)] for x in ijk])
+    scale = abs(t3).max() * (3 * o * o * abs(W).max() + 3 * o * abs(F).max())
+    assert abs(got - ref).max() <= 8 * np.finfo(typ).eps * scale
