@@ -292,7 +292,7 @@ def q_time(o, v, blksize=4, seed=20261202):
             "q_time_s": a.elapsed_ms(b) / 1e3, "wall_s": time.perf_counter() - w0,
             "first_call_s": a0.elapsed_ms(b0) / 1e3, "e_bracket": eb, "e_paren": ep,
             "note": "second call of one QEngine: host->device copies of the integral slices (PCIe), IJK->ABC "
-                    "gather, W builders, all task GEMMs, finalize and reductions; the first call also "
+                    "gather, W builders, all quadruples and reductions; the first call also "
                     "allocates the buffers and plans every launch (first_call_s)"}
 
 

@@ -355,8 +355,8 @@ __device__ __forceinline__ void stage_rows(T *lds, const OwnOrbit<PAIR> &w, cons
 // One output tile per workgroup, as above, reads a source once per coefficient; for the ring operator
 // (five coefficients in three sources per part) that was 15 tiles instead of 9 through L2, which bound it.
 // The LDS tile is double buffered (one barrier per source tile) and the loads run three tiles ahead.  HBM
-// bounds it: at nocc=10, nvir=90 in FP64 it moves 14.8 GB in 3.6 ms (7.4 ms a tile at a time); in FP32, rows
-// of half a line, 24 GB in 9.1 ms at nocc=12, nvir=120.
+// bounds it: at nocc=10, nvir=90 in FP64 it moves 14.1 GB in 3.6 ms (7.4 ms a tile at a time); in FP32, rows
+// of half a line, 27.7 GB in 9.1 ms at nocc=12, nvir=120.
 template <typename T> struct PlaceBufs {
     const T *b[3];
 };

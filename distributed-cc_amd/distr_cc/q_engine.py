@@ -187,7 +187,7 @@ class QEngine:
         ext = {x: bs for x in 'abcd'}
         ext.update({'e': vp, 'f': vp})
         ext.update({x: o for x in 'ijklmn'})
-        # chunks bound z4/t4 and the W_vvvvoo slots; with neither only the partials
+        # a chunk bounds z4/t4, or the W_vvvvoo slots of its tasks (by the same rule); with neither the partials
         fused = self.fused
         size = self.quad_chunk if fused and self.w_mode == "dense" else self.chunk
         nmax = min(size, len(tasks))

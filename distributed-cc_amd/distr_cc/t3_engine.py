@@ -729,7 +729,7 @@ class TriplesEngine:
         Y[lm][z][c,a,b] for a range of spectators z is one plain GEMM (N = (z,c,a,b), K = the pairs l <= m, Y as
         the ring reads it), and one gather pass adds, for every target, the two products s of each of its three
         pairs, whose permutations are the six of the group.  Summed over source blocks instead, six GEMMs of
-        n3 x n3 per element, these terms were 4.8 (nocc=10) to 5.6 (nocc=12) times the flops."""
+        n3 x n3 per element, these terms were 4.8 (nocc=10) to 5.4 (nocc=12) times the flops."""
         o, v = self.nocc, self.nvir
         v3, npr = v ** 3, self.npairs
         blocks = self._xp_store.size // v3
